@@ -39,7 +39,7 @@ def _args():
     ap.add_argument("--warmup", type=int, default=2)
     ap.add_argument("--config", type=int, default=2,
                     help="benchmark configuration: 2 fwd+BPTT (default), 1 or 3 forward, 4 the firing-rate "
-                         "sweep of the event push against the deterministic row pull (B=32)")
+                         "sweep of the event against the deterministic forward (B=32)")
     ap.add_argument("--rates", default="1,5,20,50", help="config 4: target mean rates in Hz")
     ap.add_argument("--mode", default="event", choices=["event", "deterministic"])
     ap.add_argument("--loss", default="mse", choices=["mse", "reference"],
@@ -229,7 +229,7 @@ class RateCalibrator:
 
 
 def sweep_rates(args):
-    """Config 4: forward throughput of the event push and the deterministic row pull at
+    """Config 4: forward throughput of the event and the deterministic mode at
     several mean firing rates.  One factor scales the recurrent weights only (the role of
     the reference's recurrent_weight_scale, models.py:664; the LGN and background weights stay
     as generated); it is set per target rate by bisection in log space on whole rollouts (the
@@ -289,12 +289,9 @@ def sweep_rates(args):
                      "event_ms_per_step": round(ev_ms, 4), "pull_ms_per_step": round(pl_ms, 4),
                      "event_kernel_us_per_step": ev_k, "pull_kernel_us_per_step": pl_k,
                      "rec_events_per_step": round(events),
-                     # push bytes: 8-byte entry + one 4-byte atomic per event, over the whole
-                     # event forward's kernel time (the pushes run inside the step launch);
-                     # pull: every post-row entry (4 bytes) + the active entries' weight and
-                     # type (5), over the pull kernel's time
-                     "event_push_GBps": round(events * 12 / (sum(ev_k.values()) * 1e-6) / 1e9, 1),
-                     "pull_GBps": round((S * 4 + events * 5) / (pl_k.get("push", 1e9) * 1e-6) / 1e9, 1)})
+                     # one 8-byte entry per recurrent event over the mode's whole kernel time
+                     "event_push_GBps": round(events * 8 / (sum(ev_k.values()) * 1e-6) / 1e9, 1),
+                     "pull_GBps": round(events * 8 / (sum(pl_k.values()) * 1e-6) / 1e9, 1)})
         print(json.dumps(rows[-1]), file=sys.stderr, flush=True)
     best5 = min((r for r in rows), key=lambda r: abs(r["target_hz"] - 5.0)) if rows else None
     value = B * N / (min(best5["event_ms_per_step"], best5["pull_ms_per_step"]) / 1000.0) if best5 else 0.0
@@ -304,8 +301,8 @@ def sweep_rates(args):
         "ms_per_step": min(best5["event_ms_per_step"], best5["pull_ms_per_step"]) if best5 else None,
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": f"config 4: {N} GLIF_3 neurons, {S} recurrent synapses, B={B}, T={T}, "
-                               "modulated LGN, forward; recurrent weights scaled to each rate; event push vs "
-                               "deterministic row pull",
+                               "modulated LGN, forward; recurrent weights scaled to each rate; event vs "
+                               "deterministic mode",
                    "neurons": N, "recurrent_synapses": S, "batch": B, "seq_len": T,
                    "rate_with_recurrent_weights_at_zero_hz": round(cal.floor_hz, 3) if cal.floor_hz is not None
                    else None},
@@ -558,11 +555,8 @@ def main():
     sc_host = spike_count.cpu().numpy()
     # one more, untimed step with every kernel class timed: the breakdown, and the dominant
     # class (most time per step), whose launches the timed steps bracket with HIP events.
-    # Event mode's forward is one fused launch per tick (the step of t - 1 beside the pushes,
-    # "step"), and so is deterministic mode's (the row pull of t beside the step of t, whose R
-    # takes the currents of t - 1; "step"; where the pull and the step run as two launches the
-    # row pull is "push"); "lgn" computes 64 ticks of LGN currents ahead of the loop (batch
-    # sizes up to 8); "adj" is the adjoint launch with the
+    # The forward is one launch per three ticks ("step": their currents, summed from the spikes,
+    # and their GLIF_3 steps); "adj" is the adjoint launch with the
     # previous window's weight gradients and the rest of its dz walk; "bwd_rec" the dz walk
     # over the columns the next adjoint reads.
     _lib.prof_enable(list(_lib.PROF_KINDS))
@@ -610,11 +604,6 @@ def main():
     while Rg < Wwin * B:
         Rg *= 2
     words = (N + 63) // 64
-    # LGN currents computed ahead of the loop (the "lgn" class ran): the tick's launch then
-    # pushes or pulls the recurrent events only, and in event mode the step leaves the
-    # current slot to the next LGN pass instead of clearing it
-    lgn_ahead = breakdown.get("lgn", {}).get("launches", 0) > 0
-    e_in = 0.0 if lgn_ahead else e_lgn
     tot_ms, launches = prof.get(dominant, (0.0, 0))
     # the grouped dz walk (16-float G rows) with the weight gradients deferred splits each
     # window's walk: the columns of delays <= 2 Wwin - 3 (what the next window's adjoint reads,
@@ -667,45 +656,15 @@ def main():
                      + (S - s_a) * 8 + (n_cols - cols_a + 1) * 4 + Wwin * B * (n_cols - cols_a) * 4)
         unit_desc = (f"bytes per backward window of {Wwin} timesteps (adjoint + previous window's dz rest"
                      + (")" if dw_walk else " and dW)"))
-    elif dominant == "step" and args.mode == "deterministic":
-        # per launch = one tick: the row pull (every recurrent entry's bitmap index, and the
-        # LGN ones when their currents are not computed ahead, 4 bytes; the row pointers; each
-        # active entry's batch mask, weight and type, 9 bytes; the currents written) beside the
-        # GLIF_3 step's state stream per (b, n) -- reads the previous tick's pulled I and its
-        # LGN currents (I2 or the LGN ring's slot), R, P (nb floats each), A (2 floats), v, r
-        # (int16); writes R, P, A, v, r and the saved voltage -- the per-neuron constants
-        # (7 floats) and the background rows (8 bytes per synapse)
-        active = (e_rec + e_in) / max(T, 1)
-        tables = 1 if lgn_ahead else 2
-        per_bn = (4 * nb * 4 + 14) + (2 * nb * 4 + 18)
-        alg_bytes = ((S + (0 if lgn_ahead else tb.lgn.n_syn)) * 4 + tables * (N + 1) * 4 + active * 9
-                     + tables * nb * B * N * 4 + B * N * per_bn + N * 28 + tb.bkg.n_syn * 8)
-        unit_desc = "bytes per forward timestep (deterministic row pull beside the GLIF_3 step)"
-    elif dominant == "step":
-        # per launch = one tick: the GLIF_3 step's state stream per (b, n) -- reads I, R, P
-        # (nb floats each), A (2 floats), v, r (int16); writes R, P, A, v, r, the saved voltage
-        # and, without the LGN ring, I (cleared) -- the per-neuron constants (7 floats), the
-        # background rows (8 bytes per synapse), and the tick's pushed events (8-byte entry +
-        # one 4-byte atomic each; the LGN events too when their currents are not computed ahead)
-        active = (e_rec + e_in) / max(T, 1)
-        per_bn = (3 * nb * 4 + 14) + ((2 if lgn_ahead else 3) * nb * 4 + 18)
-        alg_bytes = B * N * per_bn + N * 28 + tb.bkg.n_syn * 8 + active * 12
-        unit_desc = "bytes per forward timestep (GLIF_3 step + the tick's pushed events)"
-    elif dominant == "lgn":
-        # per launch = 64 ticks of LGN currents: every LGN entry (input, weight, type: 9
-        # bytes), the row pointers, the segment's tick masks per (input, batch entry), 8 bytes,
-        # and the 64 current slots written ([nb][B][N] floats each)
-        alg_bytes = (tb.lgn.n_syn * 9 + (N + 1) * 4 + tb.lgn.n_cols * B * 8 + 64 * nb * B * N * 4)
-        unit_desc = "bytes per 64-tick segment of LGN currents"
-    else:
-        # per launch = one timestep's row pull: every recurrent entry's bitmap index, and the
-        # LGN ones when their currents are not computed ahead (4 bytes), the row pointers, each
-        # active entry's batch mask, weight and type (9 bytes), and the currents written
-        active = (e_rec + e_in) / max(T, 1)
-        tables = 1 if lgn_ahead else 2
-        alg_bytes = ((S + (0 if lgn_ahead else tb.lgn.n_syn)) * 4 + tables * (N + 1) * 4 + active * 9
-                     + tables * nb * B * N * 4)
-        unit_desc = "bytes per forward timestep (deterministic row pull)"
+    else:   # "step"
+        # per launch = a window of ticks: the GLIF_3 state per (b, n), read and written once (R, P:
+        # nb floats each, A: 2 floats, v, r int16), the saved voltage of every tick, the per-neuron
+        # constants (7 floats), the background rows (8 bytes per synapse), and 8 bytes per recurrent
+        # and LGN event of the window's ticks (its entry)
+        ticks = T / max(breakdown[dominant]["launches"], 1)
+        per_bn = 2 * (2 * nb * 4 + 14) + 4 * ticks
+        alg_bytes = B * N * per_bn + N * 28 + tb.bkg.n_syn * 8 + (e_rec + e_lgn) / max(T, 1) * ticks * 8
+        unit_desc = f"bytes per window of {ticks:.2f} forward timesteps (GLIF_3 steps + their events' entries)"
     # the per-step algorithmic bytes of the path's operations, independent of how the kernels
     # batch them (the op's backward re-reads its table every step; the forward's push reads each
     # event's entry): per step, op backward (dz, + dW) 9 B per synapse (entry + syn_id), the
@@ -730,20 +689,19 @@ def main():
         k_bytes = Wwin * (k5 + k4_cols(S - s_a, n_cols - cols_a))
         k_desc = (f"per-step adjoint bytes (4 + 8 nb + 13 B read, 4 + 12 nb B written per (b, n)) + op-backward "
                   f"bytes over the other {n_cols - cols_a} columns, x {Wwin} steps")
-    elif dominant == "step" and args.mode == "deterministic":
-        k_bytes = k3 + S * 9 + B * D * N / 8 + B * N * nb * 4
-        k_desc = "per-step bytes of the GLIF_3 step + the recurrent row pull (9 B per synapse, packed spikes)"
-    elif dominant == "step":
-        k_bytes = k3 + a_step * 12 + e_step * 9 + B * N * nb * 4
-        k_desc = "per-step bytes of the GLIF_3 step + the recurrent push (12 B per active column, 9 B per event)"
+    else:
+        ticks = T / max(breakdown[dominant]["launches"], 1)
+        k_bytes = ticks * (k3 + a_step * 12 + (e_step + e_lgn / max(T, 1)) * 9 + B * N * nb * 4)
+        k_desc = (f"per-step bytes of the GLIF_3 step + the recurrent and LGN events (12 B per active recurrent "
+                  f"column, 9 B per event) x {ticks:.2f} steps")
     avg_ms = tot_ms / max(launches, 1)
     own_bytes, own_desc = alg_bytes, unit_desc
     if k_bytes is not None:
         alg_bytes, unit_desc = k_bytes, k_desc
     achieved = alg_bytes / (avg_ms / 1000.0) / 1e9 if avg_ms > 0 else 0.0
     own_achieved = own_bytes / (avg_ms / 1000.0) / 1e9 if avg_ms > 0 else 0.0
-    # measured traffic per kernel class (deterministic mode's fused launch has its own)
-    traffic = load_traffic("pull_step" if (dominant == "step" and args.mode == "deterministic") else dominant)
+    # measured traffic per kernel class
+    traffic = load_traffic(dominant)
     roofline = {"kernel": dominant, "bound": "hbm", "achieved": round(achieved, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": traffic.get("bytes_per_launch") if traffic else None,

@@ -37,11 +37,11 @@ typedef enum {
 } glif_status;
 
 typedef enum {
-    GLIF_MODE_EVENT = 0,         /* event-driven push of active columns, fp32 atomics;     */
-                                 /* sums order-free, within 1e-5 of the reference's (a     */
+    GLIF_MODE_EVENT = 0,         /* sums order-free, within 1e-5 of the reference's.  Op:  */
+                                 /* event-driven push of active columns, fp32 atomics (a   */
                                  /* table with columns > 2048 synapses, whose inputs each  */
                                  /* fan out to thousands of posts, is pulled instead)      */
-    GLIF_MODE_DETERMINISTIC = 1  /* post-row pull in the reference's accumulation order   */
+    GLIF_MODE_DETERMINISTIC = 1  /* sums in the reference's accumulation order             */
 } glif_mode;
 
 typedef struct glif_table glif_table;  /* one synapse population, device resident */
@@ -312,11 +312,11 @@ int glif_sample_poisson(float lam, float exp_neg_lam, int64_t n, uint64_t seed, 
 /* ------------------------------------------------------------ profiling ------
  * No reference counterpart (the reference times whole steps with time(),
  * callbacks.py:1442-1449).  Kernel classes: 0 push, 1 step, 2 adj, 3 bwd_rec,
- * 4 bwd_lgn, 5 bwd_bkg, 6 syn_fwd, 7 syn_bwd, 8 lgn.  In the cell's event mode "step" is
- * the one launch per tick that runs the step beside that tick's pushes and "push" only the
- * push of tick 0; in deterministic mode "push" is the row pull where it runs as a launch
- * of its own.  "lgn" is the pass that computes 64 ticks of LGN currents ahead of the loop
- * (batch sizes up to 8).  "adj" includes the
+ * 4 bwd_lgn, 5 bwd_bkg, 6 syn_fwd, 7 syn_bwd, 8 lgn.  "step" is a launch of the
+ * cell's forward: three ticks, their currents summed from the spikes (or one tick, where a
+ * network's row offsets outgrow their bound: with its pushes in event mode, "push" then being the
+ * push of tick 0, or a row pull of its own in deterministic mode, and "lgn" the pass that computes
+ * 64 ticks of LGN currents ahead of the loop).  "adj" includes the
  * previous window's weight-gradient passes and the rest of its dz walk, which share its launch.
  * While bit k of `mask` is set, every launch of class k (every `every`-th, glif_prof_stride,
  * counted from glif_prof_enable; default 1) is bracketed by two HIP events on its stream.

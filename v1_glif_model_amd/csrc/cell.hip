@@ -1,6 +1,8 @@
 // The GLIF_3 cell over T steps (V1Column.call, models.py:1059-1135) and its BPTT.
 //
-// Forward, per step t (one stream, no host round trip):
+// Forward, three ticks per launch (k_win_fwd): a workgroup per range of posts and batch entry sums
+// its recurrent and LGN currents from the spikes in LDS (win_kernels.h) and steps its posts.
+// Networks whose spike-major row offsets outgrow their bound run a launch or two per step t:
 //   LGN (B <= 8; event mode from B = 3 and without per-type slots): k_lgn_rows computes
 //                 the LGN currents of 64 ticks at a time, per post row in the reference's
 //                 order, into a ring of current slots ahead of the ticks that read them
@@ -36,12 +38,16 @@
 #include "prof.h"
 #include "pull_kernels.h"
 #include "syn_kernels.h"
+#include "win_kernels.h"
 
 namespace glif {
 
 // ------------------------------------------------------------------ state ----
 constexpr int kVlossBlocks = 1024;  // blocks of the voltage-penalty reduction
 struct CellWs {
+    uint64_t *lgnbits;  // [T][B][Wl]        bit pre: x_t[b][pre] > 0 (window forward)
+    uint16_t *lgndig;   // [T][B][segments]  their digests (win_kernels.h)
+    uint16_t *zdig;     // [(T + D)][B][ranges]  the spikes' digests
     float *I;           // [2][nb][B][N]   pushed rec + LGN currents (event mode), or
                         // [2][g_rows][B][N] type sums with per-type slots
     float *R, *P;       // [nb][B][N]   psc_rise, psc (receptor-major copies of the state)
@@ -139,6 +145,13 @@ static bool ensure_side(Cell *c) {
     return true;
 }
 
+// Whether the forward runs window by window (k_win_fwd): its recurrent and LGN tables carry
+// spike-major rows, or hold no synapses.  A network whose row offsets outgrow their bound
+// (kSpkMaxOff: about half a million neurons, or ~100k with 256 delay slots) takes a launch per tick.
+static bool win_forward(const Cell *c) {
+    return (c->rec->n_syn == 0 || c->rec->spk.rows) && (c->lgn->n_syn == 0 || c->lgn->spk.rows);
+}
+
 // Backward window width (reverse ticks per table pass) and G row length.
 static int win_width(int B) { return 3 * B <= 16 ? 3 : 1; }
 static int n_windows(int T, int Wwin) { return T >= 3 ? (T - 2 + Wwin - 1) / Wwin : 0; }
@@ -162,19 +175,27 @@ static CellWs carve_cell(void *ws, const Cell *c, int32_t B, int32_t T, size_t *
     w.A = cv.take<float>(BN * 2);
     w.zbits = cv.take<uint64_t>(static_cast<size_t>(T + c->D) * B * c->W);
     w.refbits = cv.take<uint64_t>(static_cast<size_t>(T) * B * c->W);
-    w.zmask = cv.take<uint32_t>(static_cast<size_t>(T + c->D) * c->Np);
-    w.lmask = cv.take<uint32_t>(static_cast<size_t>(T) * nl);
-    w.abits = cv.take<uint64_t>(static_cast<size_t>(T + c->D) * c->W);
-    w.lbits = cv.take<uint64_t>(static_cast<size_t>(T) * ((nl + 63) / 64));
-    w.I2 = cv.take<float>(2 * BN * c->nb);  // deterministic pull beside the step: two halves
-    if (lgn_ahead(c, B, T)) {
-        w.IL = cv.take<float>(static_cast<size_t>(kLgnRing) * BN * c->nb);
-        w.lgnT = cv.take<uint64_t>(static_cast<size_t>((T + kLgnSeg - 1) / kLgnSeg) * nl * B);
+    if (win_forward(c)) {
+        w.lgnbits = cv.take<uint64_t>(static_cast<size_t>(T) * B * ((nl + 63) / 64));
+        w.lgndig = cv.take<uint16_t>(static_cast<size_t>(T) * B * ceil_div(nl, kDigInputs) * kDigHalfs);
+        w.zdig = cv.take<uint16_t>(static_cast<size_t>(T + c->D) * B * ceil_div(c->N, spike_bin(c->N)) * kDigHalfs);
+    } else {
+        w.zmask = cv.take<uint32_t>(static_cast<size_t>(T + c->D) * c->Np);
+        w.lmask = cv.take<uint32_t>(static_cast<size_t>(T) * nl);
+        w.abits = cv.take<uint64_t>(static_cast<size_t>(T + c->D) * c->W);
+        w.lbits = cv.take<uint64_t>(static_cast<size_t>(T) * ((nl + 63) / 64));
+        w.I2 = cv.take<float>(2 * BN * c->nb);  // deterministic pull beside the step: two halves
+        if (lgn_ahead(c, B, T)) {
+            w.IL = cv.take<float>(static_cast<size_t>(kLgnRing) * BN * c->nb);
+            w.lgnT = cv.take<uint64_t>(static_cast<size_t>((T + kLgnSeg - 1) / kLgnSeg) * nl * B);
+        }
     }
     w.vsave = cv.take<float>(static_cast<size_t>(T) * BN);
-    w.lgn_off = cv.take<int64_t>(T + 1);
-    w.lgn_pre = cv.take<int32_t>(static_cast<size_t>(T) * nl);
-    w.lgn_mask = cv.take<uint32_t>(static_cast<size_t>(T) * nl);
+    if (!win_forward(c)) {
+        w.lgn_off = cv.take<int64_t>(T + 1);
+        w.lgn_pre = cv.take<int32_t>(static_cast<size_t>(T) * nl);
+        w.lgn_mask = cv.take<uint32_t>(static_cast<size_t>(T) * nl);
+    }
     const int Wwin = win_width(B), nwin = std::max(n_windows(T, Wwin), 1);
     w.lw_off = cv.take<int64_t>(nwin + 1);
     w.lw_pre = cv.take<int32_t>(static_cast<size_t>(nwin) * nl);
@@ -200,7 +221,8 @@ static CellWs carve_cell(void *ws, const Cell *c, int32_t B, int32_t T, size_t *
     w.dw_rec = cv.take<float>(std::max<int64_t>(c->rec->n_syn, 1));
     w.dw_lgn = cv.take<float>(std::max<int64_t>(c->lgn->n_syn, 1));
     w.dw_bkg = cv.take<float>(std::max<int64_t>(c->bkg->n_syn, 1));
-    w.I = cv.take<float>(2 * BN * i_slots(c));   // event mode alternates between the two halves by tick
+    // event mode alternates between the two halves by tick
+    if (!win_forward(c)) w.I = cv.take<float>(2 * BN * i_slots(c));
     if (bytes) *bytes = cv.off;
     return w;
 }
@@ -852,6 +874,284 @@ k_step_push(StepArgs sa, int step_blocks, PushArgs pa) {
         step_body<false, NB>(sa, bid - push_blocks);
 }
 
+// --------------------------------------------------- forward by windows ----
+// V_t takes the PSC of t - 1, which takes the rise current of t - 2, which takes the currents
+// of t - 2: a spike of tick s first matters to the voltage of tick s + 3.  So three ticks are
+// stepped per launch, and the state is read and written once for them: the launch of ticks
+// [t0, t0 + nw) sums the currents of ticks i_lo = t0 - 2 .. i_hi - 1 <= t0, all of which follow
+// from spikes before t0, and holds R at tick i_hi - 1 and P one tick further when it ends.  The
+// windows are laid out so that the last one is a single tick: its currents then reach T - 1 and
+// R and P end there too (flush).
+//
+// A workgroup owns n_own posts of one batch entry: it sums their currents in LDS lists
+// (win_kernels.h), so nothing but spike words passes between workgroups, then steps them in
+// registers.  Both modes run it: the sums are the reference's, term by term.
+struct WinArgs {
+    CellConst k;
+    int32_t t0, nw, flush;
+    int32_t i_lo, i0, i1;          // current ticks i_lo + i0 .. i_lo + i1 - 1, i_lo = t0 - 2
+    int32_t RP, n_ranges;          // posts per workgroup, ranges of them
+    int32_t count_t0, count_t1;
+    WinSrc rec, lgn;
+    uint16_t *dig;                 // rec's digests, written for the window's ticks
+    float *v;
+    int16_t *r;
+    float *A, *R, *P;
+    const float *decay, *cf, *ad, *amp;
+    const int32_t *tref;
+    uint64_t *zbits, *refbits;
+    float *vsave, *z_out, *v_out;
+    int32_t *spike_count;
+    const int32_t *bkg_row;
+    const uint32_t *bkg_pd;
+    const uint8_t *bkg_sid;
+    const float *bkg_w;
+    const uint2 *bkg_ell;
+    int32_t bkg_ell_len, n_bkg;
+    const uint8_t *bkg;            // [T][B][n_bkg]
+    const float *basis;
+};
+
+// Background currents of post n0 + local at the launch's current ticks: every synapse of the row, weight
+// times the tick's Poisson count.  A zero count adds +/-0, which leaves a sum started at +0
+// unchanged, so the sum equals the reference's event-only one bit for bit.  cnt: the ticks'
+// counts of every input, a byte each, in LDS; nullptr: read from a.bkg.
+template <int NB>
+__device__ inline void win_bkg(const WIN_CONST WinArgs &a, const float *basis_lds, const uint32_t *cnt, int n0, uint32_t local, int b,
+                               float (&Ib)[kWinTicks][NB]) {
+    constexpr int BS = win_basis_stride(NB);
+#pragma unroll
+    for (int i = 0; i < kWinTicks; ++i)
+#pragma unroll
+        for (int q = 0; q < NB; ++q) Ib[i][q] = 0.0f;
+    const uint8_t *xb = a.bkg + (static_cast<int64_t>(a.i_lo + a.i0) * a.k.B + b) * a.n_bkg;   // tick i_lo + i0
+    const int64_t tick = static_cast<int64_t>(a.k.B) * a.n_bkg;
+    const int32_t j0 = a.bkg_ell ? 0 : (a.bkg_row + n0)[local], j1 = a.bkg_ell ? a.bkg_ell_len : (a.bkg_row + n0)[local + 1];
+    constexpr int U = 4;   // entries loaded together
+#pragma unroll 1
+    for (int32_t jb = j0; jb < j1; jb += U) {
+        uint2 e[U];        // {input | syn_id << 24, weight bits}
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int32_t j = min(jb + u, j1 - 1);
+            if (a.bkg_ell) e[u] = (a.bkg_ell + (static_cast<int64_t>(j) * a.k.N + n0))[local];
+            else e[u] = make_uint2((a.bkg_pd[j] & kLow24) | static_cast<uint32_t>(a.bkg_sid[j]) << 24,
+                                   __float_as_uint(a.bkg_w[j]));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (jb + u >= j1) break;
+            const uint32_t pre = e[u].x & kLow24;
+            uint32_t c = 0;
+            if (cnt) c = cnt[pre];
+            else
+                for (int i = a.i0; i < a.i1; ++i) c |= static_cast<uint32_t>(xb[(i - a.i0) * tick + pre]) << (8 * i);
+            const float *bs = basis_lds + (e[u].x >> 24) * BS;
+#pragma unroll
+            for (int i = 0; i < kWinTicks; ++i) {
+                const float wv = __uint_as_float(e[u].y) * static_cast<float>((c >> (8 * i)) & 0xFFu);
+#pragma unroll
+                for (int q = 0; q < NB; ++q) Ib[i][q] = Ib[i][q] + wv * bs[q];
+            }
+        }
+    }
+}
+
+// Bound by the latency of its chain (digests, visits' offsets, entries, state) and by instruction
+// issue, two thirds of its wave cycles waiting: 41 us per launch of three ticks at 66,000 neurons,
+// batch 5, 5 Hz, 250 synapses per neuron, where the launches per tick it
+// replaced took 28 us each with the LGN events' passes beside them; deterministic at batch 32: 270
+// against 3 x 240 us.  One thread per post and 6 waves per SIMD (two workgroups of 704 - 768
+// threads per CU) keep the event form in 80 registers without spills; SPLIT's second set of sums
+// spills there (4.8 against 3.6 ms for 40 ticks at batch 32), so it runs one workgroup per CU.  Not kept:
+// two posts per thread in 512 threads (71 us), 256 threads that loop over their posts (111 us), the
+// state loaded ahead of the currents (spills: 69 us).
+template <int NB, bool SPLIT>
+__global__ void __launch_bounds__(kWinMaxThreads) __attribute__((amdgpu_waves_per_eu(NB <= 5 ? (SPLIT ? 3 : 6) : 3))) k_win_fwd(WinArgs) {
+    // the arguments where the kernel finds them, read when they are used: taken by value, all of
+    // them are loaded at the start and spill
+    const WIN_CONST WinArgs &a = *(const WIN_CONST WinArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    extern __shared__ __align__(16) char win_smem[];
+    constexpr int L = (SPLIT ? 2 : 1) * kWinTicks;
+    const WinLds l = WinLds::carve(win_smem, blockDim.x, L, a.RP);
+    const WIN_CONST CellConst &k = a.k;
+    // XCD-aware order (workgroups go to the 8 XCDs round robin): an XCD takes all batch entries of
+    // consecutive ranges, which look up the same ranges' rows
+    const int per = static_cast<int>(gridDim.x) / 8;
+    const int wg = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
+    if (wg >= a.n_ranges * k.B) return;
+    const int range = wg / k.B, b = wg - range * k.B;
+    const int n0 = range * a.RP;
+    for (int i = threadIdx.x; i < L * a.RP; i += blockDim.x) l.heads[i] = -1;
+    for (int i = threadIdx.x; i < k.n_types * NB; i += blockDim.x)
+        l.basis[i / NB * win_basis_stride(NB) + i % NB] = a.basis[i];
+    __syncthreads();
+    const int64_t BN = static_cast<int64_t>(k.B) * k.N;
+    float I[L][NB];
+#pragma unroll
+    for (int i = 0; i < L; ++i)
+#pragma unroll
+        for (int q = 0; q < NB; ++q) I[i][q] = 0.0f;
+    // the entries' room, free once the currents are summed: spike words, background counts
+    uint64_t *new_words = reinterpret_cast<uint64_t *>(l.rec);   // [tick][RP / 64]
+    uint32_t *room = reinterpret_cast<uint32_t *>(l.rec) + 2 * kWinTicks * (kWinMaxThreads / kWave);
+    const bool cnt_lds = a.n_bkg <= 2 * kWinSlots * static_cast<int>(blockDim.x) - 2 * kWinTicks * (kWinMaxThreads / kWave);
+    if (a.i1 > a.i0) {
+        win_currents<NB, SPLIT>(a.rec, a.lgn, l, k.B, b, a.i_lo, a.i0, a.i1, range, a.RP, I);
+        if (cnt_lds) {
+            for (int i = threadIdx.x; i < a.n_bkg; i += blockDim.x) {
+                uint32_t c = 0;
+                for (int u = a.i0; u < a.i1; ++u)
+                    c |= static_cast<uint32_t>(a.bkg[(static_cast<int64_t>(a.i_lo + u) * k.B + b) * a.n_bkg + i]) << (8 * u);
+                room[i] = c;
+            }
+            __syncthreads();
+        }
+    }
+    // uniform 64-bit offsets and 32-bit lane offsets: scalar-base addresses
+    const uint32_t local = threadIdx.x, lane = local & (kWave - 1);
+    const int64_t bn0 = static_cast<int64_t>(b) * k.N + n0;
+    const int wave0 = __builtin_amdgcn_readfirstlane(static_cast<int>(local)) & ~(kWave - 1);
+    if (wave0 < a.RP && n0 + wave0 < k.Np) {   // whole waves
+        const int n = n0 + static_cast<int>(local);
+        const bool live = n < k.N;
+        float in[kWinTicks][NB], R[NB], P[NB];
+        float A0 = 0.0f, A1 = 0.0f, v = 0.0f, decay = 0.0f, cf = 0.0f, ad0 = 0.0f, ad1 = 0.0f, am0 = 0.0f, am1 = 0.0f;
+        int r = 0, tref = 0, spikes = 0;
+        bool z = false;
+        if (live) {
+#pragma unroll
+            for (int q = 0; q < NB; ++q) {
+                R[q] = (a.R + (q * BN + bn0))[local];
+                P[q] = (a.P + (q * BN + bn0))[local];
+            }
+            A0 = (a.A + bn0)[local];
+            A1 = (a.A + (BN + bn0))[local];
+            v = (a.v + bn0)[local];
+            r = (a.r + bn0)[local];
+            decay = (a.decay + n0)[local];
+            cf = (a.cf + n0)[local];
+            ad0 = (a.ad + 2 * n0)[2 * local];
+            ad1 = (a.ad + 2 * n0)[2 * local + 1];
+            am0 = (a.amp + 2 * n0)[2 * local];
+            am1 = (a.amp + 2 * n0)[2 * local + 1];
+            tref = (a.tref + n0)[local];
+            z = (a.zbits[(static_cast<int64_t>(a.t0 - 1 + k.D) * k.B + b) * k.W + (n0 + wave0) / kWave] >> lane) & 1ull;
+            if (a.i1 > a.i0) win_bkg<NB>(a, l.basis, cnt_lds ? room : nullptr, n0, local, b, in);
+            // the input of R: (I_rec + I_lgn) + I_bkg, times lr_scale (models.py:896-931, 979-990)
+#pragma unroll
+            for (int i = 0; i < kWinTicks; ++i)
+#pragma unroll
+                for (int q = 0; q < NB; ++q) {
+                    const float x = SPLIT ? I[i][q] + I[L - kWinTicks + i][q] : I[i][q];
+                    in[i][q] = (x + in[i][q]) * k.lr;
+                }
+        }
+        auto rise = [&](int i) {
+#pragma unroll
+            for (int q = 0; q < NB; ++q) R[q] = R[q] * k.sd[q] + in[i][q] * k.p0[q];
+        };
+        auto psc = [&]() {
+#pragma unroll
+            for (int q = 0; q < NB; ++q) P[q] = P[q] * k.sd[q] + k.dtsd[q] * R[q];
+        };
+#pragma unroll
+        for (int w = 0; w < kWinTicks; ++w) {
+            if (w >= a.nw) break;
+            const int t = a.t0 + w;
+            bool refr = false, spike = false;
+            if (live) {
+                // tick t takes P of t - 1, which takes R of t - 2
+                if (t >= 2) rise(w);
+                if (t >= 1) psc();
+                const float zp = z ? 1.0f : 0.0f;
+                float c1 = P[0];
+#pragma unroll
+                for (int q = 1; q < NB; ++q) c1 = c1 + P[q];
+                c1 = c1 + (A0 + A1);
+                const float dv = v * k.om + v * k.vgd;
+                v = (decay * dv + cf * c1) - zp;
+                A0 = ad0 * A0 + zp * am0;
+                A1 = ad1 * A1 + zp * am1;
+                r = max(r + (z ? tref : 0) - 1, 0);
+                refr = r > 0;
+                if (k.hard_reset && refr) v = 0.0f;
+                spike = !refr && (v - 1.0f) > 0.0f;
+                const int64_t tb = static_cast<int64_t>(t) * BN + bn0;
+                (a.vsave + tb)[local] = v;
+                if (a.z_out) (a.z_out + tb)[local] = spike ? 1.0f : 0.0f;
+                if (a.v_out) (a.v_out + tb)[local] = v;
+                if (spike && t >= a.count_t0 && t < a.count_t1) ++spikes;
+                z = spike;
+            }
+            const uint64_t zb = __ballot(spike), rb = __ballot(refr);
+            if (lane == 0) {
+                const int64_t word = static_cast<int64_t>(b) * k.W + (n0 + wave0) / kWave;
+                a.zbits[static_cast<int64_t>(t + k.D) * k.B * k.W + word] = zb;
+                a.refbits[static_cast<int64_t>(t) * k.B * k.W + word] = rb;
+                new_words[w * (a.RP / kWave) + wave0 / kWave] = zb;
+            }
+        }
+        if (live) {
+            if (a.flush) {
+                // t0 = T - 1, the only tick: R of T - 2, P of T - 1, R of T - 1
+                if (a.t0 >= 1) rise(1);
+                psc();
+                rise(2);
+            }
+#pragma unroll
+            for (int q = 0; q < NB; ++q) {
+                (a.R + (q * BN + bn0))[local] = R[q];
+                (a.P + (q * BN + bn0))[local] = P[q];
+            }
+            (a.A + bn0)[local] = A0;
+            (a.A + (BN + bn0))[local] = A1;
+            (a.v + bn0)[local] = v;
+            (a.r + bn0)[local] = static_cast<int16_t>(r);
+            if (a.spike_count && spikes) (a.spike_count + bn0)[local] += spikes;
+        }
+    }
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < a.nw) {
+        const int t = a.t0 + static_cast<int>(threadIdx.x);
+        win_digest(new_words + threadIdx.x * (a.RP / kWave), (min(a.RP, k.Np - n0)) / kWave,
+                   a.dig + ((static_cast<int64_t>(t + k.D) * k.B + b) * a.rec.n_seg + range) * kDigHalfs);
+    }
+}
+
+// The digests of rows of spike words (win_kernels.h): the initial history's, the LGN inputs'.
+__global__ void __launch_bounds__(kBlock)
+    k_digests(const uint64_t *__restrict__ words, int64_t rows, int32_t W, int32_t seg, int32_t n_seg,
+              uint16_t *__restrict__ dig) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= rows * n_seg) return;
+    const int64_t row = i / n_seg;
+    const int32_t w0 = static_cast<int32_t>(i - row * n_seg) * (seg / kWave);
+    win_digest(words + row * W + w0, min(seg / kWave, W - w0), dig + i * kDigHalfs);
+}
+
+// bits[row][w]: bit i of word w = x[row][64 w + i] > 0.  A thread per 8 inputs.
+__global__ void __launch_bounds__(kBlock)
+    k_pack_bits(const uint8_t *__restrict__ x, int64_t rows, int32_t n_in, int32_t W, int wide, uint8_t *__restrict__ bits) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t per = static_cast<int64_t>(W) * 8;
+    if (i >= rows * per) return;
+    const int64_t row = i / per;
+    const int32_t c = static_cast<int32_t>(i - row * per) * 8;
+    const uint8_t *p = x + row * n_in + c;
+    uint32_t m = 0;
+    if (wide && c + 8 <= n_in) {   // rows and x are multiples of 8 bytes
+        const uint64_t v = *reinterpret_cast<const uint64_t *>(p);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) m |= ((v >> (8 * u)) & 0xFFull) != 0ull ? 1u << u : 0u;
+    } else {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (c + u < n_in && p[u] != 0) m |= 1u << u;
+    }
+    bits[i] = static_cast<uint8_t>(m);
+}
+
 // ------------------------------------------------- voltage regularization ----
 // VoltageRegularization (loss_functions.py:1047-1119): penalty of the cell's output
 // voltage, range mode relu(|v - 0.5| - 0.5)^2 (zero inside [0, 1]), threshold mode
@@ -1450,6 +1750,25 @@ static void launch_pull_step(const PullArgs &pa, int pull_blocks, const StepArgs
     }
 }
 
+static void launch_win_fwd(const WinArgs &wa, bool split, int nb, dim3 grid, int threads, size_t lds, hipStream_t s) {
+    auto launch = [&](auto kernel) {
+        if (lds > 65536 && wa.t0 == 0)
+            (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      static_cast<int>(lds));
+        GLIF_PROF_LAUNCH(kernel, grid, dim3(threads), lds, s, wa);
+    };
+    switch (nb) {
+#define GLIF_WIN(NB)                                 \
+    case NB:                                         \
+        if (split) launch(k_win_fwd<NB, true>);    \
+        else launch(k_win_fwd<NB, false>);           \
+        break;
+        GLIF_WIN(1) GLIF_WIN(2) GLIF_WIN(3) GLIF_WIN(4) GLIF_WIN(5) GLIF_WIN(6) GLIF_WIN(7) GLIF_WIN(8)
+#undef GLIF_WIN
+        default: break;
+    }
+}
+
 static void launch_r_last(const StepArgs &sa, int nb, dim3 grid, size_t lds, hipStream_t s) {
     switch (nb) {
 #define GLIF_R_LAST(NB) \
@@ -1576,216 +1895,92 @@ static int plan_g_rows(Cell *c) {
     return GLIF_OK;
 }
 
+// The T-step forward, kWinTicks ticks per launch (k_win_fwd).
+static int forward_windows(Cell *c, int32_t B, int32_t T, bool split, const uint8_t *lgn, const uint8_t *bkg, glif_state *st,
+                           float *z_out, float *v_out, int32_t *spike_count, const CellWs &w, const CellConst &k,
+                           hipStream_t s) {
+    const Table *tr = c->rec, *tl = c->lgn, *tb = c->bkg;
+    const int32_t n_lgn = static_cast<int32_t>(tl->n_cols), Wl = (n_lgn + 63) / 64, n_lseg = ceil_div(n_lgn, kDigInputs);
+    if (tl->n_syn) {
+        const int64_t rows = static_cast<int64_t>(T) * B, n = rows * Wl * 8;
+        const int wide = n_lgn % 8 == 0 && reinterpret_cast<uintptr_t>(lgn) % 8 == 0;
+        hipLaunchKernelGGL(k_pack_bits, dim3(ceil_div(n, kBlock)), dim3(kBlock), 0, s, lgn, rows, n_lgn, Wl, wide,
+                           reinterpret_cast<uint8_t *>(w.lgnbits));
+        GLIF_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_digests, dim3(ceil_div(rows * n_lseg, kBlock)), dim3(kBlock), 0, s, w.lgnbits,
+                           rows, Wl, kDigInputs, n_lseg, w.lgndig);
+        GLIF_HIP(hipGetLastError());
+    }
+    WinArgs a{};
+    a.k = k;
+    a.RP = spike_bin(c->N);
+    a.n_ranges = ceil_div(c->N, a.RP);
+    hipLaunchKernelGGL(k_digests, dim3(ceil_div(static_cast<int64_t>(c->D) * B * a.n_ranges, kBlock)), dim3(kBlock), 0,
+                       s, w.zbits, static_cast<int64_t>(c->D) * B, c->W, a.RP, a.n_ranges, w.zdig);
+    GLIF_HIP(hipGetLastError());
+    a.dig = w.zdig;
+    a.count_t0 = c->trim_pre;
+    a.count_t1 = T - c->trim_post;
+    a.rec = WinSrc{w.zbits, w.zdig, tr->spk.off, tr->spk.ent, c->W, c->N, tr->spk.rows, c->D, c->D, a.RP, a.n_ranges};
+    a.lgn = WinSrc{w.lgnbits, w.lgndig, tl->spk.off, tl->spk.ent, Wl, n_lgn, tl->spk.rows, 0, 0, kDigInputs, n_lseg};
+    a.v = st->v;
+    a.r = st->r;
+    a.A = w.A;
+    a.R = w.R;
+    a.P = w.P;
+    a.decay = c->decay;
+    a.cf = c->cf;
+    a.ad = c->asc_decay;
+    a.amp = c->asc_amps;
+    a.tref = c->tref;
+    a.zbits = w.zbits;
+    a.refbits = w.refbits;
+    a.vsave = w.vsave;
+    a.z_out = z_out;
+    a.v_out = v_out;
+    a.spike_count = spike_count;
+    a.bkg_row = tb->row_ptr;
+    a.bkg_pd = tb->pd;
+    a.bkg_sid = tb->sid_row;
+    a.bkg_w = tb->w_row;
+    a.bkg_ell = tb->ell_len ? tb->ell_pw : nullptr;
+    a.bkg_ell_len = tb->ell_len;
+    a.n_bkg = static_cast<int32_t>(tb->n_cols);
+    a.bkg = bkg;
+    a.basis = tr->basis;
+    // a thread per post, and per digest that a launch lists
+    const int64_t digs = static_cast<int64_t>(c->D + kWinTicks - 1) * a.n_ranges + static_cast<int64_t>(kWinTicks) * n_lseg;
+    const int threads = static_cast<int>(std::min<int64_t>(
+        kWinMaxThreads, std::max<int64_t>(256, ceil_div(std::max<int64_t>(a.RP, digs), kWave) * kWave)));
+    const size_t lds = WinLds::bytes(threads, split ? 2 * kWinTicks : kWinTicks, a.RP, c->n_types, c->nb);
+    const dim3 grid(8 * ceil_div(static_cast<int64_t>(a.n_ranges) * B, 8));
+    for (int t0 = 0, nw = 0; t0 < T; t0 += nw) {
+        // windows of kWinTicks ticks, the first one shorter so that the last is tick T - 1 alone
+        const int before = T - 1 - t0;
+        nw = before == 0 ? 1 : (before % kWinTicks ? before % kWinTicks : kWinTicks);
+        a.t0 = t0;
+        a.nw = nw;
+        a.flush = before == 0;
+        a.i_lo = t0 - 2;
+        a.i0 = std::max(0, -a.i_lo);
+        a.i1 = std::max(a.flush ? kWinTicks : nw, a.i0);
+        ProfScope p(kProfStep, s, true);
+        launch_win_fwd(a, split, c->nb, grid, threads, lds, s);
+    }
+    GLIF_HIP(hipGetLastError());
+    return GLIF_OK;
+}
+
 static int chunks_for(const Table *t, int L) {
     return std::max(1, ceil_div(std::max(t->max_col_len, 1), static_cast<int64_t>(L) * kChunkIters));
 }
 
-}  // namespace glif
-
-using namespace glif;
-
-// ------------------------------------------------------- one step's backward ----
-// The gradient of one V1Column.call (models.py:1059-1135) as the reference's tape takes it
-// when the Keras RNN runs the cell step by step: from the gradients of the step's outputs
-// (z, v) and of its new state to those of its old state and of the three weight vectors.
-// Per (b, n), with V' the step's voltage and r' its refractory counter:
-//   gV'   = [r' == 0] gz psi(V' - 1) + dL/dv + dL/dv_state,  gz = dL/dz + dL/dz_buf'[slot 0]
-//           (zero where r' > 0 under hard reset, whose where() cuts the path)
-//   gv    = (gV' decay)(1 - vgd)                       (straight_through_dampen(v, vgd))
-//   gasc_j = gasc'_j asc_decay_j + gV' cf              (c1 = sum P + sum asc, old P and asc)
-//   gP_r  = gP'_r sd_r + gV' cf
-//   gR_r  = gR'_r sd_r + gP'_r (dt sd_r)               (P' = P sd + (dt sd) R)
-//   dy_r  = (gR'_r p0_r) lr                            (R' = R sd + (I lr) p0)
-// dy then goes through the synaptic op's gradient (glif_syn_bwd): dz over all recurrent
-// synapses, scaled by rd (straight_through_dampen(z_buf, 1 - rd)) and added to the shifted
-// dL/dz_buf' (z_buf' = [z, z_buf[:, :-N]]), and the weight gradients of the step's events.
-struct StepAdjArgs {
-    CellConst k;
-    const float *decay, *cf, *asc_decay;
-    const float *v_new;
-    const int16_t *r_new;
-    const float *gz, *gv;                                   // [B][N] (nullable)
-    const float *gzb_new, *gv_new, *gasc_new, *gR_new, *gP_new;  // the new state's (nullable)
-    float *gv_old, *gasc_old, *gR_old, *gP_old;             // the old state's (nullable)
-    float *dy;                                              // [B * N][nb]
-};
-
-__global__ void __launch_bounds__(kBlock) k_step_adj(StepAdjArgs a) {
-    const CellConst &k = a.k;
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= static_cast<int64_t>(k.B) * k.N) return;
-    const int n = static_cast<int>(i % k.N);
-    const int64_t b = i / k.N;
-    const bool refr = a.r_new[i] > 0;
-    float gzz = a.gz ? a.gz[i] : 0.0f;
-    if (a.gzb_new) gzz = gzz + a.gzb_new[b * k.D * k.N + n];
-    float gV = 0.0f;
-    if (!refr) {
-        const float vsc = a.v_new[i] - 1.0f;
-        float psi;
-        if (k.pseudo_gauss) {
-            const float q = -(vsc * vsc) / (k.gauss_std * k.gauss_std);
-            psi = expf(q) * k.damp;
-        } else {
-            const float m = 1.0f - fabsf(vsc);
-            psi = k.damp * (m > 0.0f ? m : 0.0f);
-        }
-        gV = gzz * psi;
-    }
-    if (a.gv) gV = gV + a.gv[i];
-    if (a.gv_new) gV = gV + a.gv_new[i];
-    if (k.hard_reset && refr) gV = 0.0f;
-    if (a.gv_old) a.gv_old[i] = (gV * a.decay[n]) * k.om;
-    const float gc = gV * a.cf[n];
-    if (a.gasc_old)
-        for (int j = 0; j < 2; ++j)
-            a.gasc_old[i * 2 + j] = (a.gasc_new ? a.gasc_new[i * 2 + j] * a.asc_decay[n * 2 + j] : 0.0f) + gc;
-    for (int q = 0; q < k.nb; ++q) {
-        const int64_t e = i * k.nb + q;
-        const float gRn = a.gR_new ? a.gR_new[e] : 0.0f;
-        const float gPn = a.gP_new ? a.gP_new[e] : 0.0f;
-        if (a.gP_old) a.gP_old[e] = gPn * k.sd[q] + gc;
-        if (a.gR_old) a.gR_old[e] = gRn * k.sd[q] + gPn * k.dtsd[q];
-        a.dy[e] = (gRn * k.p0[q]) * k.lr;
-    }
-}
-
-// gzb[b][c] = rd * dz[b][c] + dL/dz_buf'[b][c + N] (the shifted slots; the last slot has none)
-__global__ void __launch_bounds__(kBlock)
-    k_step_zbuf_grad(float *__restrict__ gzb, const float *__restrict__ gzb_new, int64_t n, int64_t DN, int32_t N,
-                     float rd) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float g = gzb[i] * rd;
-    if (gzb_new && i % DN < DN - N) g = g + gzb_new[i + N];
-    gzb[i] = g;
-}
-
-__global__ void __launch_bounds__(kBlock) k_u8_to_f32(float *__restrict__ dst, const uint8_t *__restrict__ src,
-                                                        int64_t n) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = static_cast<float>(src[i]);
-}
-
-struct StepWs {
-    float *dy;      // [B * N][nb]
-    float *xl, *xk; // the step's LGN spikes and background counts as floats
-    float *G;       // the op gradients' projection, shared by the tables whose G layouts agree
-};
-
-static StepWs carve_step(void *ws, const Cell *c, int32_t B, size_t *bytes) {
-    Carver cv(ws, SIZE_MAX);
-    StepWs w{};
-    const int64_t BN = static_cast<int64_t>(B) * c->N;
-    w.dy = cv.take<float>(BN * c->nb);
-    w.xl = cv.take<float>(std::max<int64_t>(static_cast<int64_t>(B) * c->lgn->n_cols, 1));
-    w.xk = cv.take<float>(std::max<int64_t>(static_cast<int64_t>(B) * c->bkg->n_cols, 1));
-    size_t g = 1;
-    for (const Table *t : {c->rec, c->lgn, c->bkg}) g = std::max(g, syn_g_floats(t, B));
-    w.G = cv.take<float>(g);
-    if (bytes) *bytes = cv.off;
-    return w;
-}
-
-extern "C" {
-
-int glif_cell_create(const glif_cell_config *cfg, const float *decay, const float *current_factor,
-                     const float *asc_decay, const float *asc_amps, const int32_t *t_ref_steps,
-                     const float *syn_decay, const float *psc_initial, glif_table *rec, glif_table *lgn,
-                     glif_table *bkg, glif_cell **out) {
-    if (!cfg || !out || !rec || !lgn || !bkg || !decay || !current_factor || !asc_decay || !asc_amps ||
-        !t_ref_steps || !syn_decay || !psc_initial)
-        return fail(GLIF_EINVAL, "NULL argument");
-    *out = nullptr;
-    Table *tr = reinterpret_cast<Table *>(rec), *tl = reinterpret_cast<Table *>(lgn),
-          *tb = reinterpret_cast<Table *>(bkg);
-    const int N = cfg->n_neurons, D = cfg->n_delay, nb = cfg->n_basis;
-    if (N <= 0 || N >= (1 << 24)) return fail(GLIF_EINVAL, "n_neurons must be in [1, 2^24)");
-    if (D <= 0 || D > 256) return fail(GLIF_EINVAL, "n_delay must be in [1, 256]");
-    if (nb <= 0 || nb > kMaxBasis) return fail(GLIF_EINVAL, "n_basis must be in [1, 8]");
-    if (tr->n_post != N || tl->n_post != N || tb->n_post != N)
-        return fail(GLIF_EINVAL, "table n_post differs from n_neurons");
-    if (tr->n_slots != D || tr->n_cols != static_cast<int64_t>(D) * N)
-        return fail(GLIF_EINVAL, "recurrent table must have n_delay slots of n_neurons columns");
-    if (tl->n_slots != 1 || tb->n_slots != 1) return fail(GLIF_EINVAL, "input tables take no delays");
-    for (Table *t : {tr, tl, tb}) {
-        if (t->n_basis != nb || t->n_types != tr->n_types ||
-            std::memcmp(t->basis_host, tr->basis_host, sizeof(float) * tr->n_types * nb) != 0)
-            return fail(GLIF_EINVAL, "all tables must share one basis table");
-    }
-    for (int i = 0; i < N; ++i)
-        if (t_ref_steps[i] < 1 || t_ref_steps[i] > 32767)
-            return fail(GLIF_EINVAL, "t_ref_steps must be in [1, 32767]");
-    Cell *c = new Cell();
-    c->cfg = *cfg;
-    c->N = N;
-    c->Np = (N + kWave - 1) / kWave * kWave;
-    c->W = c->Np / kWave;
-    c->D = D;
-    c->nb = nb;
-    c->n_types = tr->n_types;
-    for (int q = 0; q < nb; ++q) {
-        c->syn_decay[q] = syn_decay[q];
-        c->psc_initial[q] = psc_initial[q];
-        c->dtsd[q] = cfg->dt * syn_decay[q];
-    }
-    c->rec = tr;
-    c->lgn = tl;
-    c->bkg = tb;
-    auto up = [](auto **dst, const auto *src, size_t n) -> hipError_t {
-        hipError_t e = hipMalloc(reinterpret_cast<void **>(dst), n * sizeof(**dst));
-        if (e != hipSuccess) return e;
-        return hipMemcpy(*dst, src, n * sizeof(**dst), hipMemcpyHostToDevice);
-    };
-    hipError_t e;
-    if ((e = up(&c->decay, decay, N)) != hipSuccess || (e = up(&c->cf, current_factor, N)) != hipSuccess ||
-        (e = up(&c->asc_decay, asc_decay, 2 * static_cast<size_t>(N))) != hipSuccess ||
-        (e = up(&c->asc_amps, asc_amps, 2 * static_cast<size_t>(N))) != hipSuccess ||
-        (e = up(&c->tref, t_ref_steps, N)) != hipSuccess) {
-        glif_cell_destroy(reinterpret_cast<glif_cell *>(c));
-        return hip_fail(e, "cell upload");
-    }
-    if (int rc = plan_g_rows(c)) {
-        glif_cell_destroy(reinterpret_cast<glif_cell *>(c));
-        return rc;
-    }
-    *out = reinterpret_cast<glif_cell *>(c);
-    return GLIF_OK;
-}
-
-void glif_cell_destroy(glif_cell *cc) {
-    Cell *c = reinterpret_cast<Cell *>(cc);
-    if (!c) return;
-    release_side(c);
-    for (void *p : {static_cast<void *>(c->decay), static_cast<void *>(c->cf),
-                    static_cast<void *>(c->asc_decay), static_cast<void *>(c->asc_amps),
-                    static_cast<void *>(c->tref), static_cast<void *>(c->g_type)})
-        if (p) (void)hipFree(p);
-    delete c;
-}
-
-size_t glif_cell_workspace(const glif_cell *cc, int32_t B, int32_t T) {
-    if (!cc || B <= 0 || T <= 0) return 0;
-    size_t bytes = 0;
-    carve_cell(nullptr, reinterpret_cast<const Cell *>(cc), B, T, &bytes);
-    return bytes;
-}
-
-int glif_cell_forward(glif_cell *cc, int32_t B, int32_t T, int32_t mode, const uint8_t *lgn,
-                      const uint8_t *bkg, glif_state *st, float *z_out, float *v_out,
-                      int32_t *spike_count, void *ws, size_t ws_bytes, void *stream) {
-    Cell *c = reinterpret_cast<Cell *>(cc);
-    if (!c || !lgn || !bkg || !st || !st->z_buf || !st->v || !st->r || !st->asc || !st->psc_rise || !st->psc)
-        return fail(GLIF_EINVAL, "NULL argument");
-    if (B <= 0 || B > kMaxBatch) return fail(GLIF_EINVAL, "B must be in [1, 32]");
-    if (T <= 0) return fail(GLIF_EINVAL, "T must be > 0");
-    if (mode != GLIF_MODE_EVENT && mode != GLIF_MODE_DETERMINISTIC) return fail(GLIF_EINVAL, "unknown mode");
-    if (!ws || ws_bytes < glif_cell_workspace(cc, B, T)) return fail(GLIF_ENOMEM, "workspace too small");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    CellWs w = carve_cell(ws, c, B, T, nullptr);
-    const CellConst k = make_const(c, B);
-    const bool event = mode == GLIF_MODE_EVENT;
+// The T-step forward, a launch per tick (networks past the window forward's row offsets).
+static int forward_ticks(Cell *c, int32_t B, int32_t T, bool event, const uint8_t *lgn, const uint8_t *bkg,
+                         glif_state *st, float *z_out, float *v_out, int32_t *spike_count, const CellWs &w,
+                         const CellConst &k, hipStream_t s) {
     const Table *tr = c->rec, *tl = c->lgn, *tb = c->bkg;
+    const int64_t BNs = static_cast<int64_t>(B) * c->N;
     int rc;
     // event push into per-type slots ([gk][B][N] per tick) or receptor currents ([nb][B][N])
     const bool typed = event && c->push_typed;
@@ -1798,7 +1993,6 @@ int glif_cell_forward(glif_cell *cc, int32_t B, int32_t T, int32_t mode, const u
     const bool ahead = lgn_ahead(c, B, T) && (!event || (!typed && B >= kLgnEventMinBatch));
     const bool ring_is_I = event && ahead;
 
-    // input lists (LGN push in the forward, LGN / background dW in the backward)
     if (event && !ahead &&
         (rc = build_batch_mask_lists(lgn, T, B, tl->n_cols, w.lgn_off, w.lgn_pre, w.lgn_mask, w.scratch, s)))
         return rc;
@@ -1831,33 +2025,9 @@ int glif_cell_forward(glif_cell *cc, int32_t B, int32_t T, int32_t mode, const u
     la.lgnT = w.lgnT;
     la.basis = tr->basis;
     la.ring = w.IL;
-    const int Wwin = win_width(B), nwin = n_windows(T, Wwin);
-    if (nwin > 0) {
-        if ((rc = build_window_mask_lists(lgn, T, B, tl->n_cols, Wwin, nwin, w.lw_off, w.lw_pre, w.lw_mask,
-                                          w.scratch, s)))
-            return rc;
-        if ((rc = build_window_mask_lists(bkg, T, B, tb->n_cols, Wwin, nwin, w.kw_off, w.kw_pre, w.kw_mask,
-                                          w.scratch, s)))
-            return rc;
-    }
-    GLIF_HIP(hipMemcpyAsync(w.bkg_cnt, bkg, static_cast<size_t>(T) * B * tb->n_cols, hipMemcpyDeviceToDevice, s));
-    // spike history of the initial state
-    const int64_t n_init = static_cast<int64_t>(c->D) * B * c->Np;
-    if (!event && ((rc = launch_fill_u32(w.zmask, 0u, static_cast<size_t>(T + c->D) * c->Np, s)) ||
-                   (rc = launch_fill_u32(w.abits, 0u, static_cast<size_t>(T + c->D) * c->W * 2, s))))
-        return rc;
-    hipLaunchKernelGGL(k_init_history, dim3(ceil_div(n_init, kBlock)), dim3(kBlock), 0, s, st->z_buf, k,
-                       w.zbits, event ? nullptr : w.zmask,
-                       event ? nullptr : w.abits);
-    GLIF_HIP(hipGetLastError());
     const int slots = typed ? c->g_rows : c->nb;
     if (event && !ring_is_I && (rc = launch_fill_u32(w.I, 0u, 2 * static_cast<size_t>(B) * c->N * slots, s)))
         return rc;
-    const int64_t BNs = static_cast<int64_t>(B) * c->N;
-    hipLaunchKernelGGL(k_state_layout, dim3(ceil_div(BNs, kBlock)), dim3(kBlock), 0, s, st->psc_rise, st->psc,
-                       st->asc, w.R, w.P, w.A, BNs, c->nb, 1);
-    GLIF_HIP(hipGetLastError());
-
     const size_t lds = sizeof(float) * c->n_types * c->nb;
     StepArgs sa{};
     sa.k = k;
@@ -2093,6 +2263,246 @@ int glif_cell_forward(glif_cell *cc, int32_t B, int32_t T, int32_t mode, const u
         x.bkg_x = bkg + static_cast<int64_t>(T - 1) * B * tb->n_cols;
         launch_r_last(x, c->nb, step_grid, lds, s);
     }
+    GLIF_HIP(hipGetLastError());
+    return GLIF_OK;
+}
+
+}  // namespace glif
+
+using namespace glif;
+
+// ------------------------------------------------------- one step's backward ----
+// The gradient of one V1Column.call (models.py:1059-1135) as the reference's tape takes it
+// when the Keras RNN runs the cell step by step: from the gradients of the step's outputs
+// (z, v) and of its new state to those of its old state and of the three weight vectors.
+// Per (b, n), with V' the step's voltage and r' its refractory counter:
+//   gV'   = [r' == 0] gz psi(V' - 1) + dL/dv + dL/dv_state,  gz = dL/dz + dL/dz_buf'[slot 0]
+//           (zero where r' > 0 under hard reset, whose where() cuts the path)
+//   gv    = (gV' decay)(1 - vgd)                       (straight_through_dampen(v, vgd))
+//   gasc_j = gasc'_j asc_decay_j + gV' cf              (c1 = sum P + sum asc, old P and asc)
+//   gP_r  = gP'_r sd_r + gV' cf
+//   gR_r  = gR'_r sd_r + gP'_r (dt sd_r)               (P' = P sd + (dt sd) R)
+//   dy_r  = (gR'_r p0_r) lr                            (R' = R sd + (I lr) p0)
+// dy then goes through the synaptic op's gradient (glif_syn_bwd): dz over all recurrent
+// synapses, scaled by rd (straight_through_dampen(z_buf, 1 - rd)) and added to the shifted
+// dL/dz_buf' (z_buf' = [z, z_buf[:, :-N]]), and the weight gradients of the step's events.
+struct StepAdjArgs {
+    CellConst k;
+    const float *decay, *cf, *asc_decay;
+    const float *v_new;
+    const int16_t *r_new;
+    const float *gz, *gv;                                   // [B][N] (nullable)
+    const float *gzb_new, *gv_new, *gasc_new, *gR_new, *gP_new;  // the new state's (nullable)
+    float *gv_old, *gasc_old, *gR_old, *gP_old;             // the old state's (nullable)
+    float *dy;                                              // [B * N][nb]
+};
+
+__global__ void __launch_bounds__(kBlock) k_step_adj(StepAdjArgs a) {
+    const CellConst &k = a.k;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= static_cast<int64_t>(k.B) * k.N) return;
+    const int n = static_cast<int>(i % k.N);
+    const int64_t b = i / k.N;
+    const bool refr = a.r_new[i] > 0;
+    float gzz = a.gz ? a.gz[i] : 0.0f;
+    if (a.gzb_new) gzz = gzz + a.gzb_new[b * k.D * k.N + n];
+    float gV = 0.0f;
+    if (!refr) {
+        const float vsc = a.v_new[i] - 1.0f;
+        float psi;
+        if (k.pseudo_gauss) {
+            const float q = -(vsc * vsc) / (k.gauss_std * k.gauss_std);
+            psi = expf(q) * k.damp;
+        } else {
+            const float m = 1.0f - fabsf(vsc);
+            psi = k.damp * (m > 0.0f ? m : 0.0f);
+        }
+        gV = gzz * psi;
+    }
+    if (a.gv) gV = gV + a.gv[i];
+    if (a.gv_new) gV = gV + a.gv_new[i];
+    if (k.hard_reset && refr) gV = 0.0f;
+    if (a.gv_old) a.gv_old[i] = (gV * a.decay[n]) * k.om;
+    const float gc = gV * a.cf[n];
+    if (a.gasc_old)
+        for (int j = 0; j < 2; ++j)
+            a.gasc_old[i * 2 + j] = (a.gasc_new ? a.gasc_new[i * 2 + j] * a.asc_decay[n * 2 + j] : 0.0f) + gc;
+    for (int q = 0; q < k.nb; ++q) {
+        const int64_t e = i * k.nb + q;
+        const float gRn = a.gR_new ? a.gR_new[e] : 0.0f;
+        const float gPn = a.gP_new ? a.gP_new[e] : 0.0f;
+        if (a.gP_old) a.gP_old[e] = gPn * k.sd[q] + gc;
+        if (a.gR_old) a.gR_old[e] = gRn * k.sd[q] + gPn * k.dtsd[q];
+        a.dy[e] = (gRn * k.p0[q]) * k.lr;
+    }
+}
+
+// gzb[b][c] = rd * dz[b][c] + dL/dz_buf'[b][c + N] (the shifted slots; the last slot has none)
+__global__ void __launch_bounds__(kBlock)
+    k_step_zbuf_grad(float *__restrict__ gzb, const float *__restrict__ gzb_new, int64_t n, int64_t DN, int32_t N,
+                     float rd) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    float g = gzb[i] * rd;
+    if (gzb_new && i % DN < DN - N) g = g + gzb_new[i + N];
+    gzb[i] = g;
+}
+
+__global__ void __launch_bounds__(kBlock) k_u8_to_f32(float *__restrict__ dst, const uint8_t *__restrict__ src,
+                                                        int64_t n) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = static_cast<float>(src[i]);
+}
+
+struct StepWs {
+    float *dy;      // [B * N][nb]
+    float *xl, *xk; // the step's LGN spikes and background counts as floats
+    float *G;       // the op gradients' projection, shared by the tables whose G layouts agree
+};
+
+static StepWs carve_step(void *ws, const Cell *c, int32_t B, size_t *bytes) {
+    Carver cv(ws, SIZE_MAX);
+    StepWs w{};
+    const int64_t BN = static_cast<int64_t>(B) * c->N;
+    w.dy = cv.take<float>(BN * c->nb);
+    w.xl = cv.take<float>(std::max<int64_t>(static_cast<int64_t>(B) * c->lgn->n_cols, 1));
+    w.xk = cv.take<float>(std::max<int64_t>(static_cast<int64_t>(B) * c->bkg->n_cols, 1));
+    size_t g = 1;
+    for (const Table *t : {c->rec, c->lgn, c->bkg}) g = std::max(g, syn_g_floats(t, B));
+    w.G = cv.take<float>(g);
+    if (bytes) *bytes = cv.off;
+    return w;
+}
+
+extern "C" {
+
+int glif_cell_create(const glif_cell_config *cfg, const float *decay, const float *current_factor,
+                     const float *asc_decay, const float *asc_amps, const int32_t *t_ref_steps,
+                     const float *syn_decay, const float *psc_initial, glif_table *rec, glif_table *lgn,
+                     glif_table *bkg, glif_cell **out) {
+    if (!cfg || !out || !rec || !lgn || !bkg || !decay || !current_factor || !asc_decay || !asc_amps ||
+        !t_ref_steps || !syn_decay || !psc_initial)
+        return fail(GLIF_EINVAL, "NULL argument");
+    *out = nullptr;
+    Table *tr = reinterpret_cast<Table *>(rec), *tl = reinterpret_cast<Table *>(lgn),
+          *tb = reinterpret_cast<Table *>(bkg);
+    const int N = cfg->n_neurons, D = cfg->n_delay, nb = cfg->n_basis;
+    if (N <= 0 || N >= (1 << 24)) return fail(GLIF_EINVAL, "n_neurons must be in [1, 2^24)");
+    if (D <= 0 || D > 256) return fail(GLIF_EINVAL, "n_delay must be in [1, 256]");
+    if (nb <= 0 || nb > kMaxBasis) return fail(GLIF_EINVAL, "n_basis must be in [1, 8]");
+    if (tr->n_post != N || tl->n_post != N || tb->n_post != N)
+        return fail(GLIF_EINVAL, "table n_post differs from n_neurons");
+    if (tr->n_slots != D || tr->n_cols != static_cast<int64_t>(D) * N)
+        return fail(GLIF_EINVAL, "recurrent table must have n_delay slots of n_neurons columns");
+    if (tl->n_slots != 1 || tb->n_slots != 1) return fail(GLIF_EINVAL, "input tables take no delays");
+    for (Table *t : {tr, tl, tb}) {
+        if (t->n_basis != nb || t->n_types != tr->n_types ||
+            std::memcmp(t->basis_host, tr->basis_host, sizeof(float) * tr->n_types * nb) != 0)
+            return fail(GLIF_EINVAL, "all tables must share one basis table");
+    }
+    for (int i = 0; i < N; ++i)
+        if (t_ref_steps[i] < 1 || t_ref_steps[i] > 32767)
+            return fail(GLIF_EINVAL, "t_ref_steps must be in [1, 32767]");
+    Cell *c = new Cell();
+    c->cfg = *cfg;
+    c->N = N;
+    c->Np = (N + kWave - 1) / kWave * kWave;
+    c->W = c->Np / kWave;
+    c->D = D;
+    c->nb = nb;
+    c->n_types = tr->n_types;
+    for (int q = 0; q < nb; ++q) {
+        c->syn_decay[q] = syn_decay[q];
+        c->psc_initial[q] = psc_initial[q];
+        c->dtsd[q] = cfg->dt * syn_decay[q];
+    }
+    c->rec = tr;
+    c->lgn = tl;
+    c->bkg = tb;
+    auto up = [](auto **dst, const auto *src, size_t n) -> hipError_t {
+        hipError_t e = hipMalloc(reinterpret_cast<void **>(dst), n * sizeof(**dst));
+        if (e != hipSuccess) return e;
+        return hipMemcpy(*dst, src, n * sizeof(**dst), hipMemcpyHostToDevice);
+    };
+    hipError_t e;
+    if ((e = up(&c->decay, decay, N)) != hipSuccess || (e = up(&c->cf, current_factor, N)) != hipSuccess ||
+        (e = up(&c->asc_decay, asc_decay, 2 * static_cast<size_t>(N))) != hipSuccess ||
+        (e = up(&c->asc_amps, asc_amps, 2 * static_cast<size_t>(N))) != hipSuccess ||
+        (e = up(&c->tref, t_ref_steps, N)) != hipSuccess) {
+        glif_cell_destroy(reinterpret_cast<glif_cell *>(c));
+        return hip_fail(e, "cell upload");
+    }
+    if (int rc = plan_g_rows(c)) {
+        glif_cell_destroy(reinterpret_cast<glif_cell *>(c));
+        return rc;
+    }
+    *out = reinterpret_cast<glif_cell *>(c);
+    return GLIF_OK;
+}
+
+void glif_cell_destroy(glif_cell *cc) {
+    Cell *c = reinterpret_cast<Cell *>(cc);
+    if (!c) return;
+    release_side(c);
+    for (void *p : {static_cast<void *>(c->decay), static_cast<void *>(c->cf),
+                    static_cast<void *>(c->asc_decay), static_cast<void *>(c->asc_amps),
+                    static_cast<void *>(c->tref), static_cast<void *>(c->g_type)})
+        if (p) (void)hipFree(p);
+    delete c;
+}
+
+size_t glif_cell_workspace(const glif_cell *cc, int32_t B, int32_t T) {
+    if (!cc || B <= 0 || T <= 0) return 0;
+    size_t bytes = 0;
+    carve_cell(nullptr, reinterpret_cast<const Cell *>(cc), B, T, &bytes);
+    return bytes;
+}
+
+int glif_cell_forward(glif_cell *cc, int32_t B, int32_t T, int32_t mode, const uint8_t *lgn,
+                      const uint8_t *bkg, glif_state *st, float *z_out, float *v_out,
+                      int32_t *spike_count, void *ws, size_t ws_bytes, void *stream) {
+    Cell *c = reinterpret_cast<Cell *>(cc);
+    if (!c || !lgn || !bkg || !st || !st->z_buf || !st->v || !st->r || !st->asc || !st->psc_rise || !st->psc)
+        return fail(GLIF_EINVAL, "NULL argument");
+    if (B <= 0 || B > kMaxBatch) return fail(GLIF_EINVAL, "B must be in [1, 32]");
+    if (T <= 0) return fail(GLIF_EINVAL, "T must be > 0");
+    if (mode != GLIF_MODE_EVENT && mode != GLIF_MODE_DETERMINISTIC) return fail(GLIF_EINVAL, "unknown mode");
+    if (!ws || ws_bytes < glif_cell_workspace(cc, B, T)) return fail(GLIF_ENOMEM, "workspace too small");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    CellWs w = carve_cell(ws, c, B, T, nullptr);
+    const CellConst k = make_const(c, B);
+    const bool event = mode == GLIF_MODE_EVENT;
+    const Table *tl = c->lgn, *tb = c->bkg;
+    int rc;
+    const bool win = win_forward(c);
+    // input lists of the backward's LGN / background dW
+    const int Wwin = win_width(B), nwin = n_windows(T, Wwin);
+    if (nwin > 0) {
+        if ((rc = build_window_mask_lists(lgn, T, B, tl->n_cols, Wwin, nwin, w.lw_off, w.lw_pre, w.lw_mask,
+                                          w.scratch, s)))
+            return rc;
+        if ((rc = build_window_mask_lists(bkg, T, B, tb->n_cols, Wwin, nwin, w.kw_off, w.kw_pre, w.kw_mask,
+                                          w.scratch, s)))
+            return rc;
+    }
+    GLIF_HIP(hipMemcpyAsync(w.bkg_cnt, bkg, static_cast<size_t>(T) * B * tb->n_cols, hipMemcpyDeviceToDevice, s));
+    // spike history of the initial state
+    const int64_t n_init = static_cast<int64_t>(c->D) * B * c->Np;
+    if (!event && !win && ((rc = launch_fill_u32(w.zmask, 0u, static_cast<size_t>(T + c->D) * c->Np, s)) ||
+                   (rc = launch_fill_u32(w.abits, 0u, static_cast<size_t>(T + c->D) * c->W * 2, s))))
+        return rc;
+    hipLaunchKernelGGL(k_init_history, dim3(ceil_div(n_init, kBlock)), dim3(kBlock), 0, s, st->z_buf, k,
+                       w.zbits, event || win ? nullptr : w.zmask,
+                       event || win ? nullptr : w.abits);
+    GLIF_HIP(hipGetLastError());
+    const int64_t BNs = static_cast<int64_t>(B) * c->N;
+    hipLaunchKernelGGL(k_state_layout, dim3(ceil_div(BNs, kBlock)), dim3(kBlock), 0, s, st->psc_rise, st->psc,
+                       st->asc, w.R, w.P, w.A, BNs, c->nb, 1);
+    GLIF_HIP(hipGetLastError());
+
+    if (win) rc = forward_windows(c, B, T, !event, lgn, bkg, st, z_out, v_out, spike_count, w, k, s);
+    else rc = forward_ticks(c, B, T, event, lgn, bkg, st, z_out, v_out, spike_count, w, k, s);
+    if (rc) return rc;
     GLIF_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_state_layout, dim3(ceil_div(BNs, kBlock)), dim3(kBlock), 0, s, st->psc_rise, st->psc,
                        st->asc, w.R, w.P, w.A, BNs, c->nb, 0);

@@ -31,6 +31,11 @@ constexpr int kGsRowBits = 29;
 constexpr uint32_t kGsRowMask = (1u << kGsRowBits) - 1u;
 static_assert(kGsCols < 7, "column-in-group 7 marks padding (3 bits above the row)");
 
+// spike-major rows: delays per row, and the most posts of a range (a workgroup of the window
+// kernels owns a range, a thread per post)
+constexpr int kSpkDelays = 8;
+constexpr int kSpkMaxBin = 768;
+
 // ---- error plumbing -------------------------------------------------------
 void set_error(const std::string &msg);
 int fail(int code, const std::string &msg);
@@ -78,6 +83,17 @@ struct PermPlan {
     uint16_t *off2 = nullptr;  // [n] per destination: staging position - superblock start
     float *mid = nullptr;      // [n] staging of the plan's own, or nullptr (callers pass one)
 };
+
+// Spike-major rows (win_kernels.h), range of `bin` posts by range: row q * n_pre + pre of a range
+// holds the synapses of presynaptic neuron pre onto it with delays kSpkDelays q + 1 .., in
+// ascending (column, synapse id).  rows = 0: not built.
+struct SpikeRows {
+    int32_t bin = 0, rows = 0;  // posts per range, rows per range
+    int32_t *off = nullptr;     // [ranges * rows + 1] first entry of (range, row)
+    uint2 *ent = nullptr;       // [n_syn] {post & 0xFFFF | (delay - 1) % kSpkDelays << 16 | syn_id << 24, weight bits}
+    int32_t *src = nullptr;     // [n_syn] column-grouped position of the synapse
+};
+int32_t spike_bin(int32_t n_post);
 
 struct Table {
     int64_t n_syn = 0;
@@ -147,6 +163,7 @@ struct Table {
     // Each is built only when no post receives more than three quarters of the types.  The
     // type-major copies above stay as they are.
     CompactRows cg, og;
+    SpikeRows spk;
     // two-pass plans (tables of at least kPermMinSyn synapses): the column-grouped weight copy
     // (P = order) and weight gradients from the column-grouped order back to the reference
     // order (P = order_inv)

@@ -245,7 +245,8 @@ static void free_table(Table *t) {
                     t->pd, t->sid_row, t->w_row, t->ph_ptr, t->ph_order, t->ph_pw, t->ell_pw, t->ell_src,
                     t->chunk_desc, t->dwu, t->dzc, t->pidx, t->order_inv, t->ph_inv, t->ph_src, t->gs_seg, t->gs_pw, t->gs_src,
                     t->cg.ps, t->cg.ph_pw, t->cg.gs_seg, t->cg.gs_pw, t->cg.gs_src, t->cg.gtype,
-                    t->og.ps, t->og.ph_pw, t->og.gs_seg, t->og.gs_pw, t->og.gs_src, t->og.gtype};
+                    t->og.ps, t->og.ph_pw, t->og.gs_seg, t->og.gs_pw, t->og.gs_src, t->og.gtype,
+                    t->spk.off, t->spk.ent, t->spk.src};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     delete[] t->basis_host;
@@ -375,6 +376,62 @@ static int build_own_rows(Table *t, const int32_t *col_ptr, const uint32_t *ps, 
     int rc;
     if ((rc = build_compact(t, col_ptr, ps, ph_src, rank.data(), gk, t->og))) return rc;
     return upload(&t->og.gtype, gtype.data(), gtype.size());
+}
+
+// Offsets a table's spike-major rows may take: 1 GB of them (past that the per-tick kernels of
+// cell.hip serve the table).
+constexpr int64_t kSpkMaxOff = int64_t(1) << 28;
+
+// Posts per range of a population of n_post, whole waves of them: 48 ranges for a small one, 94
+// for a column (66,000: 704 posts, two workgroups of the window kernels per CU at batch 5), more
+// past kSpkMaxBin posts each.  Every range looks up every spike, so fewer, larger ranges cost
+// less until the chip is no longer filled.
+int32_t spike_bin(int32_t n_post) {
+    const int32_t want = std::max((n_post + 93) / 94, std::min((n_post + 47) / 48, 384));
+    return std::min(kSpkMaxBin, (want + kWave - 1) / kWave * kWave);
+}
+
+// The spike-major rows from the column-grouped order (ps[k] = post | syn_id << 24): a stable
+// counting sort of its synapses, row by row in ascending (column, id), by (range, row).
+static int build_spike_rows(Table *t, const int32_t *col_ptr, const uint32_t *ps) {
+    const int32_t bin = spike_bin(t->n_post), nf = (t->n_post + bin - 1) / bin;
+    const int64_t groups = (t->n_slots + kSpkDelays - 1) / kSpkDelays, rows = groups * t->n_pre;
+    if (t->n_syn == 0 || rows * nf > kSpkMaxOff) return GLIF_OK;
+    std::vector<int32_t> off(rows * nf + 1, 0), src(t->n_syn);
+    std::vector<uint2> ent(t->n_syn);
+    std::vector<int32_t> at(nf);
+    // f(column position, range) over a row's synapses in ascending (column, id)
+    auto each = [&](int64_t row, auto &&f) {
+        const int64_t q = row / t->n_pre, pre = row - q * t->n_pre;
+        const int64_t d_end = std::min<int64_t>(t->n_slots, (q + 1) * kSpkDelays);
+        for (int64_t d = q * kSpkDelays; d < d_end; ++d) {
+            const int64_t c = d * t->n_pre + pre;
+            for (int32_t k = col_ptr[c]; k < col_ptr[c + 1]; ++k) f(k, d, (ps[k] & kLow24) / bin);
+        }
+    };
+    for (int64_t row = 0; row < rows; ++row) {
+        each(row, [&](int32_t, int64_t, int32_t f) { ++at[f]; });
+        for (int32_t f = 0; f < nf; ++f) {
+            off[f * rows + row + 1] = at[f];
+            at[f] = 0;
+        }
+    }
+    for (int64_t i = 0; i < rows * nf; ++i) off[i + 1] += off[i];
+    for (int64_t row = 0; row < rows; ++row) {
+        each(row, [&](int32_t k, int64_t d, int32_t f) {
+            const int32_t i = off[f * rows + row] + at[f]++;
+            ent[i] = make_uint2((ps[k] & 0xFFFFu) | static_cast<uint32_t>(d % kSpkDelays) << 16 | (ps[k] >> 24) << 24, 0u);
+            src[i] = k;
+        });
+        std::fill(at.begin(), at.end(), 0);
+    }
+    int rc;
+    if ((rc = upload(&t->spk.off, off.data(), off.size())) || (rc = upload(&t->spk.ent, ent.data(), ent.size())) ||
+        (rc = upload(&t->spk.src, src.data(), src.size())))
+        return rc;
+    t->spk.bin = bin;
+    t->spk.rows = static_cast<int32_t>(rows);
+    return GLIF_OK;
 }
 
 }  // namespace glif
@@ -602,7 +659,8 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
         }
         if (n_syn) (void)hipMemset(*wp, 0, n_syn * sizeof(float));
     }
-    if ((rc = build_own_rows(t, col_ptr.data(), ps.data(), ph_src.data()))) {
+    if ((rc = build_own_rows(t, col_ptr.data(), ps.data(), ph_src.data())) ||
+        (rc = build_spike_rows(t, col_ptr.data(), ps.data()))) {
         free_table(t);
         return rc;
     }
@@ -651,6 +709,11 @@ int glif_table_set_weights(glif_table *tt, const float *w, void *stream) {
     if (t->n_gs) {
         hipLaunchKernelGGL(k_gather_ell_w, dim3(grid_for(t->n_gs)), dim3(kBlock), 0, s, t->gs_pw, t->w_col,
                            t->gs_src, t->n_gs);
+        GLIF_HIP(hipGetLastError());
+    }
+    if (t->spk.rows) {
+        hipLaunchKernelGGL(k_gather_pair_w, dim3(grid_for(t->n_syn)), dim3(kBlock), 0, s, t->spk.ent, t->w_col,
+                           t->spk.src, t->n_syn);
         GLIF_HIP(hipGetLastError());
     }
     // the compact-row copies (a cell's, the table's own)
