@@ -599,7 +599,7 @@ def main():
 
     # roofline of the dominant kernel
     D, nb, nt = tb.max_delay, tb.n_basis, tb.basis.shape[0]
-    Wwin = 3 if 3 * B <= 16 else 1
+    Wwin = 3 if 3 * B <= 32 else 1
     Rg = 4
     while Rg < Wwin * B:
         Rg *= 2

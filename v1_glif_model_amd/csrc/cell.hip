@@ -23,9 +23,9 @@
 //   k_adj         per tick t: gz_t -> gV_t -> gP_{t-1} -> gR_{t-2} -> G_{t-2}
 //   k_bwd_rec_gs_dw  dz of the window's steps t0-2, t0-3, .. over the recurrent columns
 //                 of delays <= 2 Wwin - 3, one pass over the grouped row-sliced table
-//                 (16-float G rows), with the dW of the window's active columns behind
-//                 it; the other columns' dz run in the next window's adjoint launch
-//                 (k_adj_dw); other row lengths: k_bwd_rec, dz and dW in one type-phased pass
+//                 with the dW of the window's active columns behind it; with 16-float G rows
+//                 the other columns' dz run in the next window's adjoint launch (k_adj_dw);
+//                 without that order: k_bwd_rec, dz and dW in one type-phased pass
 //   k_bwd_in      dW of the LGN / background events of the window's steps
 // A window is legal because dz_s depends only on dz_{>= s+3}: a spike reaches the
 // rise current one step later, the PSC the next, the voltage the one after.
@@ -153,7 +153,9 @@ static bool win_forward(const Cell *c) {
 }
 
 // Backward window width (reverse ticks per table pass) and G row length.
-static int win_width(int B) { return 3 * B <= 16 ? 3 : 1; }
+// Three ticks while their batch entries fit a 32-float row: one walk of 128-byte rows for three of
+// 32- or 64-byte ones (batch 7 at 66,000 neurons: 295 us per 3 ticks against 431; batch 10: 315 against 581).
+static int win_width(int B) { return 3 * B <= 32 ? 3 : 1; }
 static int n_windows(int T, int Wwin) { return T >= 3 ? (T - 2 + Wwin - 1) / Wwin : 0; }
 static int ring_size(const Cell *c) { return c->D + 6; }
 
@@ -1209,7 +1211,7 @@ __global__ void __launch_bounds__(kBlock)
 
 // --------------------------------------------------------------- adjoint ----
 constexpr int kDelayUnroll = 8;
-constexpr int kAdjMaxWin = 3;  // reverse ticks per window (3 when 3 * B <= 16, else 1)
+constexpr int kAdjMaxWin = 3;  // reverse ticks per window (3 when 3 * B <= 32, else 1)
 
 struct AdjArgs {
     CellConst k;
@@ -1475,9 +1477,10 @@ __global__ void __launch_bounds__(kBlock) k_bwd_rec(ColArgs a, ActWin act) {
     bwd_cols<LG, 2>(a, act);
 }
 
+template <int LG, bool SPLIT>
 __global__ void __launch_bounds__(kBlock) k_bwd_rec_gs(GsArgs a, ActWin act) {
     __shared__ float stage[kBlock / kWave * kGsStage];
-    bwd_groups<4>(a, act, stage, blockIdx.x);
+    bwd_groups<LG, SPLIT>(a, act, stage, blockIdx.x);
 }
 
 // dW of one window's active recurrent columns next to the grouped walk (which computes
@@ -1508,12 +1511,14 @@ __device__ inline void rec_dw_body(const RecDwArgs &a, const ActWin &act, int64_
     {
         // the element lookups are issued at clamped, in-range positions before any is tested
         const ActWin::Col ci = act.col(min(c, a.n_cols - 1));
-        uint64_t wd[16];
+        for (int e0 = 0; e0 < a.n_elem; e0 += 16) {
+            uint64_t wd[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) wd[e] = act.word(ci, min(e, a.n_elem - 1));
+            for (int e = 0; e < 16; ++e) wd[e] = act.word(ci, min(e0 + e, a.n_elem - 1));
 #pragma unroll
-        for (int e = 0; e < 16; ++e)
-            if (e < a.n_elem && act.bit(ci, wd[e])) m |= 1u << e;
+            for (int e = 0; e < 16; ++e)
+                if (e0 + e < a.n_elem && act.bit(ci, wd[e])) m |= 1u << (e0 + e);
+        }
         if (c >= a.n_cols) m = 0;
         if (m) {
             lo = a.col_ptr[c];
@@ -1651,11 +1656,12 @@ struct WinDw {
     int32_t rec_blocks, lgn_blocks;
 };
 
+template <int LG, bool SPLIT>
 __global__ void __launch_bounds__(kBlock) k_bwd_rec_gs_dw(GsArgs a, ActWin act, int walk_blocks, WinDw p) {
     __shared__ float stage[kBlock / kWave * kGsStage];
     int64_t bid = blockIdx.x;
     if (bid < walk_blocks) {
-        bwd_groups<4>(a, act, stage, bid);
+        bwd_groups<LG, SPLIT>(a, act, stage, bid);
         return;
     }
     bid -= walk_blocks;
@@ -1678,13 +1684,33 @@ __global__ void __launch_bounds__(kBlock) k_adj_dw(AdjArgs a, int adj_blocks, Wa
     int64_t bid = blockIdx.x;
     if (bid < p.walk_blocks) {
         extern __shared__ float lds_f[];  // kBlock / kWave * kGsStage floats of the launch's LDS
-        bwd_groups<4>(p.gb, p.act, lds_f, bid);
+        bwd_groups<4, false>(p.gb, p.act, lds_f, bid);
         return;
     }
     bid -= p.walk_blocks;
     if (bid < adj_blocks) adj_body<NB>(a, bid);
     else if (bid < adj_blocks + p.dw.rec_blocks) rec_dw_body(p.dw.da, p.dw.act, bid - adj_blocks);
     else bwd_in_body<false>(p.dw.la, bid - adj_blocks - p.dw.rec_blocks, p.dw.lgn_blocks);
+}
+
+// The grouped walk over R-float G rows (4, 8, 16 or 32), with the window's dW passes behind it (dw) or alone.
+static void launch_bwd_gs(const GsArgs &ga, int R, const ActWin &act, int walk_blocks, const WinDw *dw, hipStream_t s) {
+    const dim3 grid(walk_blocks + (dw ? dw->rec_blocks + dw->lgn_blocks : 0));
+    if (grid.x == 0) return;
+    auto launch = [&](auto with_dw, auto alone) {
+        if (dw) GLIF_PROF_LAUNCH(with_dw, grid, dim3(kBlock), 0, s, ga, act, walk_blocks, *dw);
+        else GLIF_PROF_LAUNCH(alone, grid, dim3(kBlock), 0, s, ga, act);
+    };
+    switch (R / 4) {
+#define GLIF_GS(LG)                                                                       \
+    case LG:                                                                              \
+        if (ga.split) launch(k_bwd_rec_gs_dw<LG, true>, k_bwd_rec_gs<LG, true>);          \
+        else launch(k_bwd_rec_gs_dw<LG, false>, k_bwd_rec_gs<LG, false>);                 \
+        break;
+        GLIF_GS(1) GLIF_GS(2) GLIF_GS(4) GLIF_GS(8)
+#undef GLIF_GS
+        default: break;
+    }
 }
 
 static void launch_bwd_in(const BwdInArgs &ia, int64_t max_units, hipStream_t s) {
@@ -2534,9 +2560,8 @@ int glif_cell_backward(glif_cell *cc, int32_t B, int32_t T, const float *gz, con
     // padding elements of each G row stay zero
     const size_t g_elems = static_cast<size_t>(c->N) * c->g_rows * g_row(win_width(B), B);
     if ((rc = launch_fill_u32(w.G, 0u, 2 * g_elems, s))) return rc;
-    // the grouped row-sliced walk serves 16-float G rows
     const bool cg = c->g_compact;
-    const bool gs = (cg ? tr->cg.n_gs : tr->n_gs) > 0 && g_row(win_width(B), B) == 16;
+    const bool gs = (cg ? tr->cg.n_gs : tr->n_gs) > 0;   // the grouped row-sliced walk
     if (dw_rec && (rc = launch_fill_u32(w.dw_rec, 0u, tr->n_syn, s))) return rc;
     if (dw_lgn && (rc = launch_fill_u32(w.dw_lgn, 0u, tl->n_syn, s))) return rc;
     if (dw_bkg && (rc = launch_fill_u32(w.dw_bkg, 0u, tb->n_syn, s))) return rc;
@@ -2579,6 +2604,7 @@ int glif_cell_backward(glif_cell *cc, int32_t B, int32_t T, const float *gz, con
                dw_rec ? w.dw_rec : nullptr, nullptr, cg ? 1 : 0};
     GsArgs ga{tr->n_cols, (tr->n_cols + kGsCols - 1) / kGsCols, 0, cg ? tr->cg.gs_seg : tr->gs_seg,
               cg ? tr->cg.gs_pw : tr->gs_pw, w.G};
+    ga.split = gs_split(ga.n_groups, Rg / 4);
     RecDwArgs da{tr->n_cols, 0, hm, lm, Rg, tr->col_ptr, cg ? tr->cg.ps : tr->ps, w.G, w.dw_rec};
     ActWin act{w.zbits, w.dZ, tr->n_cols, 0, B, c->D, c->W, c->N, ring};
 
@@ -2619,8 +2645,9 @@ int glif_cell_backward(glif_cell *cc, int32_t B, int32_t T, const float *gz, con
     // slices the walk reads from the L2, and they run in window j + 1's adjoint launch instead
     // (class-pair types, 46 MB: 39.4 against 37.7 ms of backward per step beside the walk; 121
     // type-major rows, 511 MB: 108.4 against 103.3).
-    const bool defer = gs && dw_rec;
-    const bool dw_with_walk = defer && g_elems * sizeof(float) <= (size_t(32) << 20);
+    // Other row lengths, and a split walk, walk every column in the window's own launch.
+    const bool defer = gs && dw_rec && Rg == 16 && !ga.split;
+    const bool dw_with_walk = gs && dw_rec && (!defer || g_elems * sizeof(float) <= (size_t(32) << 20));
     WalkRest prev{};
     bool have_prev = false;
     const int64_t n_groups = (tr->n_cols + kGsCols - 1) / kGsCols;
@@ -2650,7 +2677,7 @@ int glif_cell_backward(glif_cell *cc, int32_t B, int32_t T, const float *gz, con
         la.s0 = s0;
         {
             ProfScope p(kProfBwdRec, s, true);
-            if (dw_with_walk) {
+            if (gs) {
                 GsArgs g1 = ga;
                 g1.g_hi = g_split;
                 WinDw dw{};
@@ -2659,14 +2686,8 @@ int glif_cell_backward(glif_cell *cc, int32_t B, int32_t T, const float *gz, con
                 dw.la = la;
                 dw.rec_blocks = ceil_div(tr->n_cols, kBlock);
                 dw.lgn_blocks = dw_lgn ? grid_subwaves(lgn_units, kWave) : 0;
-                const int wb = g_split > 0 ? ceil_div(g_split * 4, kBlock) : 0;
-                GLIF_PROF_LAUNCH(k_bwd_rec_gs_dw, dim3(wb + dw.rec_blocks + dw.lgn_blocks), dim3(kBlock), 0, s, g1,
-                                 act, wb, dw);
-            } else if (gs) {
-                GsArgs g1 = ga;
-                g1.g_hi = g_split;
-                if (g_split > 0)
-                    GLIF_PROF_LAUNCH(k_bwd_rec_gs, dim3(ceil_div(g_split * 4, kBlock)), dim3(kBlock), 0, s, g1, act);
+                launch_bwd_gs(g1, Rg, act, ceil_div(g_split * (Rg / 4) << ga.split, kBlock),
+                              dw_with_walk ? &dw : nullptr, s);
             } else {
                 launch_bwd_rec(ca, Rg, act, s);
             }
@@ -2685,7 +2706,7 @@ int glif_cell_backward(glif_cell *cc, int32_t B, int32_t T, const float *gz, con
             prev.gb.g_lo = g_split;
             prev.walk_blocks = g_split < n_groups ? ceil_div((n_groups - g_split) * 4, kBlock) : 0;
             have_prev = true;
-        } else if (dw_lgn) {
+        } else if (dw_lgn && !dw_with_walk) {
             ProfScope p(kProfBwdLgn, s, true);
             launch_bwd_in(la, lgn_units, s);
         }

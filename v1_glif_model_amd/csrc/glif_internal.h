@@ -145,7 +145,7 @@ struct Table {
     int32_t *order_inv = nullptr; // [n_syn]       position of synapse s in the column-grouped order
     int32_t *ph_inv = nullptr;    // [n_syn]       position of synapse s in the type-phased order
     int32_t *ph_src = nullptr;    // [n_syn]       column-grouped position of type-phased position k
-    // grouped row-sliced order (backward dz walks over 8- and 16-float G rows): lane group g owns
+    // grouped row-sliced order (backward dz walks): lane group g owns
     // columns kGsCols*g ..; its entries in G-row slice p (rows syn_id * n_post + post, slice p
     // = rows [n_rows * p / kGsSlices, n_rows * (p + 1) / kGsSlices)) are positions
     // [gs_seg[g * (kGsSlices + 1) + p], gs_seg[g * (kGsSlices + 1) + p + 1]), ordered by

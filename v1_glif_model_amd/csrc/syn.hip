@@ -424,10 +424,10 @@ __global__ void __launch_bounds__(kBlock) k_syn_dw_units(SynDwArgs da) { syn_dw_
 // The grouped dz walk (the first walk_blocks workgroups) beside the weight-gradient pass of
 // the active columns (the rest): both read G only, the walk is bound by its gathers' latency,
 // and one launch overlaps them.
-template <int LG>
+template <int LG, bool SPLIT>
 __global__ void __launch_bounds__(kBlock) k_syn_bwd_gs(GsArgs a, ActDense act, int walk_blocks, SynDwArgs da) {
     __shared__ float stage[kBlock / kWave * kGsStage];
-    if (static_cast<int>(blockIdx.x) < walk_blocks) bwd_groups<LG>(a, act, stage, blockIdx.x);
+    if (static_cast<int>(blockIdx.x) < walk_blocks) bwd_groups<LG, SPLIT>(a, act, stage, blockIdx.x);
     else syn_dw_body(da, blockIdx.x - walk_blocks);
 }
 
@@ -683,7 +683,7 @@ int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int3
         return fail(GLIF_ERANGE, "G rows per post * n_post * padded batch * 4 bytes must be < 4 GiB");
     ProfScope prof(kProfSynBwd, s);
     int rc;
-    const bool grouped = (cmp ? oc.n_gs : t->n_gs) && (Bp == 8 || Bp == 16);
+    const bool grouped = (cmp ? oc.n_gs : t->n_gs) > 0;
     // the work units instead of a walk whose time the longest column sets (the background
     // table's few, long columns) or that runs on few lanes (the LGN table's 17,400 columns):
     // for dz when the caller gives their partial sums room, and for dW, whose grouped-path
@@ -736,15 +736,24 @@ int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int3
         ActDense act{z, dz, t->n_cols, counts};
         GsArgs ga{t->n_cols, (t->n_cols + kGsCols - 1) / kGsCols, B, cmp ? oc.gs_seg : t->gs_seg,
                   cmp ? oc.gs_pw : t->gs_pw, G};
+        ga.split = gs_split(ga.n_groups, Bp / 4);
         SynDwArgs da{t->n_cols, B, cmp ? 1 : t->n_post, cmp ? rows : 1, Bp, counts, z, t->dwu, t->n_dwu,
                      t->col_ptr, cmp ? oc.ps : t->ps, t->order, G, dw};
         const int LG = grouped ? Bp / 4 : 2;   // no walk blocks when not grouped
-        const int walk_blocks = dz ? static_cast<int>(ceil_div(t->n_groups * LG, kBlock)) : 0;
+        const int walk_blocks = dz ? static_cast<int>(ceil_div(t->n_groups * LG << ga.split, kBlock)) : 0;
         const int dw_blocks = dw ? static_cast<int>(ceil_div(t->n_dwu, kBlock / kWave)) : 0;
         const dim3 grid(walk_blocks + dw_blocks);
         if (grid.x == 0) return GLIF_OK;   // no columns
-        if (LG == 2) hipLaunchKernelGGL(k_syn_bwd_gs<2>, grid, dim3(kBlock), 0, s, ga, act, walk_blocks, da);
-        else hipLaunchKernelGGL(k_syn_bwd_gs<4>, grid, dim3(kBlock), 0, s, ga, act, walk_blocks, da);
+        auto launch = [&](auto whole, auto split) {
+            if (ga.split) hipLaunchKernelGGL(split, grid, dim3(kBlock), 0, s, ga, act, walk_blocks, da);
+            else hipLaunchKernelGGL(whole, grid, dim3(kBlock), 0, s, ga, act, walk_blocks, da);
+        };
+        switch (LG) {
+            case 1: launch(k_syn_bwd_gs<1, false>, k_syn_bwd_gs<1, true>); break;
+            case 2: launch(k_syn_bwd_gs<2, false>, k_syn_bwd_gs<2, true>); break;
+            case 4: launch(k_syn_bwd_gs<4, false>, k_syn_bwd_gs<4, true>); break;
+            default: launch(k_syn_bwd_gs<8, false>, k_syn_bwd_gs<8, true>); break;
+        }
         GLIF_HIP(hipGetLastError());
         return GLIF_OK;
     }

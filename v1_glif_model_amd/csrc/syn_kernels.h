@@ -312,15 +312,15 @@ __device__ inline void bwd_cols(const ColArgs &a, const Act &act) {
     }
 }
 
-// ---- grouped row-sliced backward (16-float G rows) ------------------------------
-// dz of every column over the grouped row-sliced order: lane group g (4 lanes, lane q
-// holding floats 4q..4q+3 of a row) owns columns kGsCols*g .. (4 of them); it walks its entries of
-// one G-row slice at a time, 8 per step (one 64-byte load, lane q holding entries 2q and
-// 2q+1, shared in the group by DPP), and adds w * G[row] into the column's accumulator.
+// ---- grouped row-sliced backward (4- to 32-float G rows) ------------------------------
+// dz of every column over the grouped row-sliced order: lane group g (LG lanes, lane q
+// holding floats 4q..4q+3 of a row) owns columns kGsCols*g .. (4 of them), or shares them with one or
+// three others (gs_split); it walks its entries of one G-row slice at a time, 8 per step (one
+// 64-byte load, shared in the group by DPP or lane swizzles), and adds w * G[row] into the column's accumulator.
 // Every wave finishes a slice before starting the next, so the waves in flight gather
 // from one quarter of G at a time, and a group owns its columns, so dz needs no atomics.
 // Each column sums its entries in G-row order (syn_id, then post), the order of
-// bwd_cols.  The dW of active columns is a separate pass (k_bwd_rec_dw in cell.hip):
+// bwd_cols; split, the lane groups' sums of their slices are added in that order.  The dW of active columns is a separate pass (k_bwd_rec_dw in cell.hip):
 // holding it here costs a third more registers and a second walk per group.
 //
 // Measured on MI355X with a config-2-sized table (16.5M synapses, 330k columns, G 21 MB):
@@ -328,6 +328,10 @@ __device__ inline void bwd_cols(const ColArgs &a, const Act &act) {
 // 27.7M L2 requests (its 8-byte entry loads are re-requested), a row-sorted walk without
 // slices 18.5M but misses L2 on 42% of them; the slices bring the misses down while the
 // 8-entry loads keep the requests near one per synapse.
+// Measured (us per 3-tick window of the cell's backward): 5,000 neurons at batch 5 53 -> 27, 12,007 at
+// batch 5 66 -> 42, 30,011 at batch 5 (2,800 waves unsplit) 68, split 81; 66,000 at batch 2 142, split 160.
+constexpr int64_t kGsSplitWaves = 2048;
+
 struct GsArgs {
     int64_t n_cols, n_groups;
     int32_t n_elem;
@@ -337,7 +341,18 @@ struct GsArgs {
     // the groups walked: [g_lo, g_hi), g_hi = 0 for every group from g_lo; g_lo a multiple of
     // the groups of a wave (kWave / LG)
     int64_t g_lo = 0, g_hi = 0;
+    // log2 of the lane groups that share a column group (gs_split): each walks kGsSlices >> split
+    // of its slices, and their sums are added in slice order
+    int32_t split = 0;
 };
+
+// Column groups shared by two or four lane groups when the walk would otherwise run on few waves: a
+// lane group's walk is a chain of dependent loads (entries, then rows), and with few waves per SIMD
+// their latency is the walk's time.  groups x lanes: its lanes unsplit.
+inline int gs_split(int64_t groups, int lanes) {
+    const int64_t waves = groups * lanes / kWave;
+    return waves < kGsSplitWaves / 2 ? 2 : waves < kGsSplitWaves ? 1 : 0;
+}
 
 // value of lane `src` of this lane's quad (DPP quad_perm broadcast)
 __device__ inline uint32_t quad_bcast(uint32_t v, int src) {
@@ -349,29 +364,39 @@ __device__ inline uint32_t quad_bcast(uint32_t v, int src) {
     }
 }
 
-// value of lane `src` of this lane's group of LG lanes (LG = 2: the lane pairs of a quad,
+// value of lane `src` of this lane's group of LG lanes (LG = 8: a swizzle; LG = 1: its own; LG = 2: the lane pairs of a quad,
 // quad_perm [src, src, 2 + src, 2 + src]; LG = 4: the quad)
 template <int LG>
 __device__ inline uint32_t group_bcast(uint32_t v, int src) {
-    static_assert(LG == 2 || LG == 4, "lane groups of 2 or 4");
+    static_assert(LG == 1 || LG == 2 || LG == 4 || LG == 8, "lane groups of 1, 2, 4 or 8");
+    if (LG == 1) return v;
+    if (LG == 8) {
+        // lane (lane & 24) | src of each half wave
+#define GLIF_OCT(s) case s: return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(static_cast<int>(v), (s << 5) | 0x18));
+        switch (src) { GLIF_OCT(0) GLIF_OCT(1) GLIF_OCT(2) GLIF_OCT(3) GLIF_OCT(4) GLIF_OCT(5) GLIF_OCT(6) GLIF_OCT(7) }
+#undef GLIF_OCT
+    }
     if (LG == 4) return quad_bcast(v, src);
     return src == 0 ? static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xA0, 0xF, 0xF, false))
                     : static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xF5, 0xF, 0xF, false));
 }
 
-// LDS floats per wave for the dz staging of bwd_groups: [R][columns per wave + 1] for
-// LG = 4 (16 floats x 16 kGsCols columns) or LG = 2 (8 x 32 kGsCols), whichever is larger
-constexpr int kGsStage = 16 * (16 * kGsCols + 1) > 8 * (32 * kGsCols + 1) ? 16 * (16 * kGsCols + 1)
-                                                                           : 8 * (32 * kGsCols + 1);
+// LDS floats per wave for the dz staging of bwd_groups: [R][columns per wave + 1], R = 4 LG floats
+// by (kWave / LG) * kGsCols columns; LG = 8 takes the most
+constexpr int kGsStage = 32 * (8 * kGsCols + 1);
+static_assert(kGsStage >= 16 * (16 * kGsCols + 1) && kGsStage >= 8 * (32 * kGsCols + 1) && kGsStage >= 4 * (64 * kGsCols + 1));
 
-// LG lanes per G row (R = 4 LG floats, LG = 2 or 4), lane q holding floats 4q..4q+3; a chunk
-// of 8 entries is 8 / LG entries per lane (one or two 16-byte loads).  stage: kGsStage floats
-// of LDS per wave of the block.
-template <int LG, class Act>
+// LG lanes per G row (R = 4 LG floats, LG = 1, 2, 4 or 8), lane q holding floats 4q..4q+3; a chunk
+// of 8 entries is 8 / LG entries per lane (8 to 64 bytes).  stage: kGsStage floats
+// of LDS per wave of the block.  SPLIT: a.split may be above 0.
+template <int LG, bool SPLIT, class Act>
 __device__ inline void bwd_groups(const GsArgs &a, const Act &act, float *stage, int64_t bid) {
-    constexpr int R = 4 * LG, EPL = 8 / LG, CW = (kWave / LG) * kGsCols;
-    const int q = threadIdx.x % LG;
-    const int64_t g = a.g_lo + (bid * blockDim.x + threadIdx.x) / LG;
+    constexpr int R = 4 * LG, EPL = 8 / LG;
+    static_assert(kGsSlices == 4);
+    const int sh = SPLIT ? a.split : 0, S = 1 << sh, CW = (kWave / LG >> sh) * kGsCols;
+    const int lane = threadIdx.x % kWave;
+    const int q = threadIdx.x % LG, sub = (lane / LG) & (S - 1);
+    const int64_t g = a.g_lo + ((bid * blockDim.x + threadIdx.x) / LG >> sh);
     // a group past the end walks nothing but still takes part in the staging below
     const bool own = g < (a.g_hi ? a.g_hi : a.n_groups);
     const char *Gb = reinterpret_cast<const char *>(a.G) + static_cast<uint32_t>(q) * 16u;
@@ -381,16 +406,20 @@ __device__ inline void bwd_groups(const GsArgs &a, const Act &act, float *stage,
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[j][i] = 0.0f;
     const int32_t *sg = a.seg + (own ? g : 0) * (kGsSlices + 1);
-    int32_t lo = own ? sg[0] : 0;
-    for (int p = 0; p < kGsSlices; ++p) {
+    const int p0 = sub * (kGsSlices >> sh), p1 = p0 + (kGsSlices >> sh);
+    int32_t lo = own ? sg[p0] : 0;
+    for (int p = p0; p < p1; ++p) {
         const int32_t hi = own ? sg[p + 1] : 0;
         for (int32_t k0 = lo; k0 < hi; k0 += 8) {
             uint2 my[EPL];
+            if constexpr (EPL == 1) my[0] = a.pw[k0 + q];
+            else {
 #pragma unroll
-            for (int h = 0; h < EPL; h += 2) {
-                const uint4 v = *reinterpret_cast<const uint4 *>(a.pw + k0 + EPL * q + h);
-                my[h] = make_uint2(v.x, v.y);
-                my[h + 1] = make_uint2(v.z, v.w);
+                for (int h = 0; h < EPL; h += 2) {
+                    const uint4 v = *reinterpret_cast<const uint4 *>(a.pw + k0 + EPL * q + h);
+                    my[h] = make_uint2(v.x, v.y);
+                    my[h + 1] = make_uint2(v.z, v.w);
+                }
             }
             float4 gv[8];
 #pragma unroll
@@ -419,25 +448,28 @@ __device__ inline void bwd_groups(const GsArgs &a, const Act &act, float *stage,
         lo = hi;
     }
     // dz through LDS: the wave's groups own CW consecutive columns, so each element's
-    // values leave as coalesced stores
-    const int lane = threadIdx.x % kWave;
+    // values leave as coalesced stores (split: each lane group's sums, added in slice order)
     float *st = stage + (threadIdx.x / kWave) * kGsStage;
-    const int gl = lane / LG;
+    constexpr int CWS = (kWave / LG) * kGsCols;
+    const int gl = lane / LG >> sh;
 #pragma unroll
     for (int j = 0; j < kGsCols; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) st[(4 * q + i) * (CW + 1) + kGsCols * gl + j] = acc[j][i];
+        for (int i = 0; i < 4; ++i) st[(4 * q + i) * (CWS + 1) + sub * CW + kGsCols * gl + j] = acc[j][i];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int64_t cw0 = (g - gl) * kGsCols;
     const int64_t c_end = a.g_hi ? min(a.n_cols, a.g_hi * kGsCols) : a.n_cols;
-#pragma unroll
     for (int cc = lane; cc < CW; cc += kWave) {
         const int64_t c = cw0 + cc;
         if (c < c_end) {
             const typename Act::Col ci = act.col(c);
-            for (int e = 0; e < a.n_elem; ++e) *act.out(ci, e) = st[e * (CW + 1) + cc];
+            for (int e = 0; e < a.n_elem; ++e) {
+                float x = st[e * (CWS + 1) + cc];
+                for (int u = 1; u < S; ++u) x = x + st[e * (CWS + 1) + u * CW + cc];
+                *act.out(ci, e) = x;
+            }
         }
     }
 }
