@@ -1,0 +1,73 @@
+"""GPU parity of the op's backward over work units and over the split column walk, and of the counts
+pull over the padded rows, against the C oracle, at the sizes where they can go wrong: batches around
+the padded row lengths (1 to 32), columns of no, one and a few synapses, around a unit's 256 synapses
+and over many of them, runs of more columns than a wave has lane groups, counts and spikes.  The
+forward bit for bit (also where a count is infinite), dz and dW within 1e-5 of each element's sum of
+absolute terms + 1e-6 (a sum of at most a few thousand float32 terms is off by far less)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import cpu as orc
+from oracle import dense
+from v1_glif_model_amd.tables import SynapseTable as Tab
+
+pytestmark = pytest.mark.gpu
+
+N = 2200
+LENGTHS = {
+    # a column beyond 2048 synapses: always the units
+    "long": [0, 1, 2, 255, 256, 257, 512, 513, 2100, 0, 3] + [1] * 130 + [7] * 40 + [100, 156, 1, 0],
+    # runs of short columns: units up to 8 batch entries, the walk above
+    "short": [0, 5, 9, 1, 3, 0, 2, 4] * 17 + [300, 1, 0],
+    # middling columns: units at every batch
+    "middle": [97, 130, 256, 300, 0, 64, 511] * 5,
+}
+
+
+def _table(kind, rng):
+    if kind == "even":   # 10 of 100 inputs each, the last posts fewer: rows that pad well
+        pairs = [np.stack([np.full(k, p), np.sort(rng.permutation(100)[:k])], -1)
+                 for p in range(N) for k in [10 if p < N - 3 else N - p]]
+        ind, n_cols = np.concatenate(pairs), 100
+    else:
+        cols = [np.stack([rng.permutation(N)[:k], np.full(k, c)], -1) for c, k in enumerate(LENGTHS[kind])]
+        ind, n_cols = np.concatenate(cols), len(LENGTHS[kind])
+        ind = ind[np.lexsort((ind[:, 1], ind[:, 0]))]
+    n = len(ind)
+    return Tab(ind[:, 0].astype(np.int64), ind[:, 1].astype(np.int64), rng.normal(0, 1, n).astype(np.float32),
+               rng.integers(0, 5, n).astype(np.uint8), N, n_cols), ind
+
+
+@pytest.mark.parametrize("counts", [False, True])
+@pytest.mark.parametrize("kind", ["long", "short", "middle", "even"])
+@pytest.mark.parametrize("B", [1, 4, 5, 9, 16, 17, 32])
+def test_units(B, kind, counts):
+    from v1_glif_model_amd.ops import SynapseTable
+    rng = np.random.default_rng(B)
+    tab, ind = _table(kind, rng)
+    basis = rng.random((5, 4)).astype(np.float32)
+    print(B, kind, counts, flush=True)
+    t = SynapseTable(ind, tab.syn_id, (N, tab.n_cols), basis)
+    t.set_weights(torch.tensor(tab.weight, device="cuda"))
+    z = (rng.random((B, tab.n_cols)) < 0.3).astype(np.float32)
+    if counts:
+        z *= rng.integers(1, 4, z.shape).astype(np.float32)
+    dy = rng.normal(0, 1, (B * N, 4)).astype(np.float32)
+    dz, dw = t.backward(torch.tensor(z, device="cuda"), torch.tensor(dy, device="cuda"), counts=counts)
+    rdz, rdw = orc.syn_bwd(tab, z, basis, dy, use_count=counts)
+    _, _, dz_abs, dw_abs = dense.syn_bwd_f64(tab, z, basis, dy, use_count=counts)
+    assert np.max(np.abs(dz.cpu().numpy() - rdz) - 1e-5 * dz_abs) <= 1e-6
+    assert np.max(np.abs(dw.cpu().numpy() - rdw) - 1e-5 * dw_abs) <= 1e-6
+    if not counts:
+        return
+    for infinite in (False, True):
+        if infinite:
+            z[B // 2, 0] = np.inf
+        with np.errstate(invalid="ignore"):
+            ref = orc.syn_fwd(tab, z, basis, use_count=True)
+        got = t.forward(torch.tensor(z, device="cuda"), counts=True, mode="deterministic").cpu().numpy()
+        np.testing.assert_array_equal(got, ref)
+        if kind == "even":   # pulled in event mode too
+            ev = t.forward(torch.tensor(z, device="cuda"), counts=True, mode="event").cpu().numpy()
+            np.testing.assert_array_equal(ev, ref)

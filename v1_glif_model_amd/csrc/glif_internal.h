@@ -18,9 +18,12 @@ constexpr int kMaxBasis = 8;
 constexpr int kMaxBatch = 32;
 constexpr uint32_t kLow24 = 0x00FFFFFFu;
 constexpr int kChunkEntries = 512;
-// work units of the op-level weight-gradient pass: at most 64 consecutive columns and this many
-// synapses, or one chunk of this many synapses of a longer column
-constexpr int kDwUnitEntries = 1024;
+// work units of the op-level passes over columns: at most 64 consecutive columns and this many
+// synapses, or one chunk of this many synapses of a longer column.  Small units give a small table
+// enough waves (backward at batch 5, 1024 -> 256: 100,000 synapses 36 -> 16 us); a large one has
+// enough of the others, and fewer of them pass over its inactive columns faster (16.5M synapses,
+// batch 5: 201 us with 256 against 193)
+constexpr int dw_unit_entries(int64_t n_syn) { return n_syn < (4 << 20) ? 256 : 1024; }
 constexpr int kChunkRows = 63;
 // grouped row-sliced backward order: kGsCols columns per lane group,
 // kGsSlices equal ranges of G rows, segments padded to kGsPad entries
@@ -132,10 +135,10 @@ struct Table {
     int32_t n_chunks = 0;
     int4 *chunk_desc = nullptr;   // [n_chunks]
     // work units of the op-level weight-gradient pass over the column-grouped table: unit u is
-    // {first column, columns, first position, end position} (kDwUnitEntries)
+    // {first column, columns, first position, end position} (dw_unit_entries)
     int32_t n_dwu = 0;
     int4 *dwu = nullptr;          // [n_dwu]
-    // columns whose units hold one column each (a column of more than kDwUnitEntries synapses
+    // columns whose units hold one column each (a column of more than dw_unit_entries synapses
     // spreads over several): {column, first unit, units, 0}, for the chunked dz pass
     int32_t n_dzc = 0;
     int4 *dzc = nullptr;          // [n_dzc]

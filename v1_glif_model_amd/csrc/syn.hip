@@ -17,13 +17,18 @@ namespace glif {
 // column scan pushes it on one wave, so their time is the longest column's serial chain (a
 // 6600-synapse column: ~4 ms for dz, ~5 ms for the push); the units split long columns over many
 // waves and cost at most ~1.5x the walk on short ones (runs of short columns use few lanes).
-constexpr int32_t kUnitDzMinColLen = 2 * kDwUnitEntries;
+constexpr int32_t kUnitDzMinColLen = 2048;
 // The event push takes the units when the column scan (a wave per 64 columns) would run on fewer
 // waves than this (the LGN table's 17,400 columns: 272 waves) or a column has more synapses than
 // one unit (its chunks then go to waves of their own).
 constexpr int64_t kPushUnitsMaxScanWaves = 2048;
-// dz takes the units too when the walk would run on fewer lanes than this.
+constexpr int32_t kPushUnitsMinColLen = 1024;
+// The backward takes the units too when the walk would run on fewer lanes than this -- unless G's rows
+// are a cache line or more (Bp >= 16) and the columns short: a lane group then waits for few rows, while
+// the split walk streams them (whole calls, units against walk, batch 20: 25 synapses a column 42 against
+// 25 us, 50: 37 against 26, 62: 53 against 47, 132: 37 against 46; batch 1 at 25: 10 against 16).
 constexpr int64_t kUnitDzMaxWalkLanes = 1024 * kWave;
+constexpr int64_t kUnitDzMinAvgLen = 96;
 
 // ---------------------------------------------------------------- forward ----
 // Deterministic pull of Poisson-count inputs (the background form, models.py:917-931): thread
@@ -59,11 +64,71 @@ __global__ void __launch_bounds__(kBlock)
     for (int r = 0; r < nb; ++r) dst[r] = acc[r];
 }
 
+// The same over an input table's ELL copy: a thread per post and NBATCH batch entries, so an entry
+// (one coalesced load) is read once for all of them; the inputs' counts [input][batch entry] in LDS.
+// Each (post, batch entry) adds its row's active entries in row order, as k_syn_pull_dense does.
+// Background table (66,000 posts, 10 synapses each, 100 inputs), batch 32: 98 -> 28 us.
+constexpr int kEllBatch = 8;
+constexpr int64_t kEllMaxInputs = 1024;   // their counts for kEllBatch batch entries: 32 KB
+
+__global__ void __launch_bounds__(kBlock)
+    k_syn_pull_ell(const float *__restrict__ z, int32_t B, int32_t n_cols, int32_t n_post,
+                   const int32_t *__restrict__ row_ptr, const uint2 *__restrict__ ell,
+                   const float *__restrict__ basis, int n_types, int nb, float *__restrict__ I) {
+    extern __shared__ __align__(16) float ell_lds[];
+    float4 *zl = reinterpret_cast<float4 *>(ell_lds);   // [n_cols][kEllBatch]
+    float *basis_lds = ell_lds + static_cast<size_t>(n_cols) * kEllBatch;
+    const int b0 = static_cast<int>(blockIdx.y) * kEllBatch;
+    for (int i = threadIdx.x; i < n_cols * kEllBatch; i += blockDim.x) {
+        const int bb = i / n_cols, c = i - bb * n_cols;
+        const float x = b0 + bb < B ? z[static_cast<int64_t>(b0 + bb) * n_cols + c] : 0.0f;
+        ell_lds[c * kEllBatch + bb] = x > 0.0f ? x : 0.0f;
+    }
+    load_basis_lds(basis_lds, basis, n_types * nb);
+    const int64_t n = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (n >= n_post) return;
+    const int32_t len = row_ptr[n + 1] - row_ptr[n];   // without the padding, which an infinite count would turn to NaN
+    float acc[kEllBatch][kMaxBasis];
+#pragma unroll
+    for (int bb = 0; bb < kEllBatch; ++bb)
+#pragma unroll
+        for (int r = 0; r < kMaxBasis; ++r) acc[bb][r] = 0.0f;
+    for (int32_t j0 = 0; j0 < len; j0 += 4) {
+        uint2 e[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) e[u] = ell[static_cast<int64_t>(min(j0 + u, len - 1)) * n_post + n];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (j0 + u >= len) break;
+            const float w = __uint_as_float(e[u].y);
+            const float *bs = basis_lds + (e[u].x >> 24) * nb;
+            const float4 a = zl[(e[u].x & kLow24) * 2], c = zl[(e[u].x & kLow24) * 2 + 1];
+            const float x[kEllBatch] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+#pragma unroll
+            for (int r = 0; r < kMaxBasis; ++r) {
+                if (r >= nb) break;
+                const float s = bs[r];
+#pragma unroll
+                for (int bb = 0; bb < kEllBatch; ++bb)
+                    acc[bb][r] = x[bb] > 0.0f ? acc[bb][r] + (w * x[bb]) * s : acc[bb][r];
+            }
+        }
+    }
+#pragma unroll
+    for (int bb = 0; bb < kEllBatch; ++bb) {
+        if (b0 + bb >= B) break;
+        float *dst = I + (static_cast<int64_t>(b0 + bb) * n_post + n) * nb;
+#pragma unroll
+        for (int r = 0; r < kMaxBasis; ++r)
+            if (r < nb) dst[r] = acc[bb][r];
+    }
+}
+
 // Event push straight from z [B][n_cols]: a wave per 64 consecutive columns builds each
 // column's batch mask (z > 0, the test of tf.where at models.py:128-130), and all 64 lanes
 // push the wave's active columns one after another.  No column list, no count pass.
 // The event push over the table's work units (a run of up to 64 short columns, or a chunk of
-// at most kDwUnitEntries synapses of a long column), a wave per unit: the lanes hold the
+// at most dw_unit_entries synapses of a long column), a wave per unit: the lanes hold the
 // run's columns' batch masks, and all 64 lanes push each active column's share of the unit.
 // For tables whose column scan would run on few waves (few columns, or long ones).
 template <bool COUNTS>
@@ -339,72 +404,129 @@ __device__ inline void syn_dw_body(const SynDwArgs &a, int64_t bid) {
 }
 
 
-// dz over the same work units, for tables whose walk runs on few lanes or whose time a long
-// column sets (the input tables).  A wave per unit.  A run of y columns gives each column
-// L = 64 / (y rounded up to a power of 2) lanes, which sum every L-th synapse of the column and
-// add their sums in a fixed butterfly order; lane 0 of the column's lanes writes dz.  A
-// one-column unit (a whole column or one chunk of a long one) uses all 64 lanes the same way
-// into partial[unit], and k_dz_chunks adds a column's units in order.  Each term is
-// w * G[row][b], as the walks form it.
-struct DzUnitArgs {
+// dz and dW over the same work units, for tables whose walk runs on few lanes or whose time a long
+// column sets (the input tables).  A wave per unit; LG lanes hold one synapse's G row (4 floats each), so a
+// row is one request of LG lanes and is read once for both gradients.  The wave's 64 / LG lane
+// groups take the synapses of a one-column unit in turn, or share the columns of a run, a power of
+// two of groups per column, in passes where the run has more columns than groups.  dz: each group's
+// sums are added in a fixed butterfly order; a one-column unit's go to partial[unit], and k_dz_chunks
+// adds a column's units in order.  dW of a column with any input: its synapses' sum over the batch
+// entries of G[row][b] times the input value (counts) or 1, written once, straight to reference
+// order.  What bounds it is the gathers' latency (kUnitRows rows in flight per lane group, and
+// dw_unit_entries synapses a wave for enough waves).  Whole backward calls, against a lane per
+// synapse for dz, which held whole rows, and dW by a pass of its own, both over 1024-synapse
+// units: background table, 66,000 posts, batch 32, 174 -> 68 us; LGN table at batch 5, 94 -> 58.
+struct UnitArgs {
     int64_t n_cols;
-    int32_t B, hm, lm, R;  // G row of entry p: (p >> 24) * hm + (p & kLow24) * lm, R floats
+    int32_t B, hm, lm, counts;  // G row of entry p: (p >> 24) * hm + (p & kLow24) * lm, 4 LG floats
+    const float *z;       // [B][n_cols]
     const int4 *units;
     int32_t n_units;
     const int32_t *col_ptr;
     const uint32_t *ps;
     const float *w;       // column-grouped weights
+    const int32_t *order;
     const float *G;
-    float *dz;            // [B][n_cols]
-    float *partial;       // [n_units][R]
+    float *dz;            // [B][n_cols], or nullptr
+    float *partial;       // [n_units][4 LG]
+    float *dw;            // reference order, zero-filled by the caller, or nullptr
 };
 
-template <int BP>
-__device__ inline void dz_unit_body(const DzUnitArgs &a, int64_t bid) {
-    const int lane = threadIdx.x % kWave;
-    const int64_t ui = bid * (blockDim.x / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+constexpr int kUnitRows = 4;
+
+template <int LG>
+__global__ void __launch_bounds__(kBlock) k_syn_units(UnitArgs a) {
+    constexpr int SG = kWave / LG, U = kUnitRows;
+    const int lane = threadIdx.x % kWave, q = lane % LG, sg = lane / LG;
+    const int64_t ui = static_cast<int64_t>(blockIdx.x) * (blockDim.x / kWave) +
+                       __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
     if (ui >= a.n_units) return;  // the whole wave leaves together
     const int4 un = a.units[ui];
-    int sh = 0;
-    while ((1 << sh) < un.y) ++sh;  // un.y <= 64: sh <= 6, the same in every lane
-    const int L = kWave >> sh;
-    const int j = lane / L, sl = lane % L;
-    float acc[BP];
+    int cp = 1;                   // columns of a pass: a power of two of the run's, at most SG
+    while (cp < un.y && cp < SG) cp *= 2;
+    const int n = SG / cp;        // lane groups per column
+    for (int j0 = 0; j0 < un.y; j0 += cp) {
+        const int j = j0 + sg / n;
+        const bool own = j < un.y;
+        const int64_t c = un.x + (own ? j : 0);
+        int32_t k = 0, k_end = 0;
+        if (own) {
+            k = (un.y == 1 ? un.z : a.col_ptr[c]) + sg % n;
+            k_end = un.y == 1 ? un.w : a.col_ptr[c + 1];
+        }
+        float zv[4];
+        bool on[4], any = false;
 #pragma unroll
-    for (int b = 0; b < BP; ++b) acc[b] = 0.0f;
-    int32_t k = 0, k_end = 0;
-    if (un.y == 1) {
-        k = un.z + lane;
-        k_end = un.w;
-    } else if (j < un.y) {
-        k = a.col_ptr[un.x + j] + sl;
-        k_end = a.col_ptr[un.x + j + 1];
-    }
-    for (; k < k_end; k += L) {
-        const uint32_t p = a.ps[k];
-        const float wk = a.w[k];
-        const float *g = a.G + (static_cast<int64_t>(p >> 24) * a.hm + static_cast<int64_t>(p & kLow24) * a.lm) * a.R;
+        for (int i = 0; i < 4; ++i) {
+            const int b = 4 * q + i;
+            const float x = a.dw && own && b < a.B ? a.z[b * a.n_cols + c] : 0.0f;
+            on[i] = x > 0.0f;
+            zv[i] = a.counts ? x : 1.0f;
+            any |= on[i];
+        }
+        const uint64_t bal = __ballot(any);
+        const bool live = ((bal >> (sg * LG)) & ((1ull << LG) - 1ull)) != 0ull;   // the same in the group's lanes
+        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        // without dz only the active columns' synapses are read
+        if (!a.dz && !live) k = k_end;
+        for (; k < k_end; k += U * n) {
+            uint32_t p[U];
+            float wk[U];
 #pragma unroll
-        for (int b = 0; b < BP; ++b)
-            if (b < a.B) acc[b] = acc[b] + wk * g[b];
-    }
-    for (int o = L / 2; o >= 1; o >>= 1)
+            for (int u = 0; u < U; ++u) {
+                const int32_t kk = min(k + u * n, k_end - 1);
+                p[u] = a.ps[kk];
+                wk[u] = a.dz && k + u * n < k_end ? a.w[kk] : 0.0f;
+            }
+            float4 g[U];
 #pragma unroll
-        for (int b = 0; b < BP; ++b) acc[b] = acc[b] + __shfl_xor(acc[b], o, kWave);
-    if (un.y == 1) {
-        if (lane == 0)
+            for (int u = 0; u < U; ++u)
+                g[u] = reinterpret_cast<const float4 *>(a.G)[(static_cast<int64_t>(p[u] >> 24) * a.hm +
+                                                              static_cast<int64_t>(p[u] & kLow24) * a.lm) * LG + q];
+            if (a.dz) {
 #pragma unroll
-            for (int b = 0; b < BP; ++b)
-                if (b < a.B) a.partial[ui * a.R + b] = acc[b];
-    } else if (sl == 0 && j < un.y) {
+                for (int u = 0; u < U; ++u) {
+                    if (k + u * n >= k_end) break;
+                    acc[0] = acc[0] + wk[u] * g[u].x;
+                    acc[1] = acc[1] + wk[u] * g[u].y;
+                    acc[2] = acc[2] + wk[u] * g[u].z;
+                    acc[3] = acc[3] + wk[u] * g[u].w;
+                }
+            }
+            if (live) {
+                float d[U];
 #pragma unroll
-        for (int b = 0; b < BP; ++b)
-            if (b < a.B) a.dz[static_cast<int64_t>(b) * a.n_cols + un.x + j] = acc[b];
+                for (int u = 0; u < U; ++u) {
+                    d[u] = on[0] ? g[u].x * zv[0] : 0.0f;
+                    d[u] = on[1] ? d[u] + g[u].y * zv[1] : d[u];
+                    d[u] = on[2] ? d[u] + g[u].z * zv[2] : d[u];
+                    d[u] = on[3] ? d[u] + g[u].w * zv[3] : d[u];
+                }
+#pragma unroll
+                for (int o = 1; o < LG; o <<= 1)
+#pragma unroll
+                    for (int u = 0; u < U; ++u) d[u] = d[u] + __shfl_xor(d[u], o, kWave);
+                if (q == 0) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (k + u * n < k_end) a.dw[a.order[k + u * n]] = d[u];
+                }
+            }
+        }
+        if (!a.dz) continue;
+        for (int o = LG; o < n * LG; o <<= 1)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = acc[i] + __shfl_xor(acc[i], o, kWave);
+        if (!own || sg % n) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int b = 4 * q + i;
+            if (b >= a.B) continue;
+            if (un.y == 1) a.partial[ui * (4 * LG) + b] = acc[i];
+            else a.dz[b * a.n_cols + c] = acc[i];
+        }
     }
 }
-
-template <int BP>
-__global__ void __launch_bounds__(kBlock) k_dz_units(DzUnitArgs a) { dz_unit_body<BP>(a, blockIdx.x); }
 
 // dz of the one-column units' columns: thread per (column, b), the column's units in order.
 __global__ void __launch_bounds__(kBlock)
@@ -418,8 +540,6 @@ __global__ void __launch_bounds__(kBlock)
     for (int u = 1; u < d.z; ++u) s = s + partial[static_cast<int64_t>(d.y + u) * R + b];
     dz[static_cast<int64_t>(b) * n_cols + d.x] = s;
 }
-
-__global__ void __launch_bounds__(kBlock) k_syn_dw_units(SynDwArgs da) { syn_dw_body(da, blockIdx.x); }
 
 // The grouped dz walk (the first walk_blocks workgroups) beside the weight-gradient pass of
 // the active columns (the rest): both read G only, the walk is bound by its gathers' latency,
@@ -474,10 +594,13 @@ static SynWs carve_syn(void *ws, const Table *t, int32_t B, size_t *bytes, bool 
 // call, 67 against 24 us pulled at B = 5), and whether that pull uses the workspace (batch
 // masks and activity bits built from z; Poisson counts take the dense-row pull, which needs
 // none).  glif_syn_fwd validates the workspace with the same predicate syn_fwd dispatches on.
-static bool fwd_pulls(const Table *t, int32_t mode) {
-    return mode == GLIF_MODE_DETERMINISTIC || t->max_col_len > kUnitDzMinColLen;
+// Poisson counts of a few inputs pull in event mode whatever the columns' length: a fifth of them is
+// active in every batch entry (12,007 posts, 100 inputs, batch 32: 157 us pushed, 12 pulled).
+static bool ell_counts(const Table *t) { return t->ell_len > 0 && t->n_cols <= kEllMaxInputs; }
+static bool fwd_pulls(const Table *t, int32_t counts, int32_t mode) {
+    return mode == GLIF_MODE_DETERMINISTIC || t->max_col_len > kUnitDzMinColLen || (counts && ell_counts(t));
 }
-static bool fwd_uses_ws(const Table *t, int32_t counts, int32_t mode) { return fwd_pulls(t, mode) && !counts; }
+static bool fwd_uses_ws(const Table *t, int32_t counts, int32_t mode) { return fwd_pulls(t, counts, mode) && !counts; }
 
 // The op forward on a carved workspace (every buffer it reads is written first by this call,
 // so nothing in it has to start at zero).  Launches only; no allocation, no synchronisation.
@@ -486,7 +609,7 @@ static int syn_fwd(const Table *t, const float *z, int32_t B, int32_t counts, in
     const size_t lds = sizeof(float) * t->n_types * t->n_basis;
     const int64_t nI = static_cast<int64_t>(B) * t->n_post;
     // the pull's sums are the reference's, well within the event mode's bar
-    if (fwd_pulls(t, mode)) {
+    if (fwd_pulls(t, counts, mode)) {
         if (fwd_uses_ws(t, counts, mode)) {
             // the row pulls over batch masks and activity bitmaps built from z (one step, t = 0):
             // the resident chunk form where it fits, else the half-wave row pull (B * nb > 64,
@@ -528,6 +651,14 @@ static int syn_fwd(const Table *t, const float *z, int32_t B, int32_t counts, in
             GLIF_HIP(hipGetLastError());
             return GLIF_OK;
         }
+        if (ell_counts(t)) {
+            const size_t l = sizeof(float) * static_cast<size_t>(t->n_cols) * kEllBatch + lds;
+            hipLaunchKernelGGL(k_syn_pull_ell, dim3(ceil_div(t->n_post, kBlock), ceil_div(B, kEllBatch)), dim3(kBlock), l,
+                               s, z, B, static_cast<int32_t>(t->n_cols), t->n_post, t->row_ptr, t->ell_pw, t->basis,
+                               t->n_types, t->n_basis, I);
+            GLIF_HIP(hipGetLastError());
+            return GLIF_OK;
+        }
         // Poisson counts scale the weights: a thread per (b, post) over the post's row
         dim3 grid(ceil_div(nI, kBlock));
         hipLaunchKernelGGL(k_syn_pull_dense, grid, dim3(kBlock), lds, s, z, B, t->n_cols, t->n_post,
@@ -537,7 +668,7 @@ static int syn_fwd(const Table *t, const float *z, int32_t B, int32_t counts, in
     }
     int rc = launch_fill_u32(I, 0u, static_cast<size_t>(nI) * t->n_basis, s);
     if (rc) return rc;
-    if (t->n_dwu > 0 && (ceil_div(t->n_cols, kWave) < kPushUnitsMaxScanWaves || t->max_col_len > kDwUnitEntries)) {
+    if (t->n_dwu > 0 && (ceil_div(t->n_cols, kWave) < kPushUnitsMaxScanWaves || t->max_col_len > kPushUnitsMinColLen)) {
         const dim3 grid(static_cast<unsigned>(ceil_div(t->n_dwu, kBlock / kWave)));
         if (counts)
             hipLaunchKernelGGL(k_syn_push_units<true>, grid, dim3(kBlock), lds, s, z, B, t->n_cols, t->dwu, t->n_dwu,
@@ -665,10 +796,14 @@ bool same_g_layout(const Table *a, const Table *b) {
            std::memcmp(a->basis_host, b->basis_host, sizeof(float) * a->n_types * a->n_basis) == 0;
 }
 
-template <int BP>
-static void launch_dz_units(const DzUnitArgs &da, hipStream_t s) {
-    hipLaunchKernelGGL(k_dz_units<BP>, dim3(static_cast<unsigned>(ceil_div(da.n_units, kBlock / kWave))),
-                       dim3(kBlock), 0, s, da);
+static void launch_syn_units(const UnitArgs &a, int Bp, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(ceil_div(a.n_units, kBlock / kWave)));
+    switch (Bp / 4) {
+        case 1: hipLaunchKernelGGL(k_syn_units<1>, grid, dim3(kBlock), 0, s, a); break;
+        case 2: hipLaunchKernelGGL(k_syn_units<2>, grid, dim3(kBlock), 0, s, a); break;
+        case 4: hipLaunchKernelGGL(k_syn_units<4>, grid, dim3(kBlock), 0, s, a); break;
+        default: hipLaunchKernelGGL(k_syn_units<8>, grid, dim3(kBlock), 0, s, a); break;
+    }
 }
 
 int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int32_t counts, float *dz, float *dw,
@@ -690,7 +825,8 @@ int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int3
     // pass always runs over them
     const int64_t walk_lanes = (grouped ? t->n_groups : t->n_cols) * (Bp / 4);
     const bool prefer_units =
-        t->n_dwu > 0 && (t->max_col_len > kUnitDzMinColLen || walk_lanes < kUnitDzMaxWalkLanes);
+        t->n_dwu > 0 && (t->max_col_len > kUnitDzMinColLen ||
+                         (walk_lanes < kUnitDzMaxWalkLanes && (Bp <= 8 || t->n_syn >= kUnitDzMinAvgLen * t->n_cols)));
     const bool dz_units = dz && partial && prefer_units;
     const bool dw_units = dw && (grouped || prefer_units);
     // G, with the zero fill of dW beside it when the units' weight-gradient pass writes only
@@ -711,25 +847,21 @@ int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int3
                            t->n_types, t->n_basis, nullptr, rows, gP, G, g_blocks, dw, n_fill);
     }
     GLIF_HIP(hipGetLastError());
-    if (dz_units) {
-        DzUnitArgs ua{t->n_cols, B, cmp ? 1 : t->n_post, cmp ? rows : 1, Bp, t->dwu, t->n_dwu, t->col_ptr,
-                      cmp ? oc.ps : t->ps, t->w_col, G, dz, partial};
-        switch (Bp) {
-            case 4: launch_dz_units<4>(ua, s); break;
-            case 8: launch_dz_units<8>(ua, s); break;
-            case 16: launch_dz_units<16>(ua, s); break;
-            default: launch_dz_units<32>(ua, s); break;
-        }
+    if (dz_units || (dw && prefer_units)) {
+        const UnitArgs ua{t->n_cols, B, cmp ? 1 : t->n_post, cmp ? rows : 1, counts, z, t->dwu, t->n_dwu, t->col_ptr,
+                          cmp ? oc.ps : t->ps, t->w_col, t->order, G, dz_units ? dz : nullptr, partial, dw};
+        launch_syn_units(ua, Bp, s);
         GLIF_HIP(hipGetLastError());
-        if (t->n_dzc > 0) {
+        if (dz_units && t->n_dzc > 0) {
             hipLaunchKernelGGL(k_dz_chunks, dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(t->n_dzc) * B, kBlock))),
                                dim3(kBlock), 0, s, t->dzc, t->n_dzc, partial, B, Bp, t->n_cols, dz);
             GLIF_HIP(hipGetLastError());
         }
-        dz = nullptr;   // done; the passes below compute dW only
-        if (!dw) return GLIF_OK;
+        // done; what is left is a dz that found no room for the partial sums
+        dw = nullptr;
+        if (dz_units || !dz) return GLIF_OK;
     }
-    if (grouped || (dw_units && !dz)) {
+    if (grouped) {
         // the grouped row-sliced walk for dz (when grouped and dz is still wanted) beside the
         // active columns' dW over the units (every active synapse's written once, in reference
         // order)
@@ -739,7 +871,7 @@ int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int3
         ga.split = gs_split(ga.n_groups, Bp / 4);
         SynDwArgs da{t->n_cols, B, cmp ? 1 : t->n_post, cmp ? rows : 1, Bp, counts, z, t->dwu, t->n_dwu,
                      t->col_ptr, cmp ? oc.ps : t->ps, t->order, G, dw};
-        const int LG = grouped ? Bp / 4 : 2;   // no walk blocks when not grouped
+        const int LG = Bp / 4;
         const int walk_blocks = dz ? static_cast<int>(ceil_div(t->n_groups * LG << ga.split, kBlock)) : 0;
         const int dw_blocks = dw ? static_cast<int>(ceil_div(t->n_dwu, kBlock / kWave)) : 0;
         const dim3 grid(walk_blocks + dw_blocks);
@@ -756,16 +888,6 @@ int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int3
         }
         GLIF_HIP(hipGetLastError());
         return GLIF_OK;
-    }
-    if (dw_units) {
-        // dW over the units (filled beside G), dz by the column walk below (the cell's
-        // per-step backward gives no room for partial sums)
-        SynDwArgs da{t->n_cols, B, cmp ? 1 : t->n_post, cmp ? rows : 1, Bp, counts, z, t->dwu, t->n_dwu,
-                     t->col_ptr, cmp ? oc.ps : t->ps, t->order, G, dw};
-        hipLaunchKernelGGL(k_syn_dw_units, dim3(static_cast<unsigned>(ceil_div(t->n_dwu, kBlock / kWave))),
-                           dim3(kBlock), 0, s, da);
-        GLIF_HIP(hipGetLastError());
-        dw = nullptr;
     }
     // the type-phased column walk writes the active columns' synapses; the rest stay 0
     if (dw && (rc = launch_fill_u32(dw, 0u, static_cast<size_t>(t->n_syn), s))) return rc;

@@ -599,16 +599,17 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
     t->n_chunks = static_cast<int32_t>(chunk_desc.size());
     // weight-gradient work units: runs of short columns, chunks of long ones
     std::vector<int4> dwu;
+    const int unit = dw_unit_entries(n_syn);
     for (int64_t c = 0; c < n_cols;) {
         const int32_t k0 = col_ptr[c], k1 = col_ptr[c + 1];
-        if (k1 - k0 > kDwUnitEntries) {
-            for (int32_t k = k0; k < k1; k += kDwUnitEntries)
-                dwu.push_back(make_int4(static_cast<int>(c), 1, k, std::min(k + kDwUnitEntries, k1)));
+        if (k1 - k0 > unit) {
+            for (int32_t k = k0; k < k1; k += unit)
+                dwu.push_back(make_int4(static_cast<int>(c), 1, k, std::min(k + unit, k1)));
             ++c;
             continue;
         }
         int64_t m = c + 1;
-        while (m < n_cols && m - c < kWave && col_ptr[m + 1] - k0 <= kDwUnitEntries) ++m;
+        while (m < n_cols && m - c < kWave && col_ptr[m + 1] - k0 <= unit) ++m;
         dwu.push_back(make_int4(static_cast<int>(c), static_cast<int>(m - c), k0, col_ptr[m]));
         c = m;
     }
