@@ -1,5 +1,5 @@
-"""GPU parity of the op's backward over work units and over the split column walk, and of the counts
-pull over the padded rows, against the C oracle, at the sizes where they can go wrong: batches around
+"""GPU parity of the op's backward over work units and over the split column walk, of the counts
+pull over the padded rows and of the event push with a lane per receptor, against the C oracle, at the sizes where they can go wrong: batches around
 the padded row lengths (1 to 32), columns of no, one and a few synapses, around a unit's 256 synapses
 and over many of them, runs of more columns than a wave has lane groups, counts and spikes.  The
 forward bit for bit (also where a count is infinite), dz and dW within 1e-5 of each element's sum of
@@ -71,3 +71,29 @@ def test_units(B, kind, counts):
         if kind == "even":   # pulled in event mode too
             ev = t.forward(torch.tensor(z, device="cuda"), counts=True, mode="event").cpu().numpy()
             np.testing.assert_array_equal(ev, ref)
+
+
+@pytest.mark.parametrize("counts", [False, True])
+@pytest.mark.parametrize("nb", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("n_cols", [129, 131073])   # over the work units; by the column scan
+def test_push_receptors(n_cols, nb, counts):
+    from v1_glif_model_amd.ops import SynapseTable
+    rng = np.random.default_rng(nb)
+    n_post, B = 701, 3
+    cols = [(0, 1), (1, 17), (2, 64), (3, 65), (100, 200), (n_cols - 1, 130)]   # (column, synapses)
+    ind = np.concatenate([np.stack([rng.permutation(n_post)[:k], np.full(k, c)], -1) for c, k in cols])
+    ind = ind[np.lexsort((ind[:, 1], ind[:, 0]))]
+    n = len(ind)
+    tab = Tab(ind[:, 0].astype(np.int64), ind[:, 1].astype(np.int64), rng.normal(0, 1, n).astype(np.float32),
+              rng.integers(0, 7, n).astype(np.uint8), n_post, n_cols)
+    basis = rng.normal(0, 1, (7, nb)).astype(np.float32)
+    basis[rng.random(basis.shape) < 0.2] = 0.0
+    z = np.zeros((B, n_cols), np.float32)
+    for c, _ in cols:
+        z[:, c] = rng.integers(0, 3, B) if counts else rng.integers(0, 2, B)
+    print(n_cols, nb, counts, flush=True)
+    t = SynapseTable(ind, tab.syn_id, (n_post, n_cols), basis)
+    t.set_weights(torch.tensor(tab.weight, device="cuda"))
+    ev = t.forward(torch.tensor(z, device="cuda"), counts=counts, mode="event").cpu().numpy()
+    ref = orc.syn_fwd(tab, z, basis, use_count=counts)
+    assert np.max(np.abs(ev - ref) - 1e-5 * dense.syn_fwd_abs(tab, z, basis, use_count=counts)) <= 1e-6

@@ -160,6 +160,7 @@ struct Table {
     uint2 *gs_pw = nullptr;       // [n_gs]        {row | column-in-group << kGsRowBits, weight bits}
     int32_t *gs_src = nullptr;    // [n_gs]        column-grouped position of the synapse, -1 for padding
     float *basis_host = nullptr;  // host copy [n_types][n_basis]
+    int32_t basis_nnz = 0;        // its entries that are not 0
     // Compact G rows: a G row per (post, type reaching the post) instead of per (type, post).
     // cg: set by a cell, over the types reaching each post from any of its three populations;
     // og: the table's own types per post, built at creation (the op-level backward uses it).

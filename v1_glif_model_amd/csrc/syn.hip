@@ -124,6 +124,16 @@ __global__ void __launch_bounds__(kBlock)
     }
 }
 
+// One active column, by a wave; Q = 1: a lane per synapse, else Q lanes (push_column_wide).
+template <int Q, class Mult>
+__device__ inline void push_spiking(int lane, int32_t lo, int32_t hi, uint32_t m, Mult mult,
+                                    const uint32_t *__restrict__ ps, const float *__restrict__ w,
+                                    const float *basis_lds, int nb, int32_t n_post, float *__restrict__ I) {
+    const int64_t bstride = static_cast<int64_t>(n_post) * nb;
+    if (Q == 1) push_column<kWave>(lane, lo, hi, m, mult, ps, w, basis_lds, nb, bstride, nb, 1, I);
+    else push_column_wide<kWave, Q>(lane, lo, hi, m, mult, ps, w, basis_lds, nb, bstride, I);
+}
+
 // Event push straight from z [B][n_cols]: a wave per 64 consecutive columns builds each
 // column's batch mask (z > 0, the test of tf.where at models.py:128-130), and all 64 lanes
 // push the wave's active columns one after another.  No column list, no count pass.
@@ -131,7 +141,7 @@ __global__ void __launch_bounds__(kBlock)
 // at most dw_unit_entries synapses of a long column), a wave per unit: the lanes hold the
 // run's columns' batch masks, and all 64 lanes push each active column's share of the unit.
 // For tables whose column scan would run on few waves (few columns, or long ones).
-template <bool COUNTS>
+template <bool COUNTS, int Q>
 __global__ void __launch_bounds__(kBlock)
     k_syn_push_units(const float *__restrict__ z, int32_t B, int64_t n_cols, const int4 *__restrict__ units,
                      int32_t n_units, const int32_t *__restrict__ col_ptr, const uint32_t *__restrict__ ps,
@@ -155,16 +165,12 @@ __global__ void __launch_bounds__(kBlock)
         const int64_t cl = un.x + l;
         const int32_t lo = un.y == 1 ? un.z : col_ptr[cl];
         const int32_t hi = un.y == 1 ? un.w : col_ptr[cl + 1];
-        if (COUNTS)
-            push_column<kWave>(lane, lo, hi, ml, MultF32{z + cl, n_cols}, ps, w, basis_lds, nb,
-                               static_cast<int64_t>(n_post) * nb, nb, 1, I);
-        else
-            push_column<kWave>(lane, lo, hi, ml, MultOne{}, ps, w, basis_lds, nb, static_cast<int64_t>(n_post) * nb,
-                               nb, 1, I);
+        if (COUNTS) push_spiking<Q>(lane, lo, hi, ml, MultF32{z + cl, n_cols}, ps, w, basis_lds, nb, n_post, I);
+        else push_spiking<Q>(lane, lo, hi, ml, MultOne{}, ps, w, basis_lds, nb, n_post, I);
     }
 }
 
-template <bool COUNTS>
+template <bool COUNTS, int Q>
 __global__ void __launch_bounds__(kBlock)
     k_syn_push_scan(const float *__restrict__ z, int32_t B, int64_t n_cols, const int32_t *__restrict__ col_ptr,
                     const uint32_t *__restrict__ ps, const float *__restrict__ w, const float *__restrict__ basis,
@@ -187,12 +193,9 @@ __global__ void __launch_bounds__(kBlock)
             act &= act - 1ull;
             const uint32_t ml = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(m), l));
             const int64_t cl = u * kWave + l;
-            if (COUNTS)
-                push_column<kWave>(lane, col_ptr[cl], col_ptr[cl + 1], ml, MultF32{z + cl, n_cols}, ps, w,
-                                   basis_lds, nb, static_cast<int64_t>(n_post) * nb, nb, 1, I);
-            else
-                push_column<kWave>(lane, col_ptr[cl], col_ptr[cl + 1], ml, MultOne{}, ps, w, basis_lds, nb,
-                                   static_cast<int64_t>(n_post) * nb, nb, 1, I);
+            const int32_t lo = col_ptr[cl], hi = col_ptr[cl + 1];
+            if (COUNTS) push_spiking<Q>(lane, lo, hi, ml, MultF32{z + cl, n_cols}, ps, w, basis_lds, nb, n_post, I);
+            else push_spiking<Q>(lane, lo, hi, ml, MultOne{}, ps, w, basis_lds, nb, n_post, I);
         }
     }
 }
@@ -668,25 +671,28 @@ static int syn_fwd(const Table *t, const float *z, int32_t B, int32_t counts, in
     }
     int rc = launch_fill_u32(I, 0u, static_cast<size_t>(nI) * t->n_basis, s);
     if (rc) return rc;
+    const int Q = t->basis_nnz < 2 * t->n_types ? 1 : t->n_basis <= 4 ? 4 : 8;   // lanes per synapse
     if (t->n_dwu > 0 && (ceil_div(t->n_cols, kWave) < kPushUnitsMaxScanWaves || t->max_col_len > kPushUnitsMinColLen)) {
         const dim3 grid(static_cast<unsigned>(ceil_div(t->n_dwu, kBlock / kWave)));
-        if (counts)
-            hipLaunchKernelGGL(k_syn_push_units<true>, grid, dim3(kBlock), lds, s, z, B, t->n_cols, t->dwu, t->n_dwu,
-                               t->col_ptr, t->ps, t->w_col, t->basis, t->n_types, t->n_basis, t->n_post, I);
-        else
-            hipLaunchKernelGGL(k_syn_push_units<false>, grid, dim3(kBlock), lds, s, z, B, t->n_cols, t->dwu, t->n_dwu,
-                               t->col_ptr, t->ps, t->w_col, t->basis, t->n_types, t->n_basis, t->n_post, I);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, s, z, B, t->n_cols, t->dwu, t->n_dwu, t->col_ptr,
+                               t->ps, t->w_col, t->basis, t->n_types, t->n_basis, t->n_post, I);
+        };
+        if (Q == 1) counts ? launch(k_syn_push_units<true, 1>) : launch(k_syn_push_units<false, 1>);
+        else if (Q == 4) counts ? launch(k_syn_push_units<true, 4>) : launch(k_syn_push_units<false, 4>);
+        else counts ? launch(k_syn_push_units<true, 8>) : launch(k_syn_push_units<false, 8>);
         GLIF_HIP(hipGetLastError());
         return GLIF_OK;
     }
     const dim3 grid(static_cast<unsigned>(std::max<int64_t>(
         1, std::min<int64_t>(ceil_div(ceil_div(t->n_cols, kWave), kBlock / kWave), 32768))));
-    if (counts)
-        hipLaunchKernelGGL(k_syn_push_scan<true>, grid, dim3(kBlock), lds, s, z, B, t->n_cols, t->col_ptr, t->ps,
-                           t->w_col, t->basis, t->n_types, t->n_basis, t->n_post, I);
-    else
-        hipLaunchKernelGGL(k_syn_push_scan<false>, grid, dim3(kBlock), lds, s, z, B, t->n_cols, t->col_ptr, t->ps,
-                           t->w_col, t->basis, t->n_types, t->n_basis, t->n_post, I);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, s, z, B, t->n_cols, t->col_ptr, t->ps, t->w_col, t->basis,
+                           t->n_types, t->n_basis, t->n_post, I);
+    };
+    if (Q == 1) counts ? launch(k_syn_push_scan<true, 1>) : launch(k_syn_push_scan<false, 1>);
+    else if (Q == 4) counts ? launch(k_syn_push_scan<true, 4>) : launch(k_syn_push_scan<false, 4>);
+    else counts ? launch(k_syn_push_scan<true, 8>) : launch(k_syn_push_scan<false, 8>);
     GLIF_HIP(hipGetLastError());
     return GLIF_OK;
 }

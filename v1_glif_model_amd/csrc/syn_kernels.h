@@ -87,6 +87,32 @@ __device__ inline void push_column(int lane_s, int32_t lo, int32_t hi, uint32_t 
     }
 }
 
+// As push_column, with Q lanes per synapse, one for each receptor (Q >= nb): the currents of one
+// (post, batch entry) are consecutive (rstride 1), so an event's atomics leave as one request and
+// not one per receptor.  Requests bound the push; a basis with one receptor per type has one either
+// way and keeps the form above.  66,000 posts, 250 synapses each, four receptors per type, batch 5,
+// forward and backward: 290 -> 238 us, all of it the push (88 before).
+template <int L, int Q, class Mult>
+__device__ inline void push_column_wide(int lane_s, int32_t lo, int32_t hi, uint32_t bmask, Mult mult,
+                                        const uint32_t *__restrict__ ps, const float *__restrict__ w,
+                                        const float *basis_lds, int nb, int64_t bstride, float *__restrict__ I) {
+    const int r = lane_s % Q;
+    if (r >= nb) return;
+    for (int32_t k = lo + lane_s / Q; k < hi; k += L / Q) {
+        const uint32_t p = ps[k];
+        const float wk = w[k];
+        float *dst = I + static_cast<int64_t>(p & kLow24) * nb + r;
+        const float bs = basis_lds[(p >> 24) * nb + r];
+        uint32_t m = bmask;
+        while (m) {
+            const int b = __ffs(m) - 1;
+            m &= m - 1;
+            const float v = (Mult::kOne ? wk : wk * mult(b)) * bs;
+            if (v != 0.0f) unsafeAtomicAdd(dst + static_cast<int64_t>(b) * bstride, v);
+        }
+    }
+}
+
 // ---- event-driven push of one column into per-type slots ---------------------------
 // As push_column, with one atomic per (synapse, batch entry): (w * mult_b) goes to the
 // synapse's type slot of its post, I[rank * rstride + b * bstride + post] (cps[k] = post |

@@ -625,6 +625,7 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
     t->n_dzc = static_cast<int32_t>(dzc.size());
     t->basis_host = new float[static_cast<size_t>(n_types) * n_basis];
     std::memcpy(t->basis_host, basis, sizeof(float) * n_types * n_basis);
+    for (int i = 0; i < n_types * n_basis; ++i) t->basis_nnz += basis[i] != 0.0f;
     int rc = GLIF_OK;
     if ((rc = upload(&t->basis, basis, static_cast<size_t>(n_types) * n_basis)) ||
         (rc = upload(&t->col_ptr, col_ptr.data(), col_ptr.size())) ||
