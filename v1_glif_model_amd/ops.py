@@ -144,11 +144,11 @@ class SynapseTable:
             self._w_ref = w
 
     def workspace(self, B: int, device) -> torch.Tensor:
-        n = int(lib().glif_syn_workspace(self.handle, int(B)))
-        ws = self._ws.get((B, str(device)))
-        if ws is None or ws.numel() < n:
-            ws = torch.empty(max(n, 1), dtype=torch.uint8, device=device)
-            self._ws[(B, str(device))] = ws
+        # a built table's size for a batch does not change
+        ws = self._ws.get((B, device))
+        if ws is None:
+            n = int(lib().glif_syn_workspace(self.handle, int(B)))
+            ws = self._ws[(B, device)] = torch.empty(max(n, 1), dtype=torch.uint8, device=device)
         return ws
 
     def _check_z(self, z):
@@ -187,13 +187,14 @@ class SynapseTable:
                              f"got {tuple(dy.shape) if torch.is_tensor(dy) else type(dy).__name__}")
         if dy.device != self.device:
             raise ValueError(f"dy is on {dy.device}, the table on {self.device}")
+        dev = z.device
         z = z.contiguous().float()
         dy = dy.contiguous().float()
-        dz = torch.empty((B, self.n_cols), dtype=torch.float32, device=z.device) if want_dz else None
-        dw = torch.empty(self.n_syn, dtype=torch.float32, device=z.device) if want_dw else None
-        ws = self.workspace(B, z.device)
+        dz = torch.empty((B, self.n_cols), dtype=torch.float32, device=dev) if want_dz else None
+        dw = torch.empty(self.n_syn, dtype=torch.float32, device=dev) if want_dw else None
+        ws = self.workspace(B, dev)
         check(lib().glif_syn_bwd(self.handle, ptr(z), ptr(dy), B, int(counts), ptr(dz), ptr(dw),
-                                 ptr(ws), ws.numel(), stream_ptr(z.device)))
+                                 ptr(ws), ws.numel(), stream_ptr(dev)))
         return dz, dw
 
 
