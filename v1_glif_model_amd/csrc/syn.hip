@@ -479,7 +479,7 @@ __global__ void __launch_bounds__(kBlock) k_syn_units(UnitArgs a) {
             for (int u = 0; u < U; ++u) {
                 const int32_t kk = min(k + u * n, k_end - 1);
                 p[u] = a.ps[kk];
-                wk[u] = a.dz && k + u * n < k_end ? a.w[kk] : 0.0f;
+                wk[u] = a.dz ? a.w[kk] : 0.0f;
             }
             float4 g[U];
 #pragma unroll
@@ -487,14 +487,21 @@ __global__ void __launch_bounds__(kBlock) k_syn_units(UnitArgs a) {
                 g[u] = reinterpret_cast<const float4 *>(a.G)[(static_cast<int64_t>(p[u] >> 24) * a.hm +
                                                               static_cast<int64_t>(p[u] & kLow24) * a.lm) * LG + q];
             if (a.dz) {
+                // the rows' terms in pairs, then onto the sums: a quarter of the roundings at their size
+                float4 x[U];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    if (k + u * n >= k_end) break;
-                    acc[0] = acc[0] + wk[u] * g[u].x;
-                    acc[1] = acc[1] + wk[u] * g[u].y;
-                    acc[2] = acc[2] + wk[u] * g[u].z;
-                    acc[3] = acc[3] + wk[u] * g[u].w;
+                    const bool in = k + u * n < k_end;
+                    x[u].x = in ? wk[u] * g[u].x : 0.0f;
+                    x[u].y = in ? wk[u] * g[u].y : 0.0f;
+                    x[u].z = in ? wk[u] * g[u].z : 0.0f;
+                    x[u].w = in ? wk[u] * g[u].w : 0.0f;
                 }
+                static_assert(U == 4, "two pairs");
+                acc[0] = acc[0] + ((x[0].x + x[1].x) + (x[2].x + x[3].x));
+                acc[1] = acc[1] + ((x[0].y + x[1].y) + (x[2].y + x[3].y));
+                acc[2] = acc[2] + ((x[0].z + x[1].z) + (x[2].z + x[3].z));
+                acc[3] = acc[3] + ((x[0].w + x[1].w) + (x[2].w + x[3].w));
             }
             if (live) {
                 float d[U];
@@ -531,7 +538,8 @@ __global__ void __launch_bounds__(kBlock) k_syn_units(UnitArgs a) {
     }
 }
 
-// dz of the one-column units' columns: thread per (column, b), the column's units in order.
+// dz of the one-column units' columns: thread per (column, b), the column's units in order, four at
+// a time in pairs: their sums are the largest, and every rounding at that size counts.
 __global__ void __launch_bounds__(kBlock)
     k_dz_chunks(const int4 *__restrict__ dzc, int32_t n_dzc, const float *__restrict__ partial, int32_t B, int32_t R,
                 int64_t n_cols, float *__restrict__ dz) {
@@ -539,8 +547,12 @@ __global__ void __launch_bounds__(kBlock)
     if (i >= static_cast<int64_t>(n_dzc) * B) return;
     const int4 d = dzc[i / B];
     const int b = static_cast<int>(i % B);
-    float s = partial[static_cast<int64_t>(d.y) * R + b];
-    for (int u = 1; u < d.z; ++u) s = s + partial[static_cast<int64_t>(d.y + u) * R + b];
+    const float *p = partial + static_cast<int64_t>(d.y) * R + b;
+    float s = 0.0f;
+    int u = 0;
+    for (; u + 4 <= d.z; u += 4, p += 4 * static_cast<int64_t>(R))
+        s = s + ((p[0] + p[R]) + (p[2 * static_cast<int64_t>(R)] + p[3 * static_cast<int64_t>(R)]));
+    for (; u < d.z; ++u, p += R) s = s + p[0];
     dz[static_cast<int64_t>(b) * n_cols + d.x] = s;
 }
 
