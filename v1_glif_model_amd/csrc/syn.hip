@@ -418,7 +418,7 @@ __device__ inline void syn_dw_body(const SynDwArgs &a, int64_t bid) {
 // order.  What bounds it is the gathers' latency (kUnitRows rows in flight per lane group, and
 // dw_unit_entries synapses a wave for enough waves).  Whole backward calls, against a lane per
 // synapse for dz, which held whole rows, and dW by a pass of its own, both over 1024-synapse
-// units: background table, 66,000 posts, batch 32, 174 -> 68 us; LGN table at batch 5, 94 -> 58.
+// units: background table, 66,000 posts, batch 32, 174 -> 63 us; LGN table at batch 5, 94 -> 58.
 struct UnitArgs {
     int64_t n_cols;
     int32_t B, hm, lm, counts;  // G row of entry p: (p >> 24) * hm + (p & kLow24) * lm, 4 LG floats
