@@ -147,7 +147,7 @@ static bool ensure_side(Cell *c) {
 
 // Whether the forward runs window by window (k_win_fwd): its recurrent and LGN tables carry
 // spike-major rows, or hold no synapses.  A network whose row offsets outgrow their bound
-// (kSpkMaxOff: about half a million neurons, or ~100k with 256 delay slots) takes a launch per tick.
+// (kSpkMaxOff: about half a million neurons, or 80k with 256 delay slots) takes a launch per tick.
 static bool win_forward(const Cell *c) {
     return (c->rec->n_syn == 0 || c->rec->spk.rows) && (c->lgn->n_syn == 0 || c->lgn->spk.rows);
 }
@@ -2458,7 +2458,10 @@ int glif_cell_create(const glif_cell_config *cfg, const float *decay, const floa
         glif_cell_destroy(reinterpret_cast<glif_cell *>(c));
         return hip_fail(e, "cell upload");
     }
-    if (int rc = plan_g_rows(c)) {
+    int rc = plan_g_rows(c);
+    if (!rc) rc = table_set_spike_rows(tr);
+    if (!rc) rc = table_set_spike_rows(tl);
+    if (rc) {
         glif_cell_destroy(reinterpret_cast<glif_cell *>(c));
         return rc;
     }

@@ -89,7 +89,8 @@ struct PermPlan {
 
 // Spike-major rows (win_kernels.h), range of `bin` posts by range: row q * n_pre + pre of a range
 // holds the synapses of presynaptic neuron pre onto it with delays kSpkDelays q + 1 .., in
-// ascending (column, synapse id).  rows = 0: not built.
+// ascending (column, synapse id).  Made when a cell takes the table for its recurrent or LGN
+// population: nothing else reads them.  rows = 0: not built.
 struct SpikeRows {
     int32_t bin = 0, rows = 0;  // posts per range, rows per range
     int32_t *off = nullptr;     // [ranges * rows + 1] first entry of (range, row)
@@ -178,6 +179,9 @@ struct Table {
 // < g_rows).  A table that already has them keeps them if they are the same, else GLIF_EINVAL.
 // Synchronous.
 int table_set_g_rows(Table *t, const uint8_t *rank, int32_t g_rows);
+// Give a table its spike-major rows (Table::spk), unless it has them, holds no synapses or would
+// take more than kSpkMaxOff offsets.  Synchronous.
+int table_set_spike_rows(Table *t);
 
 // ---- cell ------------------------------------------------------------------
 struct Cell {

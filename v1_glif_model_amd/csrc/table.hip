@@ -315,11 +315,15 @@ static int gather_compact_weights(const Table *t, const CompactRows &c, hipStrea
     return GLIF_OK;
 }
 
+// held while a cell adds its copies to its tables: cells created from several threads may share one
+static std::mutex &table_mutex() {
+    static std::mutex mu;
+    return mu;
+}
+
 int table_set_g_rows(Table *t, const uint8_t *rank, int32_t g_rows) {
     if (g_rows <= 0 || g_rows > 255) return fail(GLIF_EINVAL, "compact G rows per post must be in [1, 255]");
-    // cells created from several threads may share a table
-    static std::mutex mu;
-    std::lock_guard<std::mutex> lock(mu);
+    std::lock_guard<std::mutex> lock(table_mutex());
     const int64_t n = t->n_syn;
     if (t->cg.rows) {
         if (t->cg.rows == g_rows && (n == 0 || std::memcmp(t->cg.rank_host, rank, n) == 0)) return GLIF_OK;
@@ -393,7 +397,7 @@ int32_t spike_bin(int32_t n_post) {
 
 // The spike-major rows from the column-grouped order (ps[k] = post | syn_id << 24): a stable
 // counting sort of its synapses, row by row in ascending (column, id), by (range, row).
-static int build_spike_rows(Table *t, const int32_t *col_ptr, const uint32_t *ps) {
+static int build_spike_rows(const Table *t, const int32_t *col_ptr, const uint32_t *ps, SpikeRows &out) {
     const int32_t bin = spike_bin(t->n_post), nf = (t->n_post + bin - 1) / bin;
     const int64_t groups = (t->n_slots + kSpkDelays - 1) / kSpkDelays, rows = groups * t->n_pre;
     if (t->n_syn == 0 || rows * nf > kSpkMaxOff) return GLIF_OK;
@@ -426,11 +430,41 @@ static int build_spike_rows(Table *t, const int32_t *col_ptr, const uint32_t *ps
         std::fill(at.begin(), at.end(), 0);
     }
     int rc;
-    if ((rc = upload(&t->spk.off, off.data(), off.size())) || (rc = upload(&t->spk.ent, ent.data(), ent.size())) ||
-        (rc = upload(&t->spk.src, src.data(), src.size())))
+    if ((rc = upload(&out.off, off.data(), off.size())) || (rc = upload(&out.ent, ent.data(), ent.size())) ||
+        (rc = upload(&out.src, src.data(), src.size())))
         return rc;
-    t->spk.bin = bin;
-    t->spk.rows = static_cast<int32_t>(rows);
+    out.bin = bin;
+    out.rows = static_cast<int32_t>(rows);
+    return GLIF_OK;
+}
+
+// the weights of a table's spike-major rows, gathered from w_col
+static int gather_spike_weights(const Table *t, hipStream_t s) {
+    if (!t->spk.rows) return GLIF_OK;
+    hipLaunchKernelGGL(k_gather_pair_w, dim3(grid_for(t->n_syn)), dim3(kBlock), 0, s, t->spk.ent, t->w_col,
+                       t->spk.src, t->n_syn);
+    GLIF_HIP(hipGetLastError());
+    return GLIF_OK;
+}
+
+int table_set_spike_rows(Table *t) {
+    std::lock_guard<std::mutex> lock(table_mutex());
+    if (t->spk.rows) return GLIF_OK;
+    std::vector<int32_t> col_ptr;
+    std::vector<uint32_t> ps;
+    SpikeRows rows;
+    int rc;
+    GLIF_HIP(hipDeviceSynchronize());  // weights set on any stream have landed in w_col
+    if ((rc = download(col_ptr, t->col_ptr, static_cast<size_t>(t->n_cols) + 1)) || (rc = download(ps, t->ps, t->n_syn)) ||
+        (rc = build_spike_rows(t, col_ptr.data(), ps.data(), rows))) {
+        for (void *p : {static_cast<void *>(rows.off), static_cast<void *>(rows.ent), static_cast<void *>(rows.src)})
+            if (p) (void)hipFree(p);
+        return rc;
+    }
+    t->spk = rows;
+    // the weights the table already holds (later ones arrive through glif_table_set_weights)
+    if ((rc = gather_spike_weights(t, nullptr))) return rc;
+    GLIF_HIP(hipDeviceSynchronize());
     return GLIF_OK;
 }
 
@@ -661,8 +695,7 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
         }
         if (n_syn) (void)hipMemset(*wp, 0, n_syn * sizeof(float));
     }
-    if ((rc = build_own_rows(t, col_ptr.data(), ps.data(), ph_src.data())) ||
-        (rc = build_spike_rows(t, col_ptr.data(), ps.data()))) {
+    if ((rc = build_own_rows(t, col_ptr.data(), ps.data(), ph_src.data()))) {
         free_table(t);
         return rc;
     }
@@ -713,13 +746,9 @@ int glif_table_set_weights(glif_table *tt, const float *w, void *stream) {
                            t->gs_src, t->n_gs);
         GLIF_HIP(hipGetLastError());
     }
-    if (t->spk.rows) {
-        hipLaunchKernelGGL(k_gather_pair_w, dim3(grid_for(t->n_syn)), dim3(kBlock), 0, s, t->spk.ent, t->w_col,
-                           t->spk.src, t->n_syn);
-        GLIF_HIP(hipGetLastError());
-    }
-    // the compact-row copies (a cell's, the table's own)
-    int rcc = gather_compact_weights(t, t->cg, s);
+    // a cell's copies (spike-major rows, compact rows) and the table's own compact rows
+    int rcc = gather_spike_weights(t, s);
+    if (!rcc) rcc = gather_compact_weights(t, t->cg, s);
     if (!rcc) rcc = gather_compact_weights(t, t->og, s);
     if (rcc) return rcc;
     if (t->ell_len) {
