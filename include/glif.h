@@ -240,6 +240,14 @@ int glif_cell_set_voltage_mask(glif_cell *c, const uint8_t *mask, int32_t n_sele
  * gz_neuron over those ticks only.  Default 0, 0 (every tick). */
 int glif_cell_set_trim(glif_cell *c, int32_t pre_delay, int32_t post_delay);
 
+/* Choose the form of the forward (for timing and testing the forms against each other; results do not
+ * depend on it in deterministic mode, in event mode within its bar): per_tick 1 = a launch per tick,
+ * 0 = windows of three ticks wherever the network allows them (default).  row_spikes: windows sum
+ * the recurrent currents from the posts' rows where a batch entry had at least that many spikes in its
+ * last three ticks (from the second window on; delays up to 6), -1 = by size (default).  The workspace size follows the
+ * form: query glif_cell_workspace again, and run a rollout's backward under the rollout's setting. */
+int glif_cell_set_forward(glif_cell *c, int32_t per_tick, int32_t row_spikes);
+
 /* Layout of the backward's per-synapse-type projection G (no counterpart in the reference,
  * whose gradient projects dy through the basis per receptor, models.py:182-241): rows per
  * post neuron (n_types, or fewer when no post receives more than three quarters of the

@@ -48,6 +48,8 @@ struct CellWs {
     uint64_t *lgnbits;  // [T][B][Wl]        bit pre: x_t[b][pre] > 0 (window forward)
     uint16_t *lgndig;   // [T][B][segments]  their digests (win_kernels.h)
     uint16_t *zdig;     // [(T + D)][B][ranges]  the spikes' digests
+    uint32_t *rate;     // [2][B][kRateRanges]  spikes of some ranges in a window (windows alternate)
+    uint8_t *hist;      // [2][B][Np]        the last 8 ticks' spikes (window forward, windows alternate)
     float *I;           // [2][nb][B][N]   pushed rec + LGN currents (event mode), or
                         // [2][g_rows][B][N] type sums with per-type slots
     float *R, *P;       // [nb][B][N]   psc_rise, psc (receptor-major copies of the state)
@@ -145,11 +147,19 @@ static bool ensure_side(Cell *c) {
     return true;
 }
 
-// Whether the forward runs window by window (k_win_fwd): its recurrent and LGN tables carry
+// Whether a mode's forward runs window by window (k_win_fwd): the cell's recurrent and LGN tables carry
 // spike-major rows, or hold no synapses.  A network whose row offsets outgrow their bound
-// (kSpkMaxOff: about half a million neurons, or 80k with 256 delay slots) takes a launch per tick.
-static bool win_forward(const Cell *c) {
-    return (c->rec->n_syn == 0 || c->rec->spk.rows) && (c->lgn->n_syn == 0 || c->lgn->spk.rows);
+// (kSpkMaxOff: about half a million neurons, or 80k with 256 delay slots) takes a launch per tick, and
+// in event mode one of more than kWinEventMaxNeurons: every range looks up every spike, where the push
+// visits its synapses only.  Us per tick, a launch per tick against windows, in event mode: 230,000 neurons
+// with 300 synapses, batch 1, 0.2 Hz 26 / 22, 51 Hz 193 / 252; batch 16 299 / 165 and 2730 / 1861;
+// 400,000 with 100: batch 1, 0.1 Hz 34 / 39, 26 Hz 79 / 166; batch 16 450 / 328 and 961 / 1950.  In deterministic mode the row pull
+// reads the whole table at any rate: 400,000, batch 1, 222 / 52 and 342 / 191; batch 16 873 / 521 and
+// 1107 / 2179.
+constexpr int32_t kWinEventMaxNeurons = 256 * 1024;
+static bool win_forward(const Cell *c, bool event) {
+    return (c->rec->n_syn == 0 || c->rec->spk.rows) && (c->lgn->n_syn == 0 || c->lgn->spk.rows) && !c->per_tick &&
+           !(event && c->N > kWinEventMaxNeurons);
 }
 
 // Backward window width (reverse ticks per table pass) and G row length.
@@ -177,11 +187,17 @@ static CellWs carve_cell(void *ws, const Cell *c, int32_t B, int32_t T, size_t *
     w.A = cv.take<float>(BN * 2);
     w.zbits = cv.take<uint64_t>(static_cast<size_t>(T + c->D) * B * c->W);
     w.refbits = cv.take<uint64_t>(static_cast<size_t>(T) * B * c->W);
-    if (win_forward(c)) {
+    const bool win = win_forward(c, false), ticks = !win_forward(c, true);   // the forms a mode may take
+    if (win) {
         w.lgnbits = cv.take<uint64_t>(static_cast<size_t>(T) * B * ((nl + 63) / 64));
         w.lgndig = cv.take<uint16_t>(static_cast<size_t>(T) * B * ceil_div(nl, kDigInputs) * kDigHalfs);
         w.zdig = cv.take<uint16_t>(static_cast<size_t>(T + c->D) * B * ceil_div(c->N, spike_bin(c->N)) * kDigHalfs);
-    } else {
+        if (c->D <= kDenseMaxDelay) {
+            w.rate = cv.take<uint32_t>(2 * static_cast<size_t>(B) * kRateRanges);
+            w.hist = cv.take<uint8_t>(2 * static_cast<size_t>(B) * c->Np);
+        }
+    }
+    if (ticks) {
         w.zmask = cv.take<uint32_t>(static_cast<size_t>(T + c->D) * c->Np);
         w.lmask = cv.take<uint32_t>(static_cast<size_t>(T) * nl);
         w.abits = cv.take<uint64_t>(static_cast<size_t>(T + c->D) * c->W);
@@ -193,7 +209,7 @@ static CellWs carve_cell(void *ws, const Cell *c, int32_t B, int32_t T, size_t *
         }
     }
     w.vsave = cv.take<float>(static_cast<size_t>(T) * BN);
-    if (!win_forward(c)) {
+    if (ticks) {
         w.lgn_off = cv.take<int64_t>(T + 1);
         w.lgn_pre = cv.take<int32_t>(static_cast<size_t>(T) * nl);
         w.lgn_mask = cv.take<uint32_t>(static_cast<size_t>(T) * nl);
@@ -224,7 +240,7 @@ static CellWs carve_cell(void *ws, const Cell *c, int32_t B, int32_t T, size_t *
     w.dw_lgn = cv.take<float>(std::max<int64_t>(c->lgn->n_syn, 1));
     w.dw_bkg = cv.take<float>(std::max<int64_t>(c->bkg->n_syn, 1));
     // event mode alternates between the two halves by tick
-    if (!win_forward(c)) w.I = cv.take<float>(2 * BN * i_slots(c));
+    if (ticks) w.I = cv.take<float>(2 * BN * i_slots(c));
     if (bytes) *bytes = cv.off;
     return w;
 }
@@ -889,13 +905,25 @@ k_step_push(StepArgs sa, int step_blocks, PushArgs pa) {
 // (win_kernels.h), so nothing but spike words passes between workgroups, then steps them in
 // registers.  Both modes run it: the sums are the reference's, term by term.
 struct WinArgs {
-    CellConst k;
+    // What a workgroup needs first comes first, and nothing is read of the launch's own arguments, which lie
+    // past the end: a line of arguments to wait for is half a us (66,000 neurons, batch 5: 37.2 us per launch
+    // with the launch's own line).
+    const float *basis;
+    const uint32_t *rate;          // [B][kRateRanges] spikes of some ranges in the window before
+    uint32_t *rate_out;            // and in this one; nullptr: not kept
     int32_t t0, nw, flush;
     int32_t i_lo, i0, i1;          // current ticks i_lo + i0 .. i_lo + i1 - 1, i_lo = t0 - 2
     int32_t RP, n_ranges;          // posts per workgroup, ranges of them
-    int32_t count_t0, count_t1;
+    int32_t B, n_types;            // k's
+    int32_t threads, per_xcd;      // lanes of a workgroup, workgroups per XCD
+    int32_t room;                  // LDS bytes before the basis (WinLds)
+    int32_t keep_hist;             // whether hist is written
+    int32_t limit;                 // 1 + the spikes of a window from which the next one takes win_dense; 0: it does not
     WinSrc rec, lgn;
+    CellConst k;
+    int32_t count_t0, count_t1;
     uint16_t *dig;                 // rec's digests, written for the window's ticks
+    uint8_t *hist;                 // [B][Np] the history after the window's ticks
     float *v;
     int16_t *r;
     float *A, *R, *P;
@@ -911,7 +939,7 @@ struct WinArgs {
     const uint2 *bkg_ell;
     int32_t bkg_ell_len, n_bkg;
     const uint8_t *bkg;            // [T][B][n_bkg]
-    const float *basis;
+    WinDense dense;
 };
 
 // Background currents of post n0 + local at the launch's current ticks: every synapse of the row, weight
@@ -975,18 +1003,19 @@ __global__ void __launch_bounds__(kWinMaxThreads) __attribute__((amdgpu_waves_pe
     const WIN_CONST WinArgs &a = *(const WIN_CONST WinArgs *)__builtin_amdgcn_kernarg_segment_ptr();
     extern __shared__ __align__(16) char win_smem[];
     constexpr int L = (SPLIT ? 2 : 1) * kWinTicks;
-    const WinLds l = WinLds::carve(win_smem, blockDim.x, L, a.RP);
+    const WinLds l = WinLds::carve(win_smem, a.threads, L, a.RP, a.room);
     const WIN_CONST CellConst &k = a.k;
     // XCD-aware order (workgroups go to the 8 XCDs round robin): an XCD takes all batch entries of
     // consecutive ranges, which look up the same ranges' rows
-    const int per = static_cast<int>(gridDim.x) / 8;
-    const int wg = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
-    if (wg >= a.n_ranges * k.B) return;
-    const int range = wg / k.B, b = wg - range * k.B;
+    const int wg = static_cast<int>(blockIdx.x % 8) * a.per_xcd + static_cast<int>(blockIdx.x / 8);
+    if (wg >= a.n_ranges * a.B) return;
+    const int range = wg / a.B, b = wg - range * a.B;
     const int n0 = range * a.RP;
-    for (int i = threadIdx.x; i < L * a.RP; i += blockDim.x) l.heads[i] = -1;
-    for (int i = threadIdx.x; i < k.n_types * NB; i += blockDim.x)
+    for (int i = threadIdx.x; i < L * a.RP; i += a.threads) l.heads[i] = -1;
+    for (int i = threadIdx.x; i < a.n_types * NB; i += a.threads)
         l.basis[i / NB * win_basis_stride(NB) + i % NB] = a.basis[i];
+    uint32_t rate = 0;
+    if (a.limit && (threadIdx.x & (kWave - 1)) < kRateRanges) rate = (a.rate + b * kRateRanges)[threadIdx.x & (kWave - 1)];
     __syncthreads();
     const int64_t BN = static_cast<int64_t>(k.B) * k.N;
     float I[L][NB];
@@ -997,11 +1026,13 @@ __global__ void __launch_bounds__(kWinMaxThreads) __attribute__((amdgpu_waves_pe
     // the entries' room, free once the currents are summed: spike words, background counts
     uint64_t *new_words = reinterpret_cast<uint64_t *>(l.rec);   // [tick][RP / 64]
     uint32_t *room = reinterpret_cast<uint32_t *>(l.rec) + 2 * kWinTicks * (kWinMaxThreads / kWave);
-    const bool cnt_lds = a.n_bkg <= 2 * kWinSlots * static_cast<int>(blockDim.x) - 2 * kWinTicks * (kWinMaxThreads / kWave);
+    const bool cnt_lds = a.n_bkg <= 2 * kWinSlots * a.threads - 2 * kWinTicks * (kWinMaxThreads / kWave);
     if (a.i1 > a.i0) {
-        win_currents<NB, SPLIT>(a.rec, a.lgn, l, k.B, b, a.i_lo, a.i0, a.i1, range, a.RP, I);
+        const bool dense = win_dense_due(rate, a.limit, a.n_ranges);
+        if (__builtin_expect(dense, 0)) win_dense(a.dense, l, a.t0, a.B, b, a.i0, a.i1, n0, a.RP, I);
+        win_currents<NB, SPLIT>(a.rec, a.lgn, !dense, l, a.B, b, a.i_lo, a.i0, a.i1, range, a.RP, I);
         if (cnt_lds) {
-            for (int i = threadIdx.x; i < a.n_bkg; i += blockDim.x) {
+            for (int i = threadIdx.x; i < a.n_bkg; i += a.threads) {
                 uint32_t c = 0;
                 for (int u = a.i0; u < a.i1; ++u)
                     c |= static_cast<uint32_t>(a.bkg[(static_cast<int64_t>(a.i_lo + u) * k.B + b) * a.n_bkg + i]) << (8 * u);
@@ -1111,6 +1142,18 @@ __global__ void __launch_bounds__(kWinMaxThreads) __attribute__((amdgpu_waves_pe
             (a.v + bn0)[local] = v;
             (a.r + bn0)[local] = static_cast<int16_t>(r);
             if (a.spike_count && spikes) (a.spike_count + bn0)[local] += spikes;
+            if (a.keep_hist) {
+                // the history: the window's ticks, then the earlier ones
+                uint32_t h = 0;
+                const int64_t word = static_cast<int64_t>(b) * k.W + (n0 + wave0) / kWave;
+                if (a.t0 > 0) h = (a.dense.hist + (static_cast<int64_t>(b) * k.Np + n0))[local];
+                else
+                    for (int d = min(k.D, 8); d >= 1; --d)
+                        h = h << 1 | static_cast<uint32_t>((a.zbits[static_cast<int64_t>(k.D - d) * k.B * k.W + word] >> lane) & 1ull);
+                for (int w = 0; w < a.nw; ++w)
+                    h = h << 1 | static_cast<uint32_t>((new_words[w * (a.RP / kWave) + wave0 / kWave] >> lane) & 1ull);
+                (a.hist + (static_cast<int64_t>(b) * k.Np + n0))[local] = static_cast<uint8_t>(h);
+            }
         }
     }
     __syncthreads();
@@ -1118,6 +1161,11 @@ __global__ void __launch_bounds__(kWinMaxThreads) __attribute__((amdgpu_waves_pe
         const int t = a.t0 + static_cast<int>(threadIdx.x);
         win_digest(new_words + threadIdx.x * (a.RP / kWave), (min(a.RP, k.Np - n0)) / kWave,
                    a.dig + ((static_cast<int64_t>(t + k.D) * k.B + b) * a.rec.n_seg + range) * kDigHalfs);
+    }
+    if (a.rate_out && threadIdx.x / kWave == 1) {   // another wave's
+        const int per = a.RP / kWave, w = static_cast<int>(lane) / per, i = static_cast<int>(lane) - w * per;
+        const int n = win_wave_scan<false>(w < a.nw && i < (k.Np - n0) / kWave ? __popcll(new_words[lane]) : 0);
+        if (lane == kWave - 1) win_rate(a.rate_out + b * kRateRanges, range, a.n_ranges, static_cast<uint32_t>(n));
     }
 }
 
@@ -1921,6 +1969,63 @@ static int plan_g_rows(Cell *c) {
     return GLIF_OK;
 }
 
+// Where the rows are summed instead of the spikes' entries (win_dense) and how: a.dense, and the LDS
+// before the basis.  Summing the rows costs a workgroup its posts' entries, the spikes' entries cost it the
+// spikes, so the line is a number of spikes per row entry.  Us per tick, spikes' entries / rows, and where they cross: the
+// history in LDS, 66,000 neurons with 250 synapses, batch 32, deterministic, 11 Hz 283 / 359, 21 Hz 508 /
+// 401, 37 Hz 834 / 486 (14 Hz, 2800 spikes in three ticks); batch 1 the same; 30,000 with 220 31 Hz (2750);
+// gathered, 66,000, batch 32, event, 21 Hz 302 / 506, 113 Hz 1510 / 684 (39 Hz, 7700); 230,000 with 300,
+// batch 1, 25 Hz (17,000); 400,000 with 100 4 Hz (5000).
+constexpr float kDenseLdsSpikes = 11.5f, kDenseSpikes = 57.0f;   // per entry of an average row
+
+static void plan_dense(const Cell *c, int32_t B, bool split, const uint8_t *hist, WinArgs &a, int threads, size_t basis,
+                       size_t &room) {
+    const Table *tr = c->rec;
+    const DevShape &ds = dev_shape();
+    WinDense &d = a.dense;
+    d.row = tr->row_ptr;
+    d.pd = tr->pd;
+    d.sid = tr->sid_row;
+    d.w = tr->w_row;
+    d.words = a.rec.words;
+    d.N = c->N;
+    d.Np = c->Np;
+    d.D = c->D;
+    // the LDS that leaves as many workgroups on a CU as there are without it (24 waves of the event form's
+    // 80 registers, 16 of the other's)
+    const size_t per_cu = static_cast<int64_t>(a.n_ranges) * B <= ds.n_cu
+                              ? 1
+                              : std::max<size_t>(1, std::min(ds.lds_per_cu / (room + basis),
+                                                             static_cast<size_t>((split ? 16 : 24) / (threads / kWave))));
+    const size_t fit = std::min(ds.lds_per_block, ds.lds_per_cu / per_cu) - basis;
+    const size_t waves = static_cast<size_t>(threads / kWave);
+    bool in_lds = false;
+    size_t most = room;
+    for (int cap : {512, 384, 320}) {
+        const size_t need = waves * cap * sizeof(uint2);
+        d.cap = cap;
+        most = need + c->Np;
+        if ((in_lds = most <= fit)) break;
+    }
+    if (!in_lds) {
+        // with one workgroup per CU it would fit: the event form of many workgroups, faster by the spikes'
+        // entries than a launch per tick at every rate
+        if (most + basis <= ds.lds_per_block) return;
+        d.cap = 512;
+        d.hist = hist;
+        most = waves * d.cap * sizeof(uint2);
+    }
+    const float row = static_cast<float>(tr->n_syn) / c->N;
+    const float spikes = row * (in_lds ? kDenseLdsSpikes : kDenseSpikes);
+    // not where that is more than 50 Hz: small networks, whose launches the question alone would lengthen
+    if (c->row_spikes < 0 && spikes > 0.05f * kWinTicks * c->N) {
+        d.hist = nullptr;
+        return;
+    }
+    a.limit = 1 + (c->row_spikes >= 0 ? c->row_spikes : static_cast<int32_t>(spikes));
+    room = std::max(room, most);
+}
+
 // The T-step forward, kWinTicks ticks per launch (k_win_fwd).
 static int forward_windows(Cell *c, int32_t B, int32_t T, bool split, const uint8_t *lgn, const uint8_t *bkg, glif_state *st,
                            float *z_out, float *v_out, int32_t *spike_count, const CellWs &w, const CellConst &k,
@@ -1978,8 +2083,18 @@ static int forward_windows(Cell *c, int32_t B, int32_t T, bool split, const uint
     const int64_t digs = static_cast<int64_t>(c->D + kWinTicks - 1) * a.n_ranges + static_cast<int64_t>(kWinTicks) * n_lseg;
     const int threads = static_cast<int>(std::min<int64_t>(
         kWinMaxThreads, std::max<int64_t>(256, ceil_div(std::max<int64_t>(a.RP, digs), kWave) * kWave)));
-    const size_t lds = WinLds::bytes(threads, split ? 2 * kWinTicks : kWinTicks, a.RP, c->n_types, c->nb);
     const dim3 grid(8 * ceil_div(static_cast<int64_t>(a.n_ranges) * B, 8));
+    size_t room = WinLds::room(threads, split ? 2 * kWinTicks : kWinTicks, a.RP);
+    const size_t basis = WinLds::basis_bytes(c->n_types, c->nb);
+    // (a row's byte offsets within a wave's run are 32 bits)
+    if (w.hist && tr->n_syn && tr->n_syn < (int64_t(1) << 30)) plan_dense(c, B, split, w.hist, a, threads, basis, room);
+    const size_t lds = room + basis;
+    a.room = static_cast<int32_t>(room);
+    a.B = B;
+    a.n_types = c->n_types;
+    a.threads = threads;
+    a.per_xcd = static_cast<int32_t>(grid.x / 8);
+    int win = 0;
     for (int t0 = 0, nw = 0; t0 < T; t0 += nw) {
         // windows of kWinTicks ticks, the first one shorter so that the last is tick T - 1 alone
         const int before = T - 1 - t0;
@@ -1990,8 +2105,20 @@ static int forward_windows(Cell *c, int32_t B, int32_t T, bool split, const uint
         a.i_lo = t0 - 2;
         a.i0 = std::max(0, -a.i_lo);
         a.i1 = std::max(a.flush ? kWinTicks : nw, a.i0);
+        WinArgs x = a;
+        if (t0 < kWinTicks) x.limit = 0;   // not a whole window before it
+        if (a.limit) {
+            x.rate = w.rate + (win & 1) * B * kRateRanges;
+            x.rate_out = w.rate + (~win & 1) * B * kRateRanges;
+        }
+        if (a.dense.hist) {
+            x.keep_hist = 1;
+            x.dense.hist = w.hist + (win & 1) * static_cast<size_t>(B) * c->Np;
+            x.hist = w.hist + (~win & 1) * static_cast<size_t>(B) * c->Np;
+        }
+        ++win;
         ProfScope p(kProfStep, s, true);
-        launch_win_fwd(a, split, c->nb, grid, threads, lds, s);
+        launch_win_fwd(x, split, c->nb, grid, threads, lds, s);
     }
     GLIF_HIP(hipGetLastError());
     return GLIF_OK;
@@ -2503,7 +2630,7 @@ int glif_cell_forward(glif_cell *cc, int32_t B, int32_t T, int32_t mode, const u
     const bool event = mode == GLIF_MODE_EVENT;
     const Table *tl = c->lgn, *tb = c->bkg;
     int rc;
-    const bool win = win_forward(c);
+    const bool win = win_forward(c, event);
     // input lists of the backward's LGN / background dW
     const int Wwin = win_width(B), nwin = n_windows(T, Wwin);
     if (nwin > 0) {
@@ -2772,6 +2899,16 @@ int glif_cell_set_g_layout(glif_cell *cc, int32_t compact) {
     c->g_compact = compact != 0;
     c->g_rows = c->g_compact ? c->g_compact_rows : c->n_types;
     c->push_typed = c->g_compact && c->basis_dense;
+    return GLIF_OK;
+}
+
+int glif_cell_set_forward(glif_cell *cc, int32_t per_tick, int32_t row_spikes) {
+    Cell *c = reinterpret_cast<Cell *>(cc);
+    if (!c) return fail(GLIF_EINVAL, "NULL cell");
+    if (per_tick != 0 && per_tick != 1) return fail(GLIF_EINVAL, "per_tick must be 0 or 1");
+    if (row_spikes < -1 || row_spikes == INT32_MAX) return fail(GLIF_EINVAL, "row_spikes must be in [-1, 2^31 - 2]");
+    c->per_tick = per_tick != 0;
+    c->row_spikes = row_spikes;
     return GLIF_OK;
 }
 

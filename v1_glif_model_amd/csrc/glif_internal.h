@@ -38,6 +38,7 @@ static_assert(kGsCols < 7, "column-in-group 7 marks padding (3 bits above the ro
 // kernels owns a range, a thread per post)
 constexpr int kSpkDelays = 8;
 constexpr int kSpkMaxBin = 768;
+constexpr int kPdPad = 2048;   // entries past the post-grouped table's end that may be loaded
 
 // ---- error plumbing -------------------------------------------------------
 void set_error(const std::string &msg);
@@ -117,7 +118,7 @@ struct Table {
     // post-grouped, each row in ascending (col, synapse id)
     int32_t *row_ptr = nullptr;   // [n_post + 1]
     int32_t *perm = nullptr;      // [n_syn]       synapse id at position j
-    uint32_t *pd = nullptr;       // [n_syn]       pre | (delay - 1) << 24
+    uint32_t *pd = nullptr;       // [n_syn + kPdPad]  pre | (delay - 1) << 24, then zeros
     uint32_t *pidx = nullptr;     // [n_syn]       (n_slots - delay) * round64(n_pre) + pre, or null
     uint8_t *sid_row = nullptr;   // [n_syn]
     float *w_row = nullptr;       // [n_syn]
@@ -213,6 +214,10 @@ struct Cell {
     // the step folding the slots through the basis, instead of one atomic per receptor
     bool basis_dense = false;
     bool push_typed = false;
+    // glif_cell_set_forward: a launch per tick in every mode; the spikes of three ticks from which
+    // the window forward sums rows, -1: by its rule
+    bool per_tick = false;
+    int32_t row_spikes = -1;
     // The LGN pass of segment s + 1 runs on a stream of the cell's own while the caller's
     // stream runs segment s's ticks (created on first use, on that call's device; events
     // order the two).  The mutex keeps concurrent forwards on one cell from interleaving their

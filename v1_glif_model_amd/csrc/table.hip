@@ -567,7 +567,7 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
                  n_gs, gs_seg, gs_pw, gs_src);
     }
 
-    std::vector<uint32_t> ps(n_syn), pd(n_syn);
+    std::vector<uint32_t> ps(n_syn), pd(n_syn + kPdPad, 0u);
     // bit index of the entry's presynaptic spike in a stack of per-slot activity planes
     // of round64(n_pre) bits, slot d at plane n_slots - d (the newest step last)
     const int64_t pre_pad = (static_cast<int64_t>(n_pre) + 63) / 64 * 64;

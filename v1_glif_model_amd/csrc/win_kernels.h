@@ -18,6 +18,10 @@
 // UnsortedSegmentSum meets the events of a post (models.py:141-169).  SPLIT (deterministic mode):
 // the two populations have lists, and sums, of their own, as the reference has; otherwise (event
 // mode) one sum takes both.
+//
+// That work grows with the spikes.  Where the batch entry's last window had many, the recurrent currents are summed from the posts' rows instead (win_dense): every entry tested
+// against a history of the last 8 ticks per neuron, the hits added in the same order, so the sums have
+// the same bits.
 #pragma once
 
 #include "glif_internal.h"
@@ -35,6 +39,7 @@ constexpr int kWinSlots = 8;      // linked entries held, per thread
 constexpr int kDigIds = 15, kDigHalfs = 16;   // a digest: u16 count, then up to kDigIds positions
 constexpr int kDigInputs = 512;   // inputs per digest
 constexpr uint32_t kNil16 = 0xFFFF;
+static_assert(kWinTicks * (kWinMaxThreads / kWave) <= kWave);   // a lane per spike word of a workgroup
 static_assert(kWinJ <= kWinSlots && kWinSlots * kWinMaxThreads < static_cast<int>(kNil16));
 
 // Row length of the basis in LDS (vector reads).
@@ -53,8 +58,27 @@ struct WinSrc {
     int32_t seg, n_seg;
 };
 
-// Write the digest of n_words spike words.
-__device__ inline void win_digest(const uint64_t *w, int n_words, uint16_t *dig) {
+// The recurrent population's rows and history (win_dense).
+struct WinDense {
+    const uint64_t *words;  // the spike words (WinSrc::words of the recurrent population)
+    const uint8_t *hist;    // [B][Np], bit k: z of tick t0 - 1 - k; nullptr: made in LDS from the words
+    const int32_t *row;     // post-grouped table: row pointers,
+    const uint32_t *pd;     // pre | (delay - 1) << 24,
+    const uint8_t *sid;
+    const float *w;
+    int32_t N, Np, D;
+    int32_t cap;            // hits queued per wave
+};
+constexpr int kDenseMaxDelay = 6;   // a delay-d spike of the first current tick is bit d + 1
+constexpr int kRateRanges = 8;      // ranges whose spikes are counted for the choice
+constexpr int kDenseU = 4;          // entries per lane tested together,
+constexpr int kDenseAhead = 3;      // and rounds of them loaded ahead (pd's padding holds that many)
+static_assert(2 * kDenseU * kWave * kDenseAhead <= kPdPad);
+constexpr int kDenseLoads = 4;      // hits per lane whose weights are loaded together
+constexpr int kDenseAdd = 4;        // hits of a post read together
+
+// Write the digest of n_words spike words; returns how many spiked.
+__device__ inline uint32_t win_digest(const uint64_t *w, int n_words, uint16_t *dig) {
     uint32_t cnt = 0;
 #pragma unroll 1
     for (int i = 0; i < n_words; ++i) {
@@ -65,6 +89,7 @@ __device__ inline void win_digest(const uint64_t *w, int n_words, uint16_t *dig)
         }
     }
     dig[0] = static_cast<uint16_t>(cnt);
+    return cnt;
 }
 
 // LDS of a workgroup of `threads` threads and RP posts: the linked entries ({weight, next |
@@ -78,14 +103,20 @@ struct WinLds {
     int32_t *heads;
     int32_t *part;
     float *basis;
-    __host__ __device__ static size_t bytes(int threads, int lists, int RP, int n_types, int nb) {
+    int threads;
+    // bytes before the basis, and of the basis
+    static size_t room(int threads, int lists, int RP) {
         return static_cast<size_t>(threads) * (kWinSlots * sizeof(uint2) + kWinK * 6 + kWinJ * 2) +
-               sizeof(int32_t) * (lists * static_cast<size_t>(RP) + 16) +
-               sizeof(float) * static_cast<size_t>(n_types) * win_basis_stride(nb);
+               sizeof(int32_t) * (lists * static_cast<size_t>(RP) + 16);
     }
-    __device__ static WinLds carve(char *p, int threads, int lists, int RP) {
+    static size_t basis_bytes(int n_types, int nb) {
+        return sizeof(float) * static_cast<size_t>(n_types) * win_basis_stride(nb);
+    }
+    __device__ static WinLds carve(char *p, int threads, int lists, int RP, int room) {
         // threads and RP are multiples of 64: every part starts on a multiple of 16 bytes
         WinLds l;
+        l.threads = threads;
+        l.basis = reinterpret_cast<float *>(p + room);
         l.rec = reinterpret_cast<uint2 *>(p);
         p += threads * kWinSlots * sizeof(uint2);
         l.vbase = reinterpret_cast<int32_t *>(p);
@@ -97,8 +128,6 @@ struct WinLds {
         l.heads = reinterpret_cast<int32_t *>(p);
         p += lists * RP * sizeof(int32_t);
         l.part = reinterpret_cast<int32_t *>(p);
-        p += 16 * sizeof(int32_t);
-        l.basis = reinterpret_cast<float *>(p);
         return l;
     }
 };
@@ -123,7 +152,7 @@ __device__ inline int win_wave_scan(int x) {
 // came before it.
 template <bool MAX>
 __device__ inline int win_scan(const WinLds &l, int v, int *total) {
-    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave, waves = blockDim.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave, waves = l.threads / kWave;
     const int x = win_wave_scan<MAX>(v);
     if (lane == kWave - 1) l.part[wv] = x;
     __syncthreads();
@@ -198,14 +227,233 @@ __device__ inline void win_sum_post(const WinLds &l, int RP, int local, float (&
     }
 }
 
+// the element at a byte offset below 4 GiB of a uniform pointer (scalar-base addresses)
+template <class T>
+__device__ inline T win_ld(const T *p, uint32_t byte) {
+    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + byte);
+}
+
+// The 8 x 8 bit matrix x (row r in byte r) transposed: Hacker's Delight's three exchanges of blocks.
+__device__ inline uint64_t win_transpose(uint64_t x) {
+    uint64_t t = (x ^ (x >> 7)) & 0x00AA00AA00AA00AAull;
+    x ^= t ^ (t << 7);
+    t = (x ^ (x >> 14)) & 0x0000CCCC0000CCCCull;
+    x ^= t ^ (t << 14);
+    t = (x ^ (x >> 28)) & 0x00000000F0F0F0F0ull;
+    return x ^ t ^ (t << 28);
+}
+
+// Whether a window takes win_dense, of the batch entry's row of the rates (n: lane j the j-th, loaded where there is
+// other work to wait for, and not by a scalar load: every wait for one waits for all).
+__device__ inline bool win_dense_due(uint32_t n, int limit, int n_ranges) {
+    uint32_t sum = 0;
+#pragma unroll
+    for (int j = 0; j < kRateRanges; ++j) sum += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(n), j));
+    return limit && static_cast<int64_t>(sum) * n_ranges >= static_cast<int64_t>(limit - 1) * kRateRanges;
+}
+
+// The spikes n of a window in range `range`, where that is one of those looked at.
+__device__ inline void win_rate(uint32_t *rate, int range, int n_ranges, uint32_t n) {
+#pragma unroll
+    for (int j = 0; j < kRateRanges; ++j)
+        if (j * n_ranges / kRateRanges == range) rate[j] = n;
+}
+
+// The recurrent currents of the ticks i_lo + [i0, i1) for the RP posts from n0 on in batch entry b, from
+// their rows: a wave takes its 64 posts' rows as one run of entries, 256 at a time, and queues the hits
+// ({entry, the ticks it arrives in << 16}) in LDS in row order; once a queue is nearly full their weights
+// and types are loaded together, in place, and added post by post, a lane per tick and receptor.  Called by every thread; leaves the heads at -1.
+template <int NB, int L>
+__device__ inline void win_dense(const WIN_CONST WinDense &a, const WinLds &l, int t0, int B, int b, int i0, int i1, int n0,
+                                 int RP, float (&s)[L][NB]) {
+    constexpr int BS = win_basis_stride(NB), U = kDenseU;
+    const int tid = threadIdx.x, threads = l.threads, lane = tid & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave), wave0 = wv * kWave;
+    // the history where it fits, then the waves' queues
+    char *base = reinterpret_cast<char *>(l.rec);
+    uint2 *queue = reinterpret_cast<uint2 *>(base + (a.hist ? 0 : a.Np)) + wv * a.cap;
+    if (!a.hist) {
+        // a thread per word: 8 neurons' bits of 8 ticks are an 8 x 8 bit matrix, transposed
+        const int W = a.Np / kWave;
+        for (int i = tid; i < W; i += threads) {
+            uint64_t x[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                x[k] = k <= a.D + 1 ? a.words[(static_cast<int64_t>(t0 - 1 - k + a.D) * B + b) * W + i] : 0ull;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                uint64_t m = 0;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) m |= (x[k] >> (8 * j) & 0xFFull) << (8 * k);
+                reinterpret_cast<uint64_t *>(base)[i * 8 + j] = win_transpose(m);
+            }
+        }
+    }
+    __syncthreads();
+    if (wave0 < RP && n0 + wave0 < a.N) {
+        // bits of a history byte shifted by delay - 1: 2, 1, 0 for the current ticks 0, 1, 2
+        uint32_t ticks = 0;
+        for (int i = i0; i < i1; ++i) ticks |= 4u >> i;
+        const int32_t rp = a.row[min(n0 + wave0 + lane, a.N)];
+        const int32_t j0 = __builtin_amdgcn_readfirstlane(rp);
+        const int32_t j1 = __builtin_amdgcn_readfirstlane(a.row[min(n0 + wave0 + kWave, a.N)]);
+        constexpr int32_t kNone = 0x7FFFFFFF;
+        int32_t first = kNone;   // this post's first hit, counted over the wave's
+        int known = 0;           // posts whose rows have begun, and where the next one's does
+        int32_t begin = 0;       // (from j0)
+        int32_t hits = 0, q0 = 0;   // hits so far, the first one in the queue
+        auto fence = [&]() {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        };
+        // LP lanes add a post's hits, one for each tick and receptor, G posts at a time
+        constexpr int LP = 3 * NB <= 4 ? 4 : 3 * NB <= 8 ? 8 : 3 * NB <= 16 ? 16 : 32, G = kWave / LP;
+        static_assert(kWinTicks == 3);
+        const int g = lane / LP;
+        const uint32_t r4 = lane % LP % NB * 4, bit = lane % LP < 3 * NB ? 0x40000u >> (lane % LP / NB) : 0u;
+        int posts = 0;         // posts done
+        float carry = 0.0f;    // the next one's sums so far (lanes 0 .. LP - 1, and their copies)
+        auto add = [&](bool last) {
+            // the queued hits' weights and types, all loads of kDenseLoads rounds together
+            fence();
+#pragma unroll 1
+            for (int32_t i0 = 0; i0 < hits - q0; i0 += kDenseLoads * kWave) {
+                uint2 e[kDenseLoads];
+                float w[kDenseLoads];
+                uint32_t sid[kDenseLoads];
+#pragma unroll
+                for (int u = 0; u < kDenseLoads; ++u) {
+                    e[u] = queue[min(i0 + u * kWave + lane, hits - q0 - 1)];
+                    w[u] = win_ld(a.w + j0, e[u].x * 4u);
+                    sid[u] = win_ld(a.sid + j0, e[u].x);
+                }
+                fence();   // a clamped lane reads a slot that another lane writes
+#pragma unroll
+                for (int u = 0; u < kDenseLoads; ++u)
+                    if (i0 + u * kWave + lane < hits - q0)
+                        queue[i0 + u * kWave + lane] = make_uint2(__float_as_uint(w[u]), sid[u] * (BS * 4) | e[u].y);
+            }
+            fence();
+            const int done_to = last ? known : known - 1;   // the last row begun is perhaps not at its end
+#pragma unroll 1
+            for (int p0 = posts; p0 < known; p0 += G) {
+                const int p = p0 + g;
+                int32_t i = __shfl(first, min(p, kWave - 1), kWave), end = __shfl(first, min(p + 1, kWave - 1), kWave);
+                i = p < known ? max(i, q0) : q0;   // a row not begun has no hits, and no first one
+                end = p < known ? (p + 1 < known ? end : hits) : q0;
+                float acc = p == posts ? carry : 0.0f;
+                const uint2 *q = queue + (i - q0);
+                auto term = [&](const uint2 e) { return __uint_as_float(e.x) * win_ld(l.basis, (e.y & 0xFFFFu) + r4); };
+#pragma unroll 1
+                for (; i + kDenseAdd <= end; i += kDenseAdd, q += kDenseAdd) {
+                    uint2 e[kDenseAdd];
+                    float x[kDenseAdd];
+#pragma unroll
+                    for (int u = 0; u < kDenseAdd; ++u) e[u] = q[u];
+#pragma unroll
+                    for (int u = 0; u < kDenseAdd; ++u) x[u] = term(e[u]);
+#pragma unroll
+                    for (int u = 0; u < kDenseAdd; ++u) acc = e[u].y & bit ? acc + x[u] : acc;
+                }
+#pragma unroll 1
+                for (; i < end; ++i, ++q) {
+                    const uint2 e = *q;
+                    const float x = term(e);
+                    acc = e.y & bit ? acc + x : acc;
+                }
+                // to the posts' lanes
+                const bool mine = lane >= p0 && lane < p0 + G && lane < done_to;
+#pragma unroll
+                for (int t = 0; t < kWinTicks; ++t)
+#pragma unroll
+                    for (int q = 0; q < NB; ++q) {
+                        const float x = __shfl(acc, (lane - p0) * LP + t * NB + q, kWave);
+                        s[t][q] = mine ? x : s[t][q];
+                    }
+                if (p0 + G >= known) carry = __shfl(acc, (known - 1 - p0) * LP + lane % LP, kWave);
+            }
+            posts = done_to;
+            fence();
+            q0 = hits;
+        };
+        const uint32_t n = static_cast<uint32_t>(j1 - j0);
+        // hist(pre): the history byte; one loop for each place it is read from, so that each waits for its
+        // own kind of load only
+        auto walk = [&](auto hist) {
+            uint32_t next[kDenseAhead][U];
+            // the entries from `at` on: past the run's end the next rows', past the table's its padding
+            auto load = [&](uint32_t (&x)[U], const uint32_t *at) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) x[u] = win_ld(at, static_cast<uint32_t>(lane + u * kWave) * 4u);
+            };
+            const uint32_t *at = a.pd + j0;
+            // the entries x of [j, j + U waves), and x loaded anew kDenseAhead rounds on (rounds past the run's
+            // end find nothing: a round that may be left out makes the next wait for every load)
+            auto round = [&](uint32_t (&x)[U], uint32_t j) {
+                uint32_t m[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) m[u] = hist(x[u] & kLow24);
+#pragma unroll
+                for (int u = 0; u < U; ++u) m[u] = (m[u] >> (x[u] >> 24)) & ticks;
+                at += U * kWave;
+                load(x, at + (kDenseAhead - 1) * U * kWave);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const uint32_t ju = j + u * kWave, in = ju < n ? min(n - ju, 64u) : 0u;   // lanes before the run's end
+                    const uint64_t on = __ballot(m[u] != 0u) & (in ? ~0ull >> (kWave - in) : 0ull);
+                    while (begin < static_cast<int32_t>(ju) + kWave) {   // a row begins here
+                        const int32_t h = hits + __popcll(on & ((1ull << (begin - ju)) - 1ull));
+                        first = lane == known ? h : first;
+                        begin = ++known < kWave ? __builtin_amdgcn_readlane(rp, known) - j0 : kNone;
+                    }
+                    if (on) {
+                        if (__builtin_amdgcn_inverse_ballot_w64(on)) {
+                            const int before = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(on >> 32),
+                                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(on), 0));
+                            queue[hits - q0 + before] = make_uint2(ju + lane, m[u] << 16);
+                        }
+                        hits += __popcll(on);
+                    }
+                }
+                if (hits - q0 > a.cap - U * kWave) add(false);
+            };
+#pragma unroll
+            for (int k = 0; k < kDenseAhead; ++k) load(next[k], at + k * U * kWave);
+#pragma unroll 1
+            for (uint32_t j = 0; j < n; j += kDenseAhead * U * kWave) {
+#pragma unroll
+                for (int k = 0; k < kDenseAhead; ++k) round(next[k], j + k * U * kWave);
+            }
+            first = lane >= known ? hits : first;   // rows that begin at the run's end
+            known = kWave;
+            add(true);
+        };
+        using lds_u8 = const __attribute__((address_space(3))) uint8_t;
+        using global_u8 = const __attribute__((address_space(1))) uint8_t;
+        if (n == 0) {
+        } else if (!a.hist) {
+            lds_u8 *h = (lds_u8 *)base;
+            walk([&](uint32_t pre) -> uint32_t { return h[pre]; });
+        } else {
+            global_u8 *h = (global_u8 *)(a.hist + static_cast<int64_t>(b) * a.Np);
+            walk([&](uint32_t pre) -> uint32_t { return h[pre]; });
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < L * RP; i += threads) l.heads[i] = -1;
+    __syncthreads();
+}
+
 // Currents of the ticks i_lo + [i0, i1) (0 <= i0, i1 <= kWinTicks) for the RP posts of range `range`
-// (the first one's number's low bits: post0) in batch entry b, from the recurrent population (rec)
-// and the inputs (inp), added to s of the post's thread: [tick], or SPLIT [population][tick].
+// (the first one's number's low bits: post0) in batch entry b, from the recurrent population (rec; not with
+// with_rec false) and the inputs (inp), added to s of the post's thread: [tick], or SPLIT [population][tick].
 // Called by every thread; heads are all -1 on entry and on return.
 template <int NB, bool SPLIT>
-__device__ inline void win_currents(const WIN_CONST WinSrc &rec, const WIN_CONST WinSrc &inp, const WinLds &l, int B, int b, int i_lo,
-                                    int i0, int i1, int range, int RP, float (&s)[(SPLIT ? 2 : 1) * kWinTicks][NB]) {
-    const int tid = threadIdx.x, threads = blockDim.x;
+__device__ inline void win_currents(const WIN_CONST WinSrc &rec, const WIN_CONST WinSrc &inp, bool with_rec, const WinLds &l,
+                                    int B, int b, int i_lo, int i0, int i1, int range, int RP,
+                                    float (&s)[(SPLIT ? 2 : 1) * kWinTicks][NB]) {
+    const int tid = threadIdx.x, threads = l.threads;
     const int n_load = kWinJ * threads, n_slots = kWinSlots * threads, n_list = kWinK * threads;
     const uint32_t post0 = static_cast<uint32_t>(range) * static_cast<uint32_t>(RP);
     // Segments in visit order: rows of n_seg, one per (delay group q, spike tick), the latest
@@ -213,7 +461,7 @@ __device__ inline void win_currents(const WIN_CONST WinSrc &rec, const WIN_CONST
     // of fewer delays, from fewer) -- then one per input tick.
     const int per = i1 - i0 - 1 + kSpkDelays, groups = (rec.D + kSpkDelays - 1) / kSpkDelays;
     const uint32_t n_rec =
-        rec.rows ? static_cast<uint32_t>(groups * per - (groups * kSpkDelays - rec.D)) * static_cast<uint32_t>(rec.n_seg) : 0u;
+        with_rec && rec.rows ? static_cast<uint32_t>(groups * per - (groups * kSpkDelays - rec.D)) * static_cast<uint32_t>(rec.n_seg) : 0u;
     const uint32_t n_all = n_rec + (inp.rows ? static_cast<uint32_t>(i1 - i0) * static_cast<uint32_t>(inp.n_seg) : 0u);
     const int32_t *off_r = rec.off + static_cast<int64_t>(range) * rec.rows;
     const int32_t *off_i = inp.off + static_cast<int64_t>(range) * inp.rows;

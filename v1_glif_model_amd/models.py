@@ -150,6 +150,13 @@ class V1Column:
         backward."""
         check(lib().glif_cell_set_g_layout(self.handle, int(bool(compact))))
 
+    def set_forward(self, per_tick: bool = False, row_spikes: int = -1):
+        """The form of the next rollouts' forward (and of their backward): a launch per tick, or windows of
+        three ticks, which sum a batch entry's recurrent currents from the posts' rows where its last three ticks
+        had at least ``row_spikes`` spikes (-1: by size).  The forms differ in time only (in
+        event mode also in the order of sums)."""
+        check(lib().glif_cell_set_forward(self.handle, int(bool(per_tick)), int(row_spikes)))
+
     def workspace(self, B: int, T: int) -> torch.Tensor:
         n = int(lib().glif_cell_workspace(self.handle, int(B), int(T)))
         ws = self._ws.get("ws")
