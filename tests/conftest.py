@@ -27,3 +27,17 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+@pytest.fixture(params=["windows", "per_tick"])
+def both_forwards(request, monkeypatch):
+    """The test twice: its cells' forward by windows of three ticks (where the network allows them), and by a
+    launch per tick."""
+    from v1_glif_model_amd import models
+    init = models.V1Column.__init__
+
+    def with_form(self, *args, **kw):
+        init(self, *args, **kw)
+        self.set_forward(per_tick=request.param == "per_tick")
+    monkeypatch.setattr(models.V1Column, "__init__", with_form)
+    return request.param

@@ -13,7 +13,7 @@ from oracle.cpu import OracleCell
 from tests.helpers import network, tiny_config
 from v1_glif_model_amd import synthetic as sy
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("both_forwards")]
 
 
 def _cell(tb_net, mode, **kw):

@@ -22,7 +22,7 @@ from tests.helpers import assert_grads_per_element, error_summary, tiny_config
 from v1_glif_model_amd import synthetic as sy
 from v1_glif_model_amd.tables import build_cell_tables
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("both_forwards")]
 
 KW = dict(gauss_std=0.3, dampening_factor=0.1, recurrent_dampening_factor=0.1, voltage_gradient_dampening=0.5,
           pseudo_gauss=True)

@@ -33,7 +33,7 @@ from tests.helpers import tiny_config
 from v1_glif_model_amd import synthetic as sy
 from v1_glif_model_amd.tables import build_cell_tables
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("both_forwards")]
 
 BATCHES = [1, 2, 3, 5, 8, 9]
 KW = dict(gauss_std=0.3, damp=0.3, rd=0.2, vgd=0.4, pseudo_gauss=True)

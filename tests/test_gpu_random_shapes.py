@@ -18,7 +18,7 @@ from tests.test_gpu_shapes import _state_np
 from v1_glif_model_amd import synthetic as sy
 from v1_glif_model_amd.tables import build_cell_tables
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("both_forwards")]
 
 
 def _draw(n_cases=40, seed=2026):

@@ -26,7 +26,7 @@ from tests.helpers import assert_grads_per_element, tiny_config
 from v1_glif_model_amd import synthetic as sy
 from v1_glif_model_amd.tables import build_cell_tables
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("both_forwards")]
 
 # (N, fan-in, D, nb, n_types, B, T, n_lgn, lgn fan-in, pseudo_gauss, input weight scale: set so
 # that 3-7 % of the (tick, batch, neuron) entries spike)
