@@ -45,3 +45,37 @@ def test_walk(n, D, B):
         scale = np.max(np.abs(e))
         assert scale > 0, k
         assert np.max(np.abs(a - e)) <= 1e-5 * scale + 1e-6, k
+
+
+def test_wide_windows_where_their_rows_fit():
+    """A batch of 6 takes windows of three ticks, whose 32-float rows outgrow 4 GiB from 33.6 million
+    rows on (here 141,000 neurons, 240 types, type by type): windows of one tick there, with both G layouts on
+    one rollout."""
+    from v1_glif_model_amd.models import V1Column
+    n, B, T = 141_000, 6, 9
+    cfg = dataclasses.replace(tiny_config(n=n, fanin=2, delays=1, n_lgn=60, lgn_fanin=3, n_bkg=6, bkg_fanin=2,
+                                          rs=3.0, ins=60.0, lgn_p=0.1),
+                              n_basis=2, n_syn_types=240, fanin_mean=2, fanin_sigma=None)
+    net = sy.make_network(cfg, seed=5, dense_basis=True)
+    lgn, bkg = sy.make_inputs(cfg, seed=6, seq_len=T, batch=B)
+    oc = OracleCell(build_cell_tables(net), gauss_std=0.5, damp=0.5, rd=0.5, vgd=0.5, pseudo_gauss=True)
+    oz, ov, oref, _ = oc.forward(lgn, bkg)
+    gz = np.random.default_rng(B).normal(0, 1, oz.shape).astype(np.float32)
+    og = oc.backward(lgn, bkg, oz, oref, ov, gz_loss=gz)
+    cell = V1Column(net, mode="deterministic", gauss_std=0.5, dampening_factor=0.5, recurrent_dampening_factor=0.5,
+                    voltage_gradient_dampening=0.5, pseudo_gauss=True)
+    assert cell.g_layout()[1]
+    cell.set_g_layout(False)
+    ws = cell.workspace(B, T)
+    cell.set_g_layout(True)
+    z, _, _ = cell.rollout(lgn, bkg, ws=ws)
+    np.testing.assert_array_equal(z.cpu().numpy().astype(np.uint8), oz)
+    for compact in (True, False):
+        cell.set_g_layout(compact)
+        print("compact", compact, flush=True)
+        g = cell.backward(gz=torch.tensor(gz, device="cuda"))
+        for k in ("rec", "lgn", "bkg"):
+            a, e = g[k].cpu().numpy(), og[k]
+            scale = np.max(np.abs(e))
+            assert scale > 0, k
+            assert np.max(np.abs(a - e)) <= 1e-5 * scale + 1e-6, (compact, k)

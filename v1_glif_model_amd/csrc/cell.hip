@@ -165,7 +165,14 @@ static bool win_forward(const Cell *c, bool event) {
 // Backward window width (reverse ticks per table pass) and G row length.
 // Three ticks while their batch entries fit a 32-float row: one walk of 128-byte rows for three of
 // 32- or 64-byte ones (batch 7 at 66,000 neurons: 295 us per 3 ticks against 431; batch 10: 315 against 581).
-static int win_width(int B) { return 3 * B <= 32 ? 3 : 1; }
+// A batch of 6 to 10 takes one tick where that row would carry G past its 4 GiB of 32-bit byte offsets (121 types type by
+// type: 277,000 neurons) and a shorter one does not.  By the type-major rows: the width must not change
+// with the G layout, the input lists of a rollout's windows being made by its forward.
+constexpr int64_t kMaxGBytes = int64_t(1) << 32;
+static int win_width(const Cell *c, int B) {
+    const int64_t rows = static_cast<int64_t>(c->N) * c->n_types;
+    return 3 * B <= 16 || (3 * B <= 32 && rows * g_row(3, B) * 4 < kMaxGBytes) ? 3 : 1;
+}
 static int n_windows(int T, int Wwin) { return T >= 3 ? (T - 2 + Wwin - 1) / Wwin : 0; }
 static int ring_size(const Cell *c) { return c->D + 6; }
 
@@ -214,7 +221,7 @@ static CellWs carve_cell(void *ws, const Cell *c, int32_t B, int32_t T, size_t *
         w.lgn_pre = cv.take<int32_t>(static_cast<size_t>(T) * nl);
         w.lgn_mask = cv.take<uint32_t>(static_cast<size_t>(T) * nl);
     }
-    const int Wwin = win_width(B), nwin = std::max(n_windows(T, Wwin), 1);
+    const int Wwin = win_width(c, B), nwin = std::max(n_windows(T, Wwin), 1);
     w.lw_off = cv.take<int64_t>(nwin + 1);
     w.lw_pre = cv.take<int32_t>(static_cast<size_t>(nwin) * nl);
     w.lw_mask = cv.take<uint32_t>(static_cast<size_t>(nwin) * nl);
@@ -2632,7 +2639,7 @@ int glif_cell_forward(glif_cell *cc, int32_t B, int32_t T, int32_t mode, const u
     int rc;
     const bool win = win_forward(c, event);
     // input lists of the backward's LGN / background dW
-    const int Wwin = win_width(B), nwin = n_windows(T, Wwin);
+    const int Wwin = win_width(c, B), nwin = n_windows(T, Wwin);
     if (nwin > 0) {
         if ((rc = build_window_mask_lists(lgn, T, B, tl->n_cols, Wwin, nwin, w.lw_off, w.lw_pre, w.lw_mask,
                                           w.scratch, s)))
@@ -2688,7 +2695,7 @@ int glif_cell_backward(glif_cell *cc, int32_t B, int32_t T, const float *gz, con
         (rc = launch_fill_u32(w.gR, 0u, BN * c->nb, s)))
         return rc;
     // padding elements of each G row stay zero
-    const size_t g_elems = static_cast<size_t>(c->N) * c->g_rows * g_row(win_width(B), B);
+    const size_t g_elems = static_cast<size_t>(c->N) * c->g_rows * g_row(win_width(c, B), B);
     if ((rc = launch_fill_u32(w.G, 0u, 2 * g_elems, s))) return rc;
     const bool cg = c->g_compact;
     const bool gs = (cg ? tr->cg.n_gs : tr->n_gs) > 0;   // the grouped row-sliced walk
@@ -2696,8 +2703,8 @@ int glif_cell_backward(glif_cell *cc, int32_t B, int32_t T, const float *gz, con
     if (dw_lgn && (rc = launch_fill_u32(w.dw_lgn, 0u, tl->n_syn, s))) return rc;
     if (dw_bkg && (rc = launch_fill_u32(w.dw_bkg, 0u, tb->n_syn, s))) return rc;
 
-    const int Wwin = win_width(B), ring = ring_size(c), Rg = g_row(Wwin, B);
-    if (static_cast<int64_t>(c->g_rows) * c->N * Rg * 4 >= (int64_t(1) << 32))
+    const int Wwin = win_width(c, B), ring = ring_size(c), Rg = g_row(Wwin, B);
+    if (static_cast<int64_t>(c->g_rows) * c->N * Rg * 4 >= kMaxGBytes)
         return fail(GLIF_ERANGE, "G rows per neuron * n_neurons * G row * 4 bytes must be < 4 GiB");
     AdjArgs aa{};
     aa.k = k;
