@@ -22,7 +22,10 @@ LENGTHS = {
     "short": [0, 5, 9, 1, 3, 0, 2, 4] * 17 + [300, 1, 0],
     # middling columns: units at every batch
     "middle": [97, 130, 256, 300, 0, 64, 511] * 5,
+    # columns of many units, whose sums several lanes add
+    "tall": [20000, 300, 0, 12345, 1],
 }
+POSTS = {"tall": 20000}
 
 
 def _table(kind, rng):
@@ -31,16 +34,16 @@ def _table(kind, rng):
                  for p in range(N) for k in [10 if p < N - 3 else N - p]]
         ind, n_cols = np.concatenate(pairs), 100
     else:
-        cols = [np.stack([rng.permutation(N)[:k], np.full(k, c)], -1) for c, k in enumerate(LENGTHS[kind])]
+        cols = [np.stack([rng.permutation(POSTS.get(kind, N))[:k], np.full(k, c)], -1) for c, k in enumerate(LENGTHS[kind])]
         ind, n_cols = np.concatenate(cols), len(LENGTHS[kind])
         ind = ind[np.lexsort((ind[:, 1], ind[:, 0]))]
     n = len(ind)
     return Tab(ind[:, 0].astype(np.int64), ind[:, 1].astype(np.int64), rng.normal(0, 1, n).astype(np.float32),
-               rng.integers(0, 5, n).astype(np.uint8), N, n_cols), ind
+               rng.integers(0, 5, n).astype(np.uint8), POSTS.get(kind, N), n_cols), ind
 
 
 @pytest.mark.parametrize("counts", [False, True])
-@pytest.mark.parametrize("kind", ["long", "short", "middle", "even"])
+@pytest.mark.parametrize("kind", ["long", "short", "middle", "even", "tall"])
 @pytest.mark.parametrize("B", [1, 4, 5, 9, 16, 17, 32])
 def test_units(B, kind, counts):
     from v1_glif_model_amd.ops import SynapseTable
@@ -48,17 +51,21 @@ def test_units(B, kind, counts):
     tab, ind = _table(kind, rng)
     basis = rng.random((5, 4)).astype(np.float32)
     print(B, kind, counts, flush=True)
-    t = SynapseTable(ind, tab.syn_id, (N, tab.n_cols), basis)
+    t = SynapseTable(ind, tab.syn_id, (tab.n_post, tab.n_cols), basis)
     t.set_weights(torch.tensor(tab.weight, device="cuda"))
     z = (rng.random((B, tab.n_cols)) < 0.3).astype(np.float32)
     if counts:
         z *= rng.integers(1, 4, z.shape).astype(np.float32)
-    dy = rng.normal(0, 1, (B * N, 4)).astype(np.float32)
-    dz, dw = t.backward(torch.tensor(z, device="cuda"), torch.tensor(dy, device="cuda"), counts=counts)
+    dy = rng.normal(0, 1, (B * tab.n_post, 4)).astype(np.float32)
+    on = lambda a: torch.tensor(a, device="cuda")
     rdz, rdw = orc.syn_bwd(tab, z, basis, dy, use_count=counts)
     _, _, dz_abs, dw_abs = dense.syn_bwd_f64(tab, z, basis, dy, use_count=counts)
-    assert np.max(np.abs(dz.cpu().numpy() - rdz) - 1e-5 * dz_abs) <= 1e-6
-    assert np.max(np.abs(dw.cpu().numpy() - rdw) - 1e-5 * dw_abs) <= 1e-6
+    for want_dz, want_dw in ((True, True), (True, False), (False, True)):   # together and alone
+        dz, dw = t.backward(on(z), on(dy), counts=counts, want_dz=want_dz, want_dw=want_dw)
+        if want_dz:
+            assert np.max(np.abs(dz.cpu().numpy() - rdz) - 1e-5 * dz_abs) <= 1e-6
+        if want_dw:
+            assert np.max(np.abs(dw.cpu().numpy() - rdw) - 1e-5 * dw_abs) <= 1e-6
     if not counts:
         return
     for infinite in (False, True):

@@ -18,12 +18,13 @@ constexpr int kMaxBasis = 8;
 constexpr int kMaxBatch = 32;
 constexpr uint32_t kLow24 = 0x00FFFFFFu;
 constexpr int kChunkEntries = 512;
-// work units of the op-level passes over columns: at most 64 consecutive columns and this many
-// synapses, or one chunk of this many synapses of a longer column.  Small units give a small table
-// enough waves (backward at batch 5, 1024 -> 256: 100,000 synapses 36 -> 16 us); a large one has
-// enough of the others, and fewer of them pass over its inactive columns faster (16.5M synapses,
-// batch 5: 201 us with 256 against 193)
-constexpr int dw_unit_entries(int64_t n_syn) { return n_syn < (4 << 20) ? 256 : 1024; }
+// Work units of the op-level passes over columns: at most 64 consecutive columns and so many
+// synapses, or one chunk of so many of a longer column.  The pass that sums dz and dW together wants waves:
+// backward calls with units of 256 / 512 / 1024: 3.9M synapses in 120,000 columns, batch 5, 57 / 73 / 87 us; 8.4M in
+// 8,000, batch 20, 103 / 103 / 125; 2.6M in 17,400, batch 20, 92 / 100 / 135 (1024 is the better one for dz alone over
+// long columns, kWideDzMinAvgLen).  The dW pass reads inactive columns' inputs only, 64 a wave: 7.8M in 120,000, batch 9,
+// 41 / 34 / 34 us, 16.5M in 330,000, batch 5, 50 / 43 / 41.
+constexpr int kUnitEntries = 256, kWideUnitEntries = 1024;
 constexpr int kChunkRows = 63;
 // grouped row-sliced backward order: kGsCols columns per lane group,
 // kGsSlices equal ranges of G rows, segments padded to kGsPad entries
@@ -100,6 +101,15 @@ struct SpikeRows {
 };
 int32_t spike_bin(int32_t n_post);
 
+// Work units over the column-grouped table: unit u is {first column, columns, first position, end
+// position}; a column that does not fit one has units of its own, n_chunked such columns {column, first unit, units, 0},
+// for the pass that adds their sums (most: the most units of one).
+struct Units {
+    int32_t n = 0, n_chunked = 0, most = 0;
+    int4 *unit = nullptr;         // [n]
+    int4 *chunked = nullptr;      // [n_chunked]
+};
+
 struct Table {
     int64_t n_syn = 0;
     int32_t n_post = 0;
@@ -136,14 +146,7 @@ struct Table {
     // kChunkEntries entries unless it is a single longer row
     int32_t n_chunks = 0;
     int4 *chunk_desc = nullptr;   // [n_chunks]
-    // work units of the op-level weight-gradient pass over the column-grouped table: unit u is
-    // {first column, columns, first position, end position} (dw_unit_entries)
-    int32_t n_dwu = 0;
-    int4 *dwu = nullptr;          // [n_dwu]
-    // columns whose units hold one column each (a column of more than dw_unit_entries synapses
-    // spreads over several): {column, first unit, units, 0}, for the chunked dz pass
-    int32_t n_dzc = 0;
-    int4 *dzc = nullptr;          // [n_dzc]
+    Units units, wide;            // of kUnitEntries and kWideUnitEntries synapses
     int32_t *ph_ptr = nullptr;    // [n_types * n_cols + 1]
     int32_t *ph_order = nullptr;  // [n_syn]       synapse id at position k
     uint2 *ph_pw = nullptr;       // [n_syn]       {post, weight bits}
@@ -271,7 +274,7 @@ inline int ceil_div(int64_t a, int64_t b) { return static_cast<int>((a + b - 1) 
 int batch_pad(int B);
 // The op's custom gradient (glif_syn_bwd) on a given G buffer of syn_g_floats(t, B) floats;
 // g_ready: G already holds this dy's rows in t's layout (built for a table with
-// same_g_layout), so only dz / dW are computed.  partial: n_dwu * batch_pad(B) floats for the
+// same_g_layout), so only dz / dW are computed.  partial: units.n * batch_pad(B) floats for the
 // unit dz pass of tables with few or long columns (nullptr: the walks only).
 size_t syn_g_floats(const Table *t, int32_t B);
 bool same_g_layout(const Table *a, const Table *b);

@@ -23,12 +23,17 @@ constexpr int32_t kUnitDzMinColLen = 2048;
 // one unit (its chunks then go to waves of their own).
 constexpr int64_t kPushUnitsMaxScanWaves = 2048;
 constexpr int32_t kPushUnitsMinColLen = 1024;
+constexpr int64_t kPushWideMinSyn = int64_t(4) << 20;   // and the wide units from here: enough waves of them
 // The backward takes the units too when the walk would run on fewer lanes than this -- unless G's rows
 // are a cache line or more (Bp >= 16) and the columns short: a lane group then waits for few rows, while
 // the split walk streams them (whole calls, units against walk, batch 20: 25 synapses a column 42 against
 // 25 us, 50: 37 against 26, 62: 53 against 47, 132: 37 against 46; batch 1 at 25: 10 against 16).
 constexpr int64_t kUnitDzMaxWalkLanes = 1024 * kWave;
 constexpr int64_t kUnitDzMinAvgLen = 96;
+// dz alone over long columns takes the wide units once they are enough waves (2.6M synapses in 17,400 columns, batch 1 / 5 /
+// 32: 34 / 54 / 86 us by small units, 29 / 41 / 83 by wide ones; with dW beside it 36 / 58 / 104 against 34 / 55 / 145; 1.8M
+// in 8,000, batch 32: 52 against 71).
+constexpr int64_t kWideDzMinAvgLen = 128, kWideDzMinSyn = int64_t(2) << 20;
 
 // ---------------------------------------------------------------- forward ----
 // Deterministic pull of Poisson-count inputs (the background form, models.py:917-931): thread
@@ -138,7 +143,7 @@ __device__ inline void push_spiking(int lane, int32_t lo, int32_t hi, uint32_t m
 // column's batch mask (z > 0, the test of tf.where at models.py:128-130), and all 64 lanes
 // push the wave's active columns one after another.  No column list, no count pass.
 // The event push over the table's work units (a run of up to 64 short columns, or a chunk of
-// at most dw_unit_entries synapses of a long column), a wave per unit: the lanes hold the
+// at most kUnitEntries synapses of a long column), a wave per unit: the lanes hold the
 // run's columns' batch masks, and all 64 lanes push each active column's share of the unit.
 // For tables whose column scan would run on few waves (few columns, or long ones).
 template <bool COUNTS, int Q>
@@ -324,7 +329,7 @@ struct SynDwArgs {
     int64_t n_cols;
     int32_t B, hm, lm, R, counts;  // G row of entry p: (p >> 24) * hm + (p & kLow24) * lm
     const float *z;  // [B][n_cols]
-    const int4 *units;  // the table's work units (Table::dwu), one wave each
+    const int4 *units;  // the table's work units (Table::wide), one wave each
     int32_t n_units;
     const int32_t *col_ptr;
     const uint32_t *ps;
@@ -416,7 +421,7 @@ __device__ inline void syn_dw_body(const SynDwArgs &a, int64_t bid) {
 // adds a column's units in order.  dW of a column with any input: its synapses' sum over the batch
 // entries of G[row][b] times the input value (counts) or 1, written once, straight to reference
 // order.  What bounds it is the gathers' latency (kUnitRows rows in flight per lane group, and
-// dw_unit_entries synapses a wave for enough waves).  Whole backward calls, against a lane per
+// kUnitEntries synapses a wave for enough waves).  Whole backward calls, against a lane per
 // synapse for dz, which held whole rows, and dW by a pass of its own, both over 1024-synapse
 // units: background table, 66,000 posts, batch 32, 174 -> 63 us; LGN table at batch 5, 94 -> 58.
 struct UnitArgs {
@@ -538,22 +543,28 @@ __global__ void __launch_bounds__(kBlock) k_syn_units(UnitArgs a) {
     }
 }
 
-// dz of the one-column units' columns: thread per (column, b), the column's units in order, four at
-// a time in pairs: their sums are the largest, and every rounding at that size counts.
+// dz of the one-column units' columns: 2^sh lanes per (column, b) take the column's units in turn, four at
+// a time in pairs (their sums are the largest, and every rounding at that size counts), and add theirs in
+// a fixed order.  One lane's chain of loads was the backward's longest part over long columns: 100 columns of
+// 40,000 synapses, batch 1, 54 -> 41 us a call with 32.
+constexpr int kChunkUnits = 8;   // units per lane
+
 __global__ void __launch_bounds__(kBlock)
-    k_dz_chunks(const int4 *__restrict__ dzc, int32_t n_dzc, const float *__restrict__ partial, int32_t B, int32_t R,
-                int64_t n_cols, float *__restrict__ dz) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= static_cast<int64_t>(n_dzc) * B) return;
-    const int4 d = dzc[i / B];
+    k_dz_chunks(const int4 *__restrict__ chunked, int32_t n_chunked, const float *__restrict__ partial, int32_t B,
+                int32_t R, int64_t n_cols, int sh, float *__restrict__ dz) {
+    const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> sh;
+    const int L = 1 << sh, l = threadIdx.x & (L - 1);
+    const bool own = i < static_cast<int64_t>(n_chunked) * B;
+    const int4 d = own ? chunked[i / B] : make_int4(0, 0, 0, 0);
     const int b = static_cast<int>(i % B);
-    const float *p = partial + static_cast<int64_t>(d.y) * R + b;
+    const int64_t step = static_cast<int64_t>(R) << sh;
+    const float *p = partial + static_cast<int64_t>(d.y + l) * R + b;
     float s = 0.0f;
-    int u = 0;
-    for (; u + 4 <= d.z; u += 4, p += 4 * static_cast<int64_t>(R))
-        s = s + ((p[0] + p[R]) + (p[2 * static_cast<int64_t>(R)] + p[3 * static_cast<int64_t>(R)]));
-    for (; u < d.z; ++u, p += R) s = s + p[0];
-    dz[static_cast<int64_t>(b) * n_cols + d.x] = s;
+    int u = l;
+    for (; u + 3 * L < d.z; u += 4 * L, p += 4 * step) s = s + ((p[0] + p[step]) + (p[2 * step] + p[3 * step]));
+    for (; u < d.z; u += L, p += step) s = s + p[0];
+    for (int o = 1; o < L; o <<= 1) s = s + __shfl_xor(s, o, kWave);
+    if (own && l == 0) dz[static_cast<int64_t>(b) * n_cols + d.x] = s;
 }
 
 // The grouped dz walk (the first walk_blocks workgroups) beside the weight-gradient pass of
@@ -583,7 +594,7 @@ struct SynWs {
     uint32_t *cm;      // [n_slots * pre_pad] batch masks (deterministic forward)
     uint64_t *cbits;   // [n_slots * pre_pad / 64] activity bitmaps
     float *G;          // the custom gradient's projection
-    float *partial;    // [n_dwu][padded B] the unit dz pass's one-column sums
+    float *partial;    // [units][padded B] the unit dz pass's one-column sums
 };
 
 // with_G: the backward's projection G too (the forward does not use it)
@@ -597,7 +608,7 @@ static SynWs carve_syn(void *ws, const Table *t, int32_t B, size_t *bytes, bool 
     const int rows = t->og.rows ? t->og.rows : t->n_types;
     if (with_G) {
         w.G = cv.take<float>(static_cast<size_t>(t->n_post) * rows * batch_pad(B));
-        w.partial = cv.take<float>(std::max<size_t>(static_cast<size_t>(t->n_dwu) * batch_pad(B), 1));
+        w.partial = cv.take<float>(std::max<size_t>(static_cast<size_t>(t->units.n) * batch_pad(B), 1));
     }
     if (bytes) *bytes = cv.off;
     return w;
@@ -684,10 +695,11 @@ static int syn_fwd(const Table *t, const float *z, int32_t B, int32_t counts, in
     int rc = launch_fill_u32(I, 0u, static_cast<size_t>(nI) * t->n_basis, s);
     if (rc) return rc;
     const int Q = t->basis_nnz < 2 * t->n_types ? 1 : t->n_basis <= 4 ? 4 : 8;   // lanes per synapse
-    if (t->n_dwu > 0 && (ceil_div(t->n_cols, kWave) < kPushUnitsMaxScanWaves || t->max_col_len > kPushUnitsMinColLen)) {
-        const dim3 grid(static_cast<unsigned>(ceil_div(t->n_dwu, kBlock / kWave)));
+    const Units &un = t->n_syn < kPushWideMinSyn ? t->units : t->wide;
+    if (un.n > 0 && (ceil_div(t->n_cols, kWave) < kPushUnitsMaxScanWaves || t->max_col_len > kPushUnitsMinColLen)) {
+        const dim3 grid(static_cast<unsigned>(ceil_div(un.n, kBlock / kWave)));
         auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, s, z, B, t->n_cols, t->dwu, t->n_dwu, t->col_ptr,
+            hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, s, z, B, t->n_cols, un.unit, un.n, t->col_ptr,
                                t->ps, t->w_col, t->basis, t->n_types, t->n_basis, t->n_post, I);
         };
         if (Q == 1) counts ? launch(k_syn_push_units<true, 1>) : launch(k_syn_push_units<false, 1>);
@@ -843,7 +855,7 @@ int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int3
     // pass always runs over them
     const int64_t walk_lanes = (grouped ? t->n_groups : t->n_cols) * (Bp / 4);
     const bool prefer_units =
-        t->n_dwu > 0 && (t->max_col_len > kUnitDzMinColLen ||
+        t->units.n > 0 && (t->max_col_len > kUnitDzMinColLen ||
                          (walk_lanes < kUnitDzMaxWalkLanes && (Bp <= 8 || t->n_syn >= kUnitDzMinAvgLen * t->n_cols)));
     const bool dz_units = dz && partial && prefer_units;
     const bool dw_units = dw && (grouped || prefer_units);
@@ -865,14 +877,19 @@ int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int3
                            t->n_types, t->n_basis, nullptr, rows, gP, G, g_blocks, dw, n_fill);
     }
     GLIF_HIP(hipGetLastError());
+    // (dW alone by the same kernel as beside dz: the same bits)
     if (dz_units || (dw && prefer_units)) {
-        const UnitArgs ua{t->n_cols, B, cmp ? 1 : t->n_post, cmp ? rows : 1, counts, z, t->dwu, t->n_dwu, t->col_ptr,
+        const bool wide = dz_units && !dw && t->n_syn >= std::max(kWideDzMinSyn, kWideDzMinAvgLen * t->n_cols);
+        const Units &un = wide ? t->wide : t->units;
+        const UnitArgs ua{t->n_cols, B, cmp ? 1 : t->n_post, cmp ? rows : 1, counts, z, un.unit, un.n, t->col_ptr,
                           cmp ? oc.ps : t->ps, t->w_col, t->order, G, dz_units ? dz : nullptr, partial, dw};
         launch_syn_units(ua, Bp, s);
         GLIF_HIP(hipGetLastError());
-        if (dz_units && t->n_dzc > 0) {
-            hipLaunchKernelGGL(k_dz_chunks, dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(t->n_dzc) * B, kBlock))),
-                               dim3(kBlock), 0, s, t->dzc, t->n_dzc, partial, B, Bp, t->n_cols, dz);
+        if (dz_units && un.n_chunked > 0) {
+            int sh = 0;
+            while (sh < 6 && kChunkUnits << sh < un.most) ++sh;
+            hipLaunchKernelGGL(k_dz_chunks, dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(un.n_chunked) * B << sh, kBlock))),
+                               dim3(kBlock), 0, s, un.chunked, un.n_chunked, partial, B, Bp, t->n_cols, sh, dz);
             GLIF_HIP(hipGetLastError());
         }
         // done; what is left is a dz that found no room for the partial sums
@@ -887,11 +904,11 @@ int syn_bwd_run(const Table *t, const float *z, const float *dy, int32_t B, int3
         GsArgs ga{t->n_cols, (t->n_cols + kGsCols - 1) / kGsCols, B, cmp ? oc.gs_seg : t->gs_seg,
                   cmp ? oc.gs_pw : t->gs_pw, G};
         ga.split = gs_split(ga.n_groups, Bp / 4);
-        SynDwArgs da{t->n_cols, B, cmp ? 1 : t->n_post, cmp ? rows : 1, Bp, counts, z, t->dwu, t->n_dwu,
+        SynDwArgs da{t->n_cols, B, cmp ? 1 : t->n_post, cmp ? rows : 1, Bp, counts, z, t->wide.unit, t->wide.n,
                      t->col_ptr, cmp ? oc.ps : t->ps, t->order, G, dw};
         const int LG = Bp / 4;
         const int walk_blocks = dz ? static_cast<int>(ceil_div(t->n_groups * LG << ga.split, kBlock)) : 0;
-        const int dw_blocks = dw ? static_cast<int>(ceil_div(t->n_dwu, kBlock / kWave)) : 0;
+        const int dw_blocks = dw ? static_cast<int>(ceil_div(t->wide.n, kBlock / kWave)) : 0;
         const dim3 grid(walk_blocks + dw_blocks);
         if (grid.x == 0) return GLIF_OK;   // no columns
         auto launch = [&](auto whole, auto split) {

@@ -180,6 +180,37 @@ static bool build_gs(int64_t n, int64_t n_cols, int64_t n_rows, const int64_t *r
     return true;
 }
 
+// Work units of at most `most` synapses: runs of short columns, chunks of long ones.
+static int build_units(int64_t n_cols, const int32_t *col_ptr, int most, Units &out) {
+    std::vector<int4> units, chunked;
+    for (int64_t c = 0; c < n_cols;) {
+        const int32_t k0 = col_ptr[c], k1 = col_ptr[c + 1];
+        if (k1 - k0 > most) {
+            for (int32_t k = k0; k < k1; k += most)
+                units.push_back(make_int4(static_cast<int>(c), 1, k, std::min(k + most, k1)));
+            ++c;
+            continue;
+        }
+        int64_t m = c + 1;
+        while (m < n_cols && m - c < kWave && col_ptr[m + 1] - k0 <= most) ++m;
+        units.push_back(make_int4(static_cast<int>(c), static_cast<int>(m - c), k0, col_ptr[m]));
+        c = m;
+    }
+    out.n = static_cast<int32_t>(units.size());
+    // every one-column unit's column, a short one that is alone in its unit among them
+    for (int32_t u = 0; u < out.n;) {
+        if (units[u].y != 1) { ++u; continue; }
+        int32_t v = u + 1;
+        while (v < out.n && units[v].y == 1 && units[v].x == units[u].x) ++v;
+        chunked.push_back(make_int4(units[u].x, u, v - u, 0));
+        out.most = std::max(out.most, v - u);
+        u = v;
+    }
+    out.n_chunked = static_cast<int32_t>(chunked.size());
+    int rc = upload(&out.unit, units.data(), units.size());
+    return rc ? rc : upload(&out.chunked, chunked.data(), chunked.size());
+}
+
 static void free_plan(PermPlan &pp) {
     void *ptrs[] = {pp.runs, pp.off1, pp.off2, pp.mid};
     for (void *p : ptrs)
@@ -243,7 +274,7 @@ static void free_table(Table *t) {
     free_plan(t->pinv);
     void *ptrs[] = {t->basis, t->col_ptr, t->order, t->ps, t->w_col, t->row_ptr, t->perm,
                     t->pd, t->sid_row, t->w_row, t->ph_ptr, t->ph_order, t->ph_pw, t->ell_pw, t->ell_src,
-                    t->chunk_desc, t->dwu, t->dzc, t->pidx, t->order_inv, t->ph_inv, t->ph_src, t->gs_seg, t->gs_pw, t->gs_src,
+                    t->chunk_desc, t->units.unit, t->units.chunked, t->wide.unit, t->wide.chunked, t->pidx, t->order_inv, t->ph_inv, t->ph_src, t->gs_seg, t->gs_pw, t->gs_src,
                     t->cg.ps, t->cg.ph_pw, t->cg.gs_seg, t->cg.gs_pw, t->cg.gs_src, t->cg.gtype,
                     t->og.ps, t->og.ph_pw, t->og.gs_seg, t->og.gs_pw, t->og.gs_src, t->og.gtype,
                     t->spk.off, t->spk.ent, t->spk.src};
@@ -631,32 +662,6 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
         n = m;
     }
     t->n_chunks = static_cast<int32_t>(chunk_desc.size());
-    // weight-gradient work units: runs of short columns, chunks of long ones
-    std::vector<int4> dwu;
-    const int unit = dw_unit_entries(n_syn);
-    for (int64_t c = 0; c < n_cols;) {
-        const int32_t k0 = col_ptr[c], k1 = col_ptr[c + 1];
-        if (k1 - k0 > unit) {
-            for (int32_t k = k0; k < k1; k += unit)
-                dwu.push_back(make_int4(static_cast<int>(c), 1, k, std::min(k + unit, k1)));
-            ++c;
-            continue;
-        }
-        int64_t m = c + 1;
-        while (m < n_cols && m - c < kWave && col_ptr[m + 1] - k0 <= unit) ++m;
-        dwu.push_back(make_int4(static_cast<int>(c), static_cast<int>(m - c), k0, col_ptr[m]));
-        c = m;
-    }
-    t->n_dwu = static_cast<int32_t>(dwu.size());
-    std::vector<int4> dzc;
-    for (int32_t u = 0; u < t->n_dwu;) {
-        if (dwu[u].y != 1) { ++u; continue; }
-        int32_t v = u + 1;
-        while (v < t->n_dwu && dwu[v].y == 1 && dwu[v].x == dwu[u].x) ++v;
-        dzc.push_back(make_int4(dwu[u].x, u, v - u, 0));
-        u = v;
-    }
-    t->n_dzc = static_cast<int32_t>(dzc.size());
     t->basis_host = new float[static_cast<size_t>(n_types) * n_basis];
     std::memcpy(t->basis_host, basis, sizeof(float) * n_types * n_basis);
     for (int i = 0; i < n_types * n_basis; ++i) t->basis_nnz += basis[i] != 0.0f;
@@ -667,8 +672,8 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
         (rc = upload(&t->ps, ps.data(), ps.size())) ||
         (rc = upload(&t->row_ptr, row_ptr.data(), row_ptr.size())) ||
         (rc = upload(&t->chunk_desc, chunk_desc.data(), chunk_desc.size())) ||
-        (rc = upload(&t->dwu, dwu.data(), dwu.size())) ||
-        (rc = upload(&t->dzc, dzc.data(), dzc.size())) ||
+        (rc = build_units(n_cols, col_ptr.data(), kUnitEntries, t->units)) ||
+        (rc = build_units(n_cols, col_ptr.data(), kWideUnitEntries, t->wide)) ||
         (rc = upload(&t->perm, perm.data(), perm.size())) ||
         (rc = upload(&t->pd, pd.data(), pd.size())) ||
         (with_pidx && (rc = upload(&t->pidx, pidx.data(), pidx.size()))) ||
