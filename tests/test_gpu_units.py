@@ -25,13 +25,15 @@ LENGTHS = {
     # columns of many units, whose sums several lanes add
     "tall": [20000, 300, 0, 12345, 1],
 }
-POSTS = {"tall": 20000}
+# rows that pad well: the counts pull, one and two, four, eight batch entries a lane by the number of posts
+POSTS = {"tall": 20000, "even 5000": 5000, "even 33000": 33000}
 
 
 def _table(kind, rng):
-    if kind == "even":   # 10 of 100 inputs each, the last posts fewer: rows that pad well
+    if kind.startswith("even"):   # 10 of 100 inputs each, the last posts fewer
+        n = POSTS.get(kind, N)
         pairs = [np.stack([np.full(k, p), np.sort(rng.permutation(100)[:k])], -1)
-                 for p in range(N) for k in [10 if p < N - 3 else N - p]]
+                 for p in range(n) for k in [10 if p < n - 3 else n - p]]
         ind, n_cols = np.concatenate(pairs), 100
     else:
         cols = [np.stack([rng.permutation(POSTS.get(kind, N))[:k], np.full(k, c)], -1) for c, k in enumerate(LENGTHS[kind])]
@@ -43,7 +45,7 @@ def _table(kind, rng):
 
 
 @pytest.mark.parametrize("counts", [False, True])
-@pytest.mark.parametrize("kind", ["long", "short", "middle", "even", "tall"])
+@pytest.mark.parametrize("kind", ["long", "short", "middle", "even", "even 5000", "even 33000", "tall"])
 @pytest.mark.parametrize("B", [1, 4, 5, 9, 16, 17, 32])
 def test_units(B, kind, counts):
     from v1_glif_model_amd.ops import SynapseTable
@@ -75,7 +77,7 @@ def test_units(B, kind, counts):
             ref = orc.syn_fwd(tab, z, basis, use_count=True)
         got = t.forward(torch.tensor(z, device="cuda"), counts=True, mode="deterministic").cpu().numpy()
         np.testing.assert_array_equal(got, ref)
-        if kind == "even":   # pulled in event mode too
+        if kind.startswith("even"):   # pulled in event mode too
             ev = t.forward(torch.tensor(z, device="cuda"), counts=True, mode="event").cpu().numpy()
             np.testing.assert_array_equal(ev, ref)
 

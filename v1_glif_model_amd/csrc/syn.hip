@@ -69,33 +69,36 @@ __global__ void __launch_bounds__(kBlock)
     for (int r = 0; r < nb; ++r) dst[r] = acc[r];
 }
 
-// The same over an input table's ELL copy: a thread per post and NBATCH batch entries, so an entry
+// The same over an input table's ELL copy: a thread per post and BB batch entries, so an entry
 // (one coalesced load) is read once for all of them; the inputs' counts [input][batch entry] in LDS.
 // Each (post, batch entry) adds its row's active entries in row order, as k_syn_pull_dense does.
-// Background table (66,000 posts, 10 synapses each, 100 inputs), batch 32: 98 -> 28 us.
-constexpr int kEllBatch = 8;
-constexpr int64_t kEllMaxInputs = 1024;   // their counts for kEllBatch batch entries: 32 KB
+// Bound by instruction issue, BB batch entries a synapse: background table (66,000 posts, 10 synapses each, 100
+// inputs), batch 32: 98 -> 28 us with BB = 8; 3,000 posts with 150 each, batch 1, BB = 8 59 us, 1 16.
+constexpr int64_t kEllMaxInputs = 1024;
+constexpr int64_t kEllMaxStage = 2048;    // counts that a workgroup stages for its 256 posts
+constexpr int32_t kEllEventMaxRow = 48;   // the longest rows pulled in event mode
+constexpr int64_t kEllMinLanes = 32768;   // posts x groups of BB batch entries: fewer leave CUs idle
 
+template <int BB>
 __global__ void __launch_bounds__(kBlock)
     k_syn_pull_ell(const float *__restrict__ z, int32_t B, int32_t n_cols, int32_t n_post,
                    const int32_t *__restrict__ row_ptr, const uint2 *__restrict__ ell,
                    const float *__restrict__ basis, int n_types, int nb, float *__restrict__ I) {
-    extern __shared__ __align__(16) float ell_lds[];
-    float4 *zl = reinterpret_cast<float4 *>(ell_lds);   // [n_cols][kEllBatch]
-    float *basis_lds = ell_lds + static_cast<size_t>(n_cols) * kEllBatch;
-    const int b0 = static_cast<int>(blockIdx.y) * kEllBatch;
-    for (int i = threadIdx.x; i < n_cols * kEllBatch; i += blockDim.x) {
+    extern __shared__ __align__(16) float ell_lds[];   // [n_cols][BB]
+    float *basis_lds = ell_lds + static_cast<size_t>(n_cols) * BB;
+    const int b0 = static_cast<int>(blockIdx.y) * BB;
+    for (int i = threadIdx.x; i < n_cols * BB; i += blockDim.x) {
         const int bb = i / n_cols, c = i - bb * n_cols;
         const float x = b0 + bb < B ? z[static_cast<int64_t>(b0 + bb) * n_cols + c] : 0.0f;
-        ell_lds[c * kEllBatch + bb] = x > 0.0f ? x : 0.0f;
+        ell_lds[c * BB + bb] = x > 0.0f ? x : 0.0f;
     }
     load_basis_lds(basis_lds, basis, n_types * nb);
     const int64_t n = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (n >= n_post) return;
     const int32_t len = row_ptr[n + 1] - row_ptr[n];   // without the padding, which an infinite count would turn to NaN
-    float acc[kEllBatch][kMaxBasis];
+    float acc[BB][kMaxBasis];
 #pragma unroll
-    for (int bb = 0; bb < kEllBatch; ++bb)
+    for (int bb = 0; bb < BB; ++bb)
 #pragma unroll
         for (int r = 0; r < kMaxBasis; ++r) acc[bb][r] = 0.0f;
     for (int32_t j0 = 0; j0 < len; j0 += 4) {
@@ -107,20 +110,21 @@ __global__ void __launch_bounds__(kBlock)
             if (j0 + u >= len) break;
             const float w = __uint_as_float(e[u].y);
             const float *bs = basis_lds + (e[u].x >> 24) * nb;
-            const float4 a = zl[(e[u].x & kLow24) * 2], c = zl[(e[u].x & kLow24) * 2 + 1];
-            const float x[kEllBatch] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+            float x[BB];
+#pragma unroll
+            for (int bb = 0; bb < BB; ++bb) x[bb] = ell_lds[(e[u].x & kLow24) * BB + bb];
 #pragma unroll
             for (int r = 0; r < kMaxBasis; ++r) {
                 if (r >= nb) break;
                 const float s = bs[r];
 #pragma unroll
-                for (int bb = 0; bb < kEllBatch; ++bb)
+                for (int bb = 0; bb < BB; ++bb)
                     acc[bb][r] = x[bb] > 0.0f ? acc[bb][r] + (w * x[bb]) * s : acc[bb][r];
             }
         }
     }
 #pragma unroll
-    for (int bb = 0; bb < kEllBatch; ++bb) {
+    for (int bb = 0; bb < BB; ++bb) {
         if (b0 + bb >= B) break;
         float *dst = I + (static_cast<int64_t>(b0 + bb) * n_post + n) * nb;
 #pragma unroll
@@ -620,11 +624,14 @@ static SynWs carve_syn(void *ws, const Table *t, int32_t B, size_t *bytes, bool 
 // call, 67 against 24 us pulled at B = 5), and whether that pull uses the workspace (batch
 // masks and activity bits built from z; Poisson counts take the dense-row pull, which needs
 // none).  glif_syn_fwd validates the workspace with the same predicate syn_fwd dispatches on.
-// Poisson counts of a few inputs pull in event mode whatever the columns' length: a fifth of them is
-// active in every batch entry (12,007 posts, 100 inputs, batch 32: 157 us pushed, 12 pulled).
+// Poisson counts of a few inputs onto short rows pull in event mode whatever the columns' length: as background a fifth of
+// them is active in every batch entry (12,007 posts, 100 inputs, batch 32: 157 us pushed, 12 pulled), and with next to none
+// a short row costs no more than the push (3,000 posts, batch 5, 40 synapses each: 15 us, pushed 14 with 0.2 % active, 42 with
+// 10 %; 150 each: 38 us, pushed 18 and 95).
 static bool ell_counts(const Table *t) { return t->ell_len > 0 && t->n_cols <= kEllMaxInputs; }
 static bool fwd_pulls(const Table *t, int32_t counts, int32_t mode) {
-    return mode == GLIF_MODE_DETERMINISTIC || t->max_col_len > kUnitDzMinColLen || (counts && ell_counts(t));
+    return mode == GLIF_MODE_DETERMINISTIC || t->max_col_len > kUnitDzMinColLen || 
+           (counts && ell_counts(t) && t->ell_len <= kEllEventMaxRow);
 }
 static bool fwd_uses_ws(const Table *t, int32_t counts, int32_t mode) { return fwd_pulls(t, counts, mode) && !counts; }
 
@@ -678,10 +685,18 @@ static int syn_fwd(const Table *t, const float *z, int32_t B, int32_t counts, in
             return GLIF_OK;
         }
         if (ell_counts(t)) {
-            const size_t l = sizeof(float) * static_cast<size_t>(t->n_cols) * kEllBatch + lds;
-            hipLaunchKernelGGL(k_syn_pull_ell, dim3(ceil_div(t->n_post, kBlock), ceil_div(B, kEllBatch)), dim3(kBlock), l,
-                               s, z, B, static_cast<int32_t>(t->n_cols), t->n_post, t->row_ptr, t->ell_pw, t->basis,
-                               t->n_types, t->n_basis, I);
+            int bb = 8;
+            while (bb > 1 && (bb >= 2 * B || bb * t->n_cols > kEllMaxStage || t->n_post * static_cast<int64_t>(ceil_div(B, bb)) < kEllMinLanes)) bb /= 2;
+            const size_t l = sizeof(float) * static_cast<size_t>(t->n_cols) * bb + lds;
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(ceil_div(t->n_post, kBlock), ceil_div(B, bb)), dim3(kBlock), l, s, z, B,
+                                   static_cast<int32_t>(t->n_cols), t->n_post, t->row_ptr, t->ell_pw, t->basis, t->n_types,
+                                   t->n_basis, I);
+            };
+            if (bb == 8) launch(k_syn_pull_ell<8>);
+            else if (bb == 4) launch(k_syn_pull_ell<4>);
+            else if (bb == 2) launch(k_syn_pull_ell<2>);
+            else launch(k_syn_pull_ell<1>);
             GLIF_HIP(hipGetLastError());
             return GLIF_OK;
         }
