@@ -2,7 +2,8 @@
 
 * the spike-major rows of the window forward (12 bytes per synapse and their offsets) come with the
   cell that reads them, for its recurrent and LGN tables, not with a table;
-* they carry the weights that the tables held before the cell was made."""
+* they carry the weights that the tables held before the cell was made, and later ones, gathered at once
+  (small tables) or in two passes (over a million synapses)."""
 import dataclasses
 
 import numpy as np
@@ -11,6 +12,7 @@ import torch
 
 from oracle.cpu import OracleCell
 from tests.helpers import tiny_config
+from tests.test_gpu_params import _state_dev
 from v1_glif_model_amd import synthetic as sy
 from v1_glif_model_amd.tables import build_cell_tables
 
@@ -45,6 +47,19 @@ def test_spike_rows_come_with_the_cell(monkeypatch):
     n = cell.rec_table.n_syn + cell.lgn_table.n_syn
     print(n, made, flush=True)
     assert made["cell"] >= 12 * n   # 2.4 million synapses: 29 MB, of 2 MB pages
+    tb = build_cell_tables(net)
+    lgn, bkg = sy.make_inputs(cfg, seed=3, seq_len=7, batch=2)
+    oc = OracleCell(tb, gauss_std=0.5, damp=0.5, rd=0.5, vgd=0.5, pseudo_gauss=True)
+    first = oc.zero_state(2)
+    first["zbuf"] = (np.random.default_rng(4).random(first["zbuf"].shape) < 0.02).astype(np.float32)
+    for scale in (1.0, 3.0):   # the second weights reach the rows too
+        with torch.no_grad():
+            cell.recurrent_weight_values.copy_(torch.tensor(tb.rec.weight * np.float32(scale)))
+        other = dataclasses.replace(tb, rec=dataclasses.replace(tb.rec, weight=tb.rec.weight * np.float32(scale)))
+        _, ov, _, ost = OracleCell(other, gauss_std=0.5, damp=0.5, rd=0.5, vgd=0.5, pseudo_gauss=True).forward(lgn, bkg, state=first)
+        _, v, st = cell.rollout(lgn, bkg, state=_state_dev(cell, first), mode="deterministic")
+        np.testing.assert_array_equal(v.cpu().numpy().view(np.uint32), ov.view(np.uint32))
+        np.testing.assert_array_equal(st[4].cpu().numpy(), ost["psc_rise"])
 
 
 def test_spike_rows_take_the_weights_already_set(monkeypatch):

@@ -98,6 +98,7 @@ struct SpikeRows {
     int32_t *off = nullptr;     // [ranges * rows + 1] first entry of (range, row)
     uint2 *ent = nullptr;       // [n_syn] {post & 0xFFFF | (delay - 1) % kSpkDelays << 16 | syn_id << 24, weight bits}
     int32_t *src = nullptr;     // [n_syn] column-grouped position of the synapse
+    PermPlan plan;              // of the weights (P = src), where the table has such plans
 };
 int32_t spike_bin(int32_t n_post);
 
@@ -132,7 +133,7 @@ struct Table {
     uint32_t *pidx = nullptr;     // [n_syn]       (n_slots - delay) * round64(n_pre) + pre, or null
     uint8_t *sid_row = nullptr;   // [n_syn]
     float *w_row = nullptr;       // [n_syn]
-    // type-phased (backward): ordered by (syn_id, column, synapse id); the type-s
+    // type-phased (backward, tables without the grouped order; else nullptr): ordered by (syn_id, column, synapse id); the type-s
     // synapses of column c are k in [ph_ptr[s * n_cols + c], ph_ptr[s * n_cols + c + 1])
     // ELL copy of the post-grouped table for single-delay (input) tables whose rows
     // pad to at most twice the synapse count: entry j of post n at j * n_post + n,

@@ -53,12 +53,12 @@ __global__ void __launch_bounds__(kBlock)
 // (blockIdx % 8); XCD x takes the x-th eighth of the destinations, so each superblock's
 // staging is read through one L2.
 __global__ void __launch_bounds__(kBlock)
-    k_perm_local(const float *__restrict__ mid, float *__restrict__ dst, const uint16_t *__restrict__ off2,
+    k_perm_local(const float *__restrict__ mid, float *__restrict__ dst, int stride, const uint16_t *__restrict__ off2,
                  int64_t n) {
     const int64_t per = gridDim.x / 8;
     const int64_t lb = static_cast<int64_t>(blockIdx.x % 8) * per + blockIdx.x / 8;
     const int64_t k = lb * blockDim.x + threadIdx.x;
-    if (k < n) dst[k] = mid[((k >> kPermShift) << kPermShift) + off2[k]];
+    if (k < n) dst[k * stride] = mid[((k >> kPermShift) << kPermShift) + off2[k]];
 }
 
 __global__ void k_gather_pair_w(uint2 *__restrict__ dst, const float *__restrict__ src,
@@ -96,17 +96,21 @@ int launch_gather_f32(float *dst, const float *src, const int32_t *idx, int64_t 
     return GLIF_OK;
 }
 
-int launch_perm_gather(float *dst, const float *src, const int32_t *idx, const PermPlan &plan, int64_t n,
-                       float *mid, hipStream_t s) {
-    if (!plan.runs) return launch_gather_f32(dst, src, idx, n, s);
+// dst[k * stride] = src[P[k]] through the two passes
+static int launch_perm(float *dst, int stride, const float *src, const PermPlan &plan, int64_t n, float *mid, hipStream_t s) {
     if (!mid) return fail(GLIF_EINVAL, "permutation plan without a staging buffer");
     hipLaunchKernelGGL(k_perm_runs, dim3(plan.n_runs), dim3(kBlock), 0, s, src, mid, plan.runs, plan.off1);
     GLIF_HIP(hipGetLastError());
     const int64_t blocks = 8 * ((n + 8 * kBlock - 1) / (8 * kBlock));
-    hipLaunchKernelGGL(k_perm_local, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, mid, dst, plan.off2,
-                       n);
+    hipLaunchKernelGGL(k_perm_local, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, mid, dst, stride,
+                       plan.off2, n);
     GLIF_HIP(hipGetLastError());
     return GLIF_OK;
+}
+
+int launch_perm_gather(float *dst, const float *src, const int32_t *idx, const PermPlan &plan, int64_t n,
+                       float *mid, hipStream_t s) {
+    return plan.runs ? launch_perm(dst, 1, src, plan, n, mid, s) : launch_gather_f32(dst, src, idx, n, s);
 }
 
 // ------------------------------------------------------------ host builds ----
@@ -272,6 +276,7 @@ static void free_table(Table *t) {
     if (!t) return;
     free_plan(t->pcol);
     free_plan(t->pinv);
+    free_plan(t->spk.plan);
     void *ptrs[] = {t->basis, t->col_ptr, t->order, t->ps, t->w_col, t->row_ptr, t->perm,
                     t->pd, t->sid_row, t->w_row, t->ph_ptr, t->ph_order, t->ph_pw, t->ell_pw, t->ell_src,
                     t->chunk_desc, t->units.unit, t->units.chunked, t->wide.unit, t->wide.chunked, t->pidx, t->order_inv, t->ph_inv, t->ph_src, t->gs_seg, t->gs_pw, t->gs_src,
@@ -295,7 +300,7 @@ static int download(std::vector<T> &dst, const T *src, size_t n) {
 
 // Compact rows from host arrays over the column-grouped positions k: col_ptr [n_cols + 1],
 // ps[k] = post | syn_id << 24, ph_src [n_syn] (column-grouped position of each type-phased
-// position) and rank[k] < rows.  Uploads ps / ph_pw / the grouped order into out (weights
+// position, or nullptr) and rank[k] < rows.  Uploads ps / ph_pw / the grouped order into out (weights
 // +0: the caller gathers them from w_col) and keeps a host copy of the ranks.
 static int build_compact(const Table *t, const int32_t *col_ptr, const uint32_t *ps, const int32_t *ph_src,
                          const uint8_t *rank, int32_t rows, CompactRows &out) {
@@ -311,15 +316,15 @@ static int build_compact(const Table *t, const int32_t *col_ptr, const uint32_t 
         cps[k] = post | static_cast<uint32_t>(rank[k]) << 24;
         src[k] = static_cast<int32_t>(k);
     }
-    std::vector<uint2> cph_pw(n);
-    for (int64_t k = 0; k < n; ++k) cph_pw[k] = make_uint2(static_cast<uint32_t>(row[ph_src[k]]), 0u);
+    std::vector<uint2> cph_pw(ph_src ? n : 0);
+    for (size_t k = 0; k < cph_pw.size(); ++k) cph_pw[k] = make_uint2(static_cast<uint32_t>(row[ph_src[k]]), 0u);
     std::vector<int32_t> gs_seg, gs_src;
     std::vector<uint2> gs_pw;
     int64_t n_groups = 0, n_gs = 0;
     build_gs(n, t->n_cols, static_cast<int64_t>(t->n_post) * rows, row.data(), col.data(), src.data(), n_groups,
              n_gs, gs_seg, gs_pw, gs_src);
     int rc;
-    if ((rc = upload(&out.ps, cps.data(), cps.size())) || (rc = upload(&out.ph_pw, cph_pw.data(), cph_pw.size())) ||
+    if ((rc = upload(&out.ps, cps.data(), cps.size())) || (ph_src && (rc = upload(&out.ph_pw, cph_pw.data(), cph_pw.size()))) ||
         (n_gs && (rc = upload(&out.gs_seg, gs_seg.data(), gs_seg.size()))) ||
         (n_gs && (rc = upload(&out.gs_pw, gs_pw.data(), gs_pw.size()))) ||
         (n_gs && (rc = upload(&out.gs_src, gs_src.data(), gs_src.size()))))
@@ -333,7 +338,7 @@ static int build_compact(const Table *t, const int32_t *col_ptr, const uint32_t 
 
 // the weights of a table's compact copies, gathered from w_col
 static int gather_compact_weights(const Table *t, const CompactRows &c, hipStream_t s) {
-    if (c.rows && t->n_syn) {
+    if (c.rows && c.ph_pw && t->n_syn) {
         hipLaunchKernelGGL(k_gather_pair_w, dim3(grid_for(t->n_syn)), dim3(kBlock), 0, s, c.ph_pw, t->w_col,
                            t->ph_src, t->n_syn);
         GLIF_HIP(hipGetLastError());
@@ -367,9 +372,9 @@ int table_set_g_rows(Table *t, const uint8_t *rank, int32_t g_rows) {
     int rc;
     GLIF_HIP(hipDeviceSynchronize());  // weights set on any stream have landed in w_col
     if ((rc = download(col_ptr, t->col_ptr, static_cast<size_t>(t->n_cols) + 1)) ||
-        (rc = download(ps, t->ps, n)) || (rc = download(ph_src, t->ph_src, n)))
+        (rc = download(ps, t->ps, n)) || (t->ph_src && (rc = download(ph_src, t->ph_src, n))))
         return rc;
-    if ((rc = build_compact(t, col_ptr.data(), ps.data(), ph_src.data(), rank, g_rows, t->cg))) return rc;
+    if ((rc = build_compact(t, col_ptr.data(), ps.data(), t->ph_src ? ph_src.data() : nullptr, rank, g_rows, t->cg))) return rc;
     // the weights the table already holds (later ones arrive through glif_table_set_weights)
     if ((rc = gather_compact_weights(t, t->cg, nullptr))) return rc;
     GLIF_HIP(hipDeviceSynchronize());
@@ -464,6 +469,8 @@ static int build_spike_rows(const Table *t, const int32_t *col_ptr, const uint32
     if ((rc = upload(&out.off, off.data(), off.size())) || (rc = upload(&out.ent, ent.data(), ent.size())) ||
         (rc = upload(&out.src, src.data(), src.size())))
         return rc;
+    // the weights through the table's own staging buffer
+    if (t->pcol.runs && (rc = build_perm_plan(&out.plan, src.data(), t->n_syn, false))) return rc;
     out.bin = bin;
     out.rows = static_cast<int32_t>(rows);
     return GLIF_OK;
@@ -472,6 +479,8 @@ static int build_spike_rows(const Table *t, const int32_t *col_ptr, const uint32
 // the weights of a table's spike-major rows, gathered from w_col
 static int gather_spike_weights(const Table *t, hipStream_t s) {
     if (!t->spk.rows) return GLIF_OK;
+    if (t->spk.plan.runs)
+        return launch_perm(reinterpret_cast<float *>(t->spk.ent) + 1, 2, t->w_col, t->spk.plan, t->n_syn, t->pcol.mid, s);
     hipLaunchKernelGGL(k_gather_pair_w, dim3(grid_for(t->n_syn)), dim3(kBlock), 0, s, t->spk.ent, t->w_col,
                        t->spk.src, t->n_syn);
     GLIF_HIP(hipGetLastError());
@@ -490,6 +499,7 @@ int table_set_spike_rows(Table *t) {
         (rc = build_spike_rows(t, col_ptr.data(), ps.data(), rows))) {
         for (void *p : {static_cast<void *>(rows.off), static_cast<void *>(rows.ent), static_cast<void *>(rows.src)})
             if (p) (void)hipFree(p);
+        free_plan(rows.plan);
         return rc;
     }
     t->spk = rows;
@@ -562,31 +572,10 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
     std::vector<int32_t> row_ptr(static_cast<size_t>(n_post) + 1), perm(n_syn);
     counting_sort(post, order.data(), n_syn, n_post, row_ptr.data(), perm.data());
 
-    // type-phased order for the backward: (syn_id, column, synapse id), by a stable
-    // counting sort of the column-grouped order by syn_id * n_cols + column
-    const int64_t n_ph = static_cast<int64_t>(n_types) * n_cols;
-    if (n_ph >= INT32_MAX) return fail(GLIF_EINVAL, "n_types * n_cols must be < 2^31");
-    std::vector<int64_t> ph_key(n_syn);
-    for (int64_t i = 0; i < n_syn; ++i) ph_key[i] = static_cast<int64_t>(syn_id[i]) * n_cols + col[i];
-    std::vector<int32_t> ph_ptr(n_ph + 1), ph_order(n_syn);
-    counting_sort(ph_key.data(), order.data(), n_syn, n_ph, ph_ptr.data(), ph_order.data());
-    std::vector<uint2> ph_pw(n_syn);
-    for (int64_t k = 0; k < n_syn; ++k) {
-        ph_pw[k].x = static_cast<uint32_t>(post[ph_order[k]]);
-        ph_pw[k].y = 0u;  // the weight, written by glif_table_set_weights
-    }
-
-    // inverse permutations: position of synapse s in the column-grouped and type-phased
-    // orders (gradients go back to reference order with coalesced writes)
-    std::vector<int32_t> order_inv(n_syn), ph_inv(n_syn), ph_src(n_syn);
-    for (int64_t k = 0; k < n_syn; ++k) {
-        order_inv[order[k]] = static_cast<int32_t>(k);
-        ph_inv[ph_order[k]] = static_cast<int32_t>(k);
-    }
-    // the weight copies other than w_col are gathered from w_col, whose order is close to
-    // theirs (the type-phased order sweeps it once per type; a group's grouped entries come
-    // from its own columns), rather than from the reference order
-    for (int64_t k = 0; k < n_syn; ++k) ph_src[k] = order_inv[ph_order[k]];
+    // inverse permutation: position of synapse s in the column-grouped order (gradients go back to reference order
+    // with coalesced writes)
+    std::vector<int32_t> order_inv(n_syn);
+    for (int64_t k = 0; k < n_syn; ++k) order_inv[order[k]] = static_cast<int32_t>(k);
     // grouped row-sliced order (backward dz walks) over the type-major rows
     std::vector<int32_t> gs_seg, gs_src;
     std::vector<uint2> gs_pw;
@@ -596,6 +585,31 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
         for (int64_t i = 0; i < n_syn; ++i) row[i] = static_cast<int64_t>(syn_id[i]) * n_post + post[i];
         build_gs(n_syn, n_cols, static_cast<int64_t>(n_types) * n_post, row.data(), col, order_inv.data(), n_groups,
                  n_gs, gs_seg, gs_pw, gs_src);
+    }
+
+    // type-phased order, for the backward of tables that have no grouped order: (syn_id, column, synapse id),
+    // by a stable counting sort of the column-grouped order by syn_id * n_cols + column.  (Compact rows' grouped order has
+    // other segments: the bound is on any rows'.)
+    const int64_t n_ph = static_cast<int64_t>(n_types) * n_cols;
+    if (n_ph >= INT32_MAX) return fail(GLIF_EINVAL, "n_types * n_cols must be < 2^31");
+    const bool phased = n_gs == 0 || n_syn + (kGsPad - 1) * static_cast<int64_t>(kGsSlices) * n_groups >= INT32_MAX;
+    std::vector<int32_t> ph_ptr, ph_order, ph_inv, ph_src;
+    std::vector<uint2> ph_pw;
+    if (phased) {
+        std::vector<int64_t> ph_key(n_syn);
+        for (int64_t i = 0; i < n_syn; ++i) ph_key[i] = static_cast<int64_t>(syn_id[i]) * n_cols + col[i];
+        ph_ptr.resize(n_ph + 1);
+        ph_order.resize(n_syn);
+        ph_inv.resize(n_syn);
+        ph_src.resize(n_syn);
+        ph_pw.resize(n_syn);
+        counting_sort(ph_key.data(), order.data(), n_syn, n_ph, ph_ptr.data(), ph_order.data());
+        for (int64_t k = 0; k < n_syn; ++k) {
+            // (the weight: glif_table_set_weights)
+            ph_pw[k] = make_uint2(static_cast<uint32_t>(post[ph_order[k]]), 0u);
+            ph_inv[ph_order[k]] = static_cast<int32_t>(k);
+            ph_src[k] = order_inv[ph_order[k]];
+        }
     }
 
     std::vector<uint32_t> ps(n_syn), pd(n_syn + kPdPad, 0u);
@@ -678,12 +692,12 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
         (rc = upload(&t->pd, pd.data(), pd.size())) ||
         (with_pidx && (rc = upload(&t->pidx, pidx.data(), pidx.size()))) ||
         (rc = upload(&t->sid_row, sid_row.data(), sid_row.size())) ||
-        (rc = upload(&t->ph_ptr, ph_ptr.data(), ph_ptr.size())) ||
-        (rc = upload(&t->ph_order, ph_order.data(), ph_order.size())) ||
+        (phased && (rc = upload(&t->ph_ptr, ph_ptr.data(), ph_ptr.size()))) ||
+        (phased && (rc = upload(&t->ph_order, ph_order.data(), ph_order.size()))) ||
         (rc = upload(&t->order_inv, order_inv.data(), order_inv.size())) ||
-        (rc = upload(&t->ph_inv, ph_inv.data(), ph_inv.size())) ||
-        (rc = upload(&t->ph_src, ph_src.data(), ph_src.size())) ||
-        (rc = upload(&t->ph_pw, ph_pw.data(), ph_pw.size())) ||
+        (phased && (rc = upload(&t->ph_inv, ph_inv.data(), ph_inv.size()))) ||
+        (phased && (rc = upload(&t->ph_src, ph_src.data(), ph_src.size()))) ||
+        (phased && (rc = upload(&t->ph_pw, ph_pw.data(), ph_pw.size()))) ||
         (ell_len && (rc = upload(&t->ell_pw, ell_pw.data(), ell_pw.size()))) ||
         (ell_len && (rc = upload(&t->ell_src, ell_src.data(), ell_src.size()))) ||
         (n_gs && (rc = upload(&t->gs_seg, gs_seg.data(), gs_seg.size()))) ||
@@ -700,7 +714,7 @@ int glif_table_create(const int64_t *post, const int64_t *col, const uint8_t *sy
         }
         if (n_syn) (void)hipMemset(*wp, 0, n_syn * sizeof(float));
     }
-    if ((rc = build_own_rows(t, col_ptr.data(), ps.data(), ph_src.data()))) {
+    if ((rc = build_own_rows(t, col_ptr.data(), ps.data(), phased ? ph_src.data() : nullptr))) {
         free_table(t);
         return rc;
     }
@@ -740,8 +754,8 @@ int glif_table_set_weights(glif_table *tt, const float *w, void *stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     int rc = launch_perm_gather(t->w_col, w, t->order, t->pcol, t->n_syn, t->pcol.mid, s);
     if (rc) return rc;
-    // the type-phased and grouped copies from w_col (near-sequential reads)
-    if (t->n_syn) {
+    // the other copies from w_col, whose order is close to theirs
+    if (t->ph_pw) {
         hipLaunchKernelGGL(k_gather_pair_w, dim3(grid_for(t->n_syn)), dim3(kBlock), 0, s, t->ph_pw, t->w_col,
                            t->ph_src, t->n_syn);
         GLIF_HIP(hipGetLastError());
