@@ -200,8 +200,8 @@ def test_backward_grouped_walk_matches_oracle(B, n, T):
 def test_many_synapse_types_forward_and_backward(B):
     """121 synapse types over 4 receptors, the shape of the reference's basis table
     (synaptic_data/basis_function_weights.csv: one row per synaptic model): G has 121 row
-    blocks, the grouped walk's rows span all of them (B = 5) and the type-phased walk has
-    121 phases (B = 2); deterministic forward bit-exact, BPTT within the bar."""
+    blocks, the grouped walk's rows span all of them (16-float rows at B = 5, 8-float at
+    B = 2); deterministic forward bit-exact, BPTT within the bar."""
     import dataclasses
     cfg = dataclasses.replace(tiny_config(rs=3.0, ins=4.0), n_syn_types=121, n_basis=4)
     tn = network(cfg, seed=11, dense_basis=True)

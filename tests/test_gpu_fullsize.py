@@ -269,8 +269,8 @@ def test_config4_forward(config4, rate):
 
 
 def test_config4_bptt_batch32(config4):
-    """B = 32: one-tick backward windows, 32-float G rows (8 lanes per column in the
-    type-phased walk), at the 50 Hz recurrent factor over 80 ms of the active regime: ticks
+    """B = 32: one-tick backward windows, 32-float G rows (8 lanes per column group
+    in the grouped walk), at the 50 Hz recurrent factor over 80 ms of the active regime: ticks
     300-379, from the state the deterministic rollout reaches at tick 300 (bit-exact with the
     oracle's), so its spike history feeds the first ticks' recurrent dW."""
     cfg, net, lgn, bkg = config4

@@ -1,6 +1,7 @@
 """GPU parity of the LGN currents computed ahead of the T loop.
 
-For batch sizes up to 8 the cell computes the LGN currents of 64 ticks at a time (k_lgn_rows)
+Where the forward runs a launch per tick (each test here runs so, and again by windows of three
+ticks, which have no such pass), for batch sizes up to 8 the cell computes the LGN currents of 64 ticks at a time (k_lgn_rows)
 into a ring of 130 current slots, the first segment before the loop and each later one on the
 cell's side stream beside the previous segment's ticks; the deterministic step
 adds a slot to the pulled recurrent currents, the event push (from batch 3) adds the recurrent

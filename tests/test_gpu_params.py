@@ -52,8 +52,8 @@ def _state_dev(cell, d):
 @pytest.mark.parametrize("pset", list(PSETS))
 @pytest.mark.parametrize("B", [2, 5])
 def test_forward_and_bptt_asymmetric(B, pset, pseudo_gauss, hard_reset):
-    """B = 2 takes the type-phased recurrent backward (8-float G rows), B = 5 the grouped
-    row-sliced walk (16-float rows)."""
+    """The recurrent backward's grouped row-sliced walk over 8-float (B = 2) and 16-float
+    (B = 5) G rows."""
     from v1_glif_model_amd.models import V1Column
     ckw, okw = _kw(pset, pseudo_gauss, hard_reset)
     cfg = tiny_config(rs=2.0, ins=3.0)

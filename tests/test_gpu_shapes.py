@@ -5,7 +5,7 @@ arithmetic and launch shapes depend on: neuron counts around the 64-lane wave (1
 130, 200), delay slots 1-9, receptors 1-8, synapse types 1-20 (dense basis), batch 1-32
 (every G row length and backward window width), sparse tables with empty columns, and both
 surrogates; cases 4 and 5 receive few of their types per neuron, so they run with compact G rows
-(grouped walk at B = 3, type-phased at B = 7) and the event push into per-type slots; the last
+(16-float rows at B = 3, 32-float at B = 7) and the event push into per-type slots; the last
 case fills all 64 accumulator lanes of the deterministic chunk pull (B = 8, nb = 8).  Per case,
 against the C oracle on the same inputs:
 

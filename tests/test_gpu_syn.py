@@ -210,7 +210,7 @@ def test_op_on_a_table_without_synapses(B):
 
 @pytest.mark.parametrize("B,nb", [(17, 8), (32, 8), (32, 1), (3, 2)])
 def test_syn_bwd_wide_and_narrow_rows(B, nb):
-    """G rows of 32 floats (B = 17-32, the type-phased column walk) and of 4 floats (B <= 4),
+    """G rows of 32 floats (B = 17-32) and of 4 floats (B <= 4),
     8 receptors and 1: the G build's dy tile at its smallest (8 posts of 32 batch entries x 8
     receptors) and its largest, padding entries written as zero."""
     import dataclasses
@@ -411,7 +411,7 @@ def test_syn_fwd_event_column_scan():
 
 def _wide_table(seed=11, n_post=2000, n_cols=150001, n_types=3):
     """A table of many short columns (0-3 synapses each): its dz walk has enough lanes at every
-    batch width, so the op walks it (grouped or type-phased) instead of using the work units."""
+    batch width, so the op walks it instead of using the work units."""
     from v1_glif_model_amd.tables import SynapseTable as Tab
     rng = np.random.default_rng(seed)
     col = np.repeat(np.arange(n_cols), rng.integers(0, 4, n_cols))
@@ -426,9 +426,8 @@ def _wide_table(seed=11, n_post=2000, n_cols=150001, n_types=3):
 
 @pytest.mark.parametrize("B", [2, 12, 32])
 def test_syn_bwd_wide_table_walks(B):
-    """The op's dz walks on a 150,001-column table: the type-phased column walk at 4- and
-    32-float G rows (B = 2, 32; dW in the same walk) and the grouped row-sliced walk at 16-float
-    rows (B = 12, dW over the work units beside it); spike and count inputs."""
+    """The op's dz walk on a 150,001-column table, the grouped row-sliced walk at 4-, 16- and
+    32-float G rows (B = 2, 12, 32) with the dW pass over the work units beside it; spike and count inputs."""
     from v1_glif_model_amd.ops import SynapseTable
     tab = _wide_table()
     rng = np.random.default_rng(B + 140)

@@ -2,7 +2,8 @@
 //
 // Forward, three ticks per launch (k_win_fwd): a workgroup per range of posts and batch entry sums
 // its recurrent and LGN currents from the spikes in LDS (win_kernels.h) and steps its posts.
-// Networks whose spike-major row offsets outgrow their bound run a launch or two per step t:
+// Networks whose spike-major row offsets outgrow their bound, and event forwards of over 262,144
+// neurons, run a launch or two per step t:
 //   LGN (B <= 8; event mode from B = 3 and without per-type slots): k_lgn_rows computes
 //                 the LGN currents of 64 ticks at a time, per post row in the reference's
 //                 order, into a ring of current slots ahead of the ticks that read them
@@ -25,7 +26,7 @@
 //                 of delays <= 2 Wwin - 3, one pass over the grouped row-sliced table
 //                 with the dW of the window's active columns behind it; with 16-float G rows
 //                 the other columns' dz run in the next window's adjoint launch (k_adj_dw);
-//                 without that order: k_bwd_rec, dz and dW in one type-phased pass
+//                 tables too long for that order: k_bwd_rec, dz and dW in one type-phased pass
 //   k_bwd_in      dW of the LGN / background events of the window's steps
 // A window is legal because dz_s depends only on dz_{>= s+3}: a spike reaches the
 // rise current one step later, the PSC the next, the voltage the one after.
@@ -995,7 +996,8 @@ __device__ inline void win_bkg(const WIN_CONST WinArgs &a, const float *basis_ld
 }
 
 // Bound by the latency of its chain (digests, visits' offsets, entries, state) and by instruction
-// issue, two thirds of its wave cycles waiting: 41 us per launch of three ticks at 66,000 neurons,
+// issue, two thirds of its wave cycles waiting (SQ_WAIT_ANY 66 % of SQ_WAVE_CYCLES at batch 5, 62 % in
+// deterministic mode at batch 32; 11 to 13 % for an issue slot): 41 us per launch of three ticks at 66,000 neurons,
 // batch 5, 5 Hz, 250 synapses per neuron, where the launches per tick it
 // replaced took 28 us each with the LGN events' passes beside them; deterministic at batch 32: 270
 // against 3 x 240 us.  One thread per post and 6 waves per SIMD (two workgroups of 704 - 768

@@ -133,8 +133,6 @@ struct Table {
     uint32_t *pidx = nullptr;     // [n_syn]       (n_slots - delay) * round64(n_pre) + pre, or null
     uint8_t *sid_row = nullptr;   // [n_syn]
     float *w_row = nullptr;       // [n_syn]
-    // type-phased (backward, tables without the grouped order; else nullptr): ordered by (syn_id, column, synapse id); the type-s
-    // synapses of column c are k in [ph_ptr[s * n_cols + c], ph_ptr[s * n_cols + c + 1])
     // ELL copy of the post-grouped table for single-delay (input) tables whose rows
     // pad to at most twice the synapse count: entry j of post n at j * n_post + n,
     // {pre | syn_id << 24, weight bits}, padding {0, +0.0f}; rows keep the
@@ -148,6 +146,9 @@ struct Table {
     int32_t n_chunks = 0;
     int4 *chunk_desc = nullptr;   // [n_chunks]
     Units units, wide;            // of kUnitEntries and kWideUnitEntries synapses
+    // type-phased (backward of tables whose padded grouped order would pass 2^31 positions; else nullptr): ordered
+    // by (syn_id, column, synapse id); the type-s synapses of column c are
+    // k in [ph_ptr[s * n_cols + c], ph_ptr[s * n_cols + c + 1])
     int32_t *ph_ptr = nullptr;    // [n_types * n_cols + 1]
     int32_t *ph_order = nullptr;  // [n_syn]       synapse id at position k
     uint2 *ph_pw = nullptr;       // [n_syn]       {post, weight bits}

@@ -8,11 +8,12 @@
 //   post-grouped table (Table::row_ptr/pd/sid_row/w_row): the synapses of post n
 //     are j in [row_ptr[n], row_ptr[n+1]) in ascending (column, synapse id);
 //     pd[j] = pre | (delay - 1) << 24.
-//   type-phased table (Table::ph_ptr/ph_pw): synapses ordered by (syn_id, column,
+//   type-phased table (Table::ph_ptr/ph_pw; only where the grouped order below would
+//     pass 2^31 positions): synapses ordered by (syn_id, column,
 //     synapse id); the type-s synapses of column c are
 //     k in [ph_ptr[s * n_cols + c], ph_ptr[s * n_cols + c + 1]);
 //     ph_pw[k] = {post, weight bits}.
-//   grouped row-sliced table (Table::gs_seg/gs_pw, recurrent tables): lane group g's
+//   grouped row-sliced table (Table::gs_seg/gs_pw): lane group g's
 //     columns 4g..4g+3, by G-row slice, then G row (syn_id * n_post + post); entries
 //     {row | column-in-group << 29, weight bits}, each segment padded to 8 entries.
 //   I  [B][n_post][nb]  (the reference's i_rec_flat [B*N, nb]).
@@ -346,7 +347,8 @@ __device__ inline void bwd_cols(const ColArgs &a, const Act &act) {
 // Every wave finishes a slice before starting the next, so the waves in flight gather
 // from one quarter of G at a time, and a group owns its columns, so dz needs no atomics.
 // Each column sums its entries in G-row order (syn_id, then post), the order of
-// bwd_cols; split, the lane groups' sums of their slices are added in that order.  The dW of active columns is a separate pass (k_bwd_rec_dw in cell.hip):
+// bwd_cols; split, the lane groups' sums of their slices are added in that order.  The dW
+// of active columns is a separate pass (rec_dw_body in cell.hip):
 // holding it here costs a third more registers and a second walk per group.
 //
 // Measured on MI355X with a config-2-sized table (16.5M synapses, 330k columns, G 21 MB):
